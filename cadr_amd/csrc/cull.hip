@@ -8,8 +8,9 @@
 // count per StateSet (the operands of vkCmdDrawIndexedIndirectCount).
 //
 // Work is split into tiles of at most blockSize*itemsPerThread drawables that
-// never cross a StateSet boundary; tiles are taken from an atomic ticket in
-// array order, so a tile only ever waits on tiles that already run.  Within a
+// never cross a StateSet boundary; tiles are taken by atomic tickets in array
+// order (dealt over several counters where small tiles need it, takeTicket),
+// so a tile only ever waits on tiles that already run or come next.  Within a
 // tile, wave w owns a contiguous run of 64*itemsPerThread drawables (item j of
 // lane l is drawable w*64*itemsPerThread + j*64 + l): loads are coalesced and
 // the visibility of 64 drawables is one wave64 ballot.  Offsets come from a
@@ -23,7 +24,7 @@
 //   cullViewKernel - one view: one workgroup per tile, visibility kept in
 //     registers, a 64-lane parallel look-back in wave 0, each visible
 //     drawable's lane storing its command at its compacted slot.  It resets
-//     its ticket and advances the epoch itself (the last workgroup to
+//     its tickets and advances the epoch itself (the last workgroup to
 //     finish), so a view costs one launch.
 //   cullViewLoopKernel - the same view pass as a persistent loop over tiles,
 //     the next tile's loads in flight during the current tile's look-back
@@ -53,13 +54,14 @@
 namespace cadr {
 
 constexpr uint32_t kViewGroup = 64;   // views whose look-backs share one wave
-constexpr uint32_t kCtlTicket = 0;    // ctl words, each on its own 128-byte line
-constexpr uint32_t kCtlDone = 32;
-constexpr uint32_t kCtlEpoch = 64;
-constexpr uint32_t kCtlError = 96;    // epoch of a launch whose look-back gave up, else 0
-constexpr uint32_t kCtlWords = 128;
-constexpr uint32_t kLdsMeshes = 64;
-constexpr uint64_t kDefaultWaitLimitUs = 1000000;  // 1 s: some ten thousand times a tile's run time   // mesh tables up to this size are staged in LDS
+constexpr uint32_t kMaxShards = 16;   // ctl words, each on its own 128-byte line
+constexpr uint32_t kCtlShard = 0;     // + 64 g: tickets of shard g; + 64 g + 32: workgroups of shard g that left
+constexpr uint32_t kCtlDone = kCtlShard + 64 * kMaxShards;  // shards whose workgroups all left
+constexpr uint32_t kCtlEpoch = kCtlDone + 32;
+constexpr uint32_t kCtlError = kCtlDone + 64;  // epoch of a launch whose look-back gave up, else 0
+constexpr uint32_t kCtlWords = kCtlDone + 96;
+constexpr uint32_t kLdsMeshes = 64;   // mesh tables up to this size are staged in LDS
+constexpr uint64_t kDefaultWaitLimitUs = 1000000;  // 1 s: some ten thousand times a tile's run time
 
 constexpr uint32_t kStateAggregate = 1;
 constexpr uint32_t kStatePrefix = 2;
@@ -82,6 +84,7 @@ struct CullParams {
 	const uint64_t* statusBase;  // [numJobs] prefix of numViews*numTiles
 	uint64_t* status;
 	uint32_t* ctl;
+	uint32_t shardShift;  // log2 of the ticket shards; beside ctl, so that the first ticket waits for one load
 	uint32_t numJobs;
 	uint32_t totalWork;
 	uint32_t splitTiles;  // batched: a job's last tiles handed out per view group
@@ -403,6 +406,66 @@ struct WaitBound {
 	uint64_t limit;
 	uint32_t epoch;
 };
+
+// Work tickets.  An atomic add on one address takes 11-12 ns on this GPU
+// whichever workgroup issues it (measured: 1024 workgroups one each, 13.5 us;
+// spread over 64 lines 2.9 us), so with one ticket counter a launch of small
+// tiles was bound by it (15,300 tiles of 1024 drawables in 24 jobs: 221 us
+// with one counter, 155 with 8; 1,206 such tiles of one view: 40 and 14 us).
+// The work items are therefore dealt to up to kMaxShards counters
+// in runs of 8 (item t belongs to shard (t / 8) mod S), and workgroup b takes
+// tickets of shard (b / 8) mod S only.  Launches of one workgroup per item
+// have exactly as many workgroups as items in every shard.
+//
+// Tickets order a shard's items, so the smallest unfinished item of a launch
+// is always held by a running workgroup, whose predecessors are done, or is
+// the next ticket of its shard.  Workgroups are dispatched round-robin over
+// the XCDs, and (b / 8) spreads a shard over all of them, so each shard has
+// running workgroups as soon as 8 S of the launch's workgroups run; the
+// bounded waits below turn anything else into an error.
+struct Shard {
+	uint32_t shift;  // log2 of the launch's shards
+	uint32_t g;      // this workgroup's shard
+};
+
+// Tiles of this many drawables never take more than one shard (shardShiftFor):
+// their kernels hold no shard registers.
+constexpr bool oneShard(uint32_t tile) { return tile * 20ull >= 150000u; }
+
+template <uint32_t TILE>
+__device__ __forceinline__ Shard homeShard(const CullParams& P)
+{
+	if constexpr (oneShard(TILE)) return Shard{0u, 0u};
+	return Shard{P.shardShift, (blockIdx.x >> 3) & ((1u << P.shardShift) - 1u)};
+}
+
+__device__ __forceinline__ uint32_t takeTicket(const CullParams& P, Shard s)
+{
+	const uint32_t r = atomicAdd(&P.ctl[kCtlShard + 64u * s.g], 1u);
+	return ((((r >> 3) << s.shift) + s.g) << 3) + (r & 7u);
+}
+
+// Called by one thread of each workgroup when it leaves: the last one of the
+// launch resets the tickets and retires the launch's epoch, so the next
+// launch on the workspace never sees this launch's status words as its own.
+// The workgroups of a shard count among themselves, then the shards.
+__device__ __forceinline__ void leaveLaunch(const CullParams& P, Shard s, uint32_t epoch)
+{
+	const uint32_t S = 1u << s.shift, runs = gridDim.x >> (s.shift + 3u), rest = gridDim.x & (8u * S - 1u);
+	const uint32_t mine = 8u * runs + (rest > s.g * 8u ? min(rest - s.g * 8u, 8u) : 0u);
+	if (atomicAdd(&P.ctl[kCtlShard + 64u * s.g + 32u], 1u) != mine - 1u) return;
+	if (S > 1u) {
+		const uint32_t shards = min(S, (gridDim.x + 7u) / 8u);
+		if (atomicAdd(&P.ctl[kCtlDone], 1u) != shards - 1u) return;
+		atomicExch(&P.ctl[kCtlDone], 0u);
+	}
+	for (uint32_t g = 0; g < S; g++) {
+		atomicExch(&P.ctl[kCtlShard + 64u * g], 0u);
+		atomicExch(&P.ctl[kCtlShard + 64u * g + 32u], 0u);
+	}
+	const uint32_t e = epoch + 1u;
+	atomicExch(&P.ctl[kCtlEpoch], e == 0u ? 1u : e);
+}
 
 // Called after an unready poll; start is 0 until the first such poll.
 __device__ __forceinline__ bool waitGiveUp(const WaitBound& B, uint64_t& start)
@@ -762,8 +825,9 @@ __device__ __forceinline__ void cullViewBody(const CullParams& P)
 	__shared__ uint32_t sMeshes[16 * kLdsMeshes];
 
 	const uint32_t tid = threadIdx.x, lane = laneId(), wave = tid / 64;
+	const Shard shard = homeShard<BLOCK * ITEMS>(P);
+	if (tid == 0) sTicket = takeTicket(P, shard);
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-	if (tid == 0) sTicket = atomicAdd(&P.ctl[kCtlTicket], 1u);
 	const cadrCullJob J = loadJob(P.jobs, 0);
 	const bool ldsMeshes = stageMeshes<BLOCK>(sMeshes, J, tid);
 	__syncthreads();
@@ -777,17 +841,8 @@ __device__ __forceinline__ void cullViewBody(const CullParams& P)
 			cullViewTile<BLOCK, ITEMS, false, FUSED>(P, J, t, epoch, meshes, sCnt, &sExcl, mat, tid, lane, wave);
 	}
 
-	// the last workgroup to finish resets the ticket and starts a new epoch
 	__syncthreads();
-	if (tid == 0) {
-		const uint32_t d = atomicAdd(&P.ctl[kCtlDone], 1u);
-		if (d == gridDim.x - 1) {
-			atomicExch(&P.ctl[kCtlTicket], 0u);
-			atomicExch(&P.ctl[kCtlDone], 0u);
-			const uint32_t e = epoch + 1u;
-			atomicExch(&P.ctl[kCtlEpoch], e == 0u ? 1u : e);
-		}
-	}
+	if (tid == 0) leaveLaunch(P, shard, epoch);
 }
 
 template <int BLOCK, int ITEMS>
@@ -809,6 +864,7 @@ __global__ __launch_bounds__(BLOCK) void cullViewKernel(CullParams P)
 // loop's extra ticket and barrier.
 template <int BLOCK, int ITEMS, bool LDS>
 __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCullJob& J, uint32_t t, uint32_t epoch,
+                                              Shard shard,
                                               const MeshTable& meshes, uint32_t* sTicket,
                                               uint32_t (*sCnt)[BLOCK / 64][ITEMS], uint32_t* sExcl, uint32_t tid,
                                               uint32_t lane, uint32_t wave)
@@ -833,7 +889,7 @@ __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCul
 			mask[j] = __ballot(vis);
 			if (lane == 0) sCnt[b][wave][j] = uint32_t(__builtin_popcountll(mask[j]));
 		}
-		if (tid == 0) *sTicket = atomicAdd(&P.ctl[kCtlTicket], 1u);
+		if (tid == 0) *sTicket = takeTicket(P, shard);
 		__syncthreads();
 
 		// the next tile's loads, in flight through this tile's look-back and stores
@@ -910,8 +966,9 @@ __global__ __launch_bounds__(BLOCK) void cullViewLoopKernel(CullParams P)
 	__shared__ uint32_t sMeshes[16 * kLdsMeshes];
 
 	const uint32_t tid = threadIdx.x, lane = laneId(), wave = tid / 64;
+	const Shard shard = homeShard<BLOCK * ITEMS>(P);
+	if (tid == 0) sTicket = takeTicket(P, shard);
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-	if (tid == 0) sTicket = atomicAdd(&P.ctl[kCtlTicket], 1u);
 	const cadrCullJob J = loadJob(P.jobs, 0);
 	const bool ldsMeshes = stageMeshes<BLOCK>(sMeshes, J, tid);
 	__syncthreads();
@@ -920,22 +977,13 @@ __global__ __launch_bounds__(BLOCK) void cullViewLoopKernel(CullParams P)
 	const MeshTable meshes{sMeshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
 	if (t < P.totalWork) {
 		if (ldsMeshes)
-			cullViewTiles<BLOCK, ITEMS, true>(P, J, t, epoch, meshes, &sTicket, sCnt, sExcl, tid, lane, wave);
+			cullViewTiles<BLOCK, ITEMS, true>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, tid, lane, wave);
 		else
-			cullViewTiles<BLOCK, ITEMS, false>(P, J, t, epoch, meshes, &sTicket, sCnt, sExcl, tid, lane, wave);
+			cullViewTiles<BLOCK, ITEMS, false>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, tid, lane, wave);
 	}
 
-	// the last workgroup to finish resets the ticket and starts a new epoch
 	__syncthreads();
-	if (tid == 0) {
-		const uint32_t d = atomicAdd(&P.ctl[kCtlDone], 1u);
-		if (d == gridDim.x - 1) {
-			atomicExch(&P.ctl[kCtlTicket], 0u);
-			atomicExch(&P.ctl[kCtlDone], 0u);
-			const uint32_t e = epoch + 1u;
-			atomicExch(&P.ctl[kCtlEpoch], e == 0u ? 1u : e);
-		}
-	}
+	if (tid == 0) leaveLaunch(P, shard, epoch);
 }
 
 // The fused kernel is latency-bound (a chain of dependent loads per item), so
@@ -981,10 +1029,11 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 	const uint32_t lane = laneId();
 	const uint32_t wave = tid / 64;
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	const Shard shard = homeShard<S::TILE>(P);
 	uint32_t job = 0, stagedJob = ~0u;
 
 	for (;;) {
-		if (tid == 0) sh.ticket = atomicAdd(&P.ctl[kCtlTicket], 1u);
+		if (tid == 0) sh.ticket = takeTicket(P, shard);
 		__syncthreads();
 		const uint32_t w = uniform(sh.ticket);
 		if (w >= P.totalWork) break;
@@ -1293,18 +1342,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		}
 	}
 
-	// the last workgroup to leave resets the ticket and retires this launch's
-	// epoch, so the next launch on the workspace (of either kernel) never sees
-	// this launch's status words as its own
-	if (tid == 0) {
-		const uint32_t d = atomicAdd(&P.ctl[kCtlDone], 1u);
-		if (d == gridDim.x - 1) {
-			atomicExch(&P.ctl[kCtlTicket], 0u);
-			atomicExch(&P.ctl[kCtlDone], 0u);
-			const uint32_t e = epoch + 1u;
-			atomicExch(&P.ctl[kCtlEpoch], e == 0u ? 1u : e);
-		}
-	}
+	if (tid == 0) leaveLaunch(P, shard, epoch);
 }
 
 // Work items of a job in a batched launch: its tiles, plus one more per
@@ -1317,11 +1355,11 @@ __host__ __device__ __forceinline__ uint64_t jobWorkItems(uint32_t numTiles, uin
 	return numTiles + split * (groups - 1);
 }
 
-// Job offsets for a batched launch (prefix sums over jobs), ticket reset and
-// a new epoch; one block, before the cull kernel on the same stream.
+// Job offsets for a batched launch (prefix sums over jobs); one block, before
+// the cull kernel on the same stream.
 __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __restrict__ jobs, uint32_t numJobs,
                                                        uint32_t splitTiles, uint32_t* __restrict__ firstWork,
-                                                       uint64_t* __restrict__ statusBase, uint32_t* __restrict__ ctl)
+                                                       uint64_t* __restrict__ statusBase)
 {
 	__shared__ uint32_t sT[256];
 	__shared__ uint64_t sS[256];
@@ -1355,13 +1393,33 @@ __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __rest
 		runS += sS[255];
 		__syncthreads();
 	}
-	if (tid == 0) {
-		firstWork[numJobs] = runT;
-		ctl[kCtlTicket] = 0;
-		ctl[kCtlDone] = 0;
-		uint32_t e = ctl[kCtlEpoch] + 1u;
-		ctl[kCtlEpoch] = e == 0u ? 1u : e;
-	}
+	if (tid == 0) firstWork[numJobs] = runT;
+}
+
+// Ticket shards (log2) for a launch of `workgroups` workgroups over `work`
+// items that move about `bytes` bytes in all.  One counter hands out an item
+// every 12 ns; an item of 75 KB takes as long at 6.3 TB/s, so as many shards
+// are taken as make the tickets twice as fast as the bytes (8 for one-view
+// tiles of 1024 drawables, 1 for 8192 or for many views).  More than that
+// loses: the look-back waits a little longer where a chain's neighbours come
+// from different counters (10M drawables in 1024 x 8 tiles, 8 shards: 64.4
+// against 60.4 us with one).  Below 256 workgroups one counter costs less
+// than the second level of leaveLaunch.
+inline uint32_t shardShiftFor(uint32_t tile, uint64_t workgroups, uint64_t work, uint64_t bytes)
+{
+	if (oneShard(tile) || workgroups < 256 || work >= (1ull << 31)) return 0;
+	const uint64_t item = bytes / work + 1;
+	uint32_t shift = 0;
+	while ((2u << shift) <= kMaxShards && workgroups >= (uint64_t(64) << shift) && (item << shift) < 150000u) shift++;
+	return shift;
+}
+
+// Bytes a job moves, about: its drawables read once (and, where its leaf
+// level is computed, 128 more for the matrices) and 3 per drawable and view
+// written (20 for about one in seven).
+inline uint64_t jobBytes(const cadrCullJob& J, bool leaf)
+{
+	return uint64_t(J.numDrawables) * (20u + (leaf ? 116u : 0u) + 3ull * J.numViews);
 }
 
 }  // namespace cadr
@@ -1645,12 +1703,13 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 	if (perCU == 0) perCU = ke.block >= 512 ? 2 : 4;
 	uint64_t grid = uint64_t(cu > 0 ? cu : 256) * perCU;
 	const uint32_t splitTiles = (config->flags & CADR_CULL_WHOLE_TILES) ? 0u : uint32_t(std::min<uint64_t>(grid, 1u << 20));
-	uint64_t totalWork = 0, statusNeed = 0;
+	uint64_t totalWork = 0, statusNeed = 0, bytes = 0;
 	for (uint32_t j = 0; j < numJobs; j++) {
 		const int rc = checkJob(hostJobs[j]);
 		if (rc != CADR_SUCCESS) return rc;
 		totalWork += jobWorkItems(hostJobs[j].numTiles, hostJobs[j].numViews, splitTiles);
 		statusNeed += uint64_t(hostJobs[j].numViews) * hostJobs[j].numTiles;
+		bytes += jobBytes(hostJobs[j], leaves != nullptr);
 	}
 	CADR_REQUIRE(totalWork < 0xffffffffull, name + ": too many tiles in one launch");
 	CADR_REQUIRE(statusNeed <= ws->statusWords, name + ": workspace has too few status words");
@@ -1661,7 +1720,7 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 	hipStream_t s = hipStream_t(stream);
 	const auto* jobs = reinterpret_cast<const cadrCullJob*>(deviceJobs);
 	hipLaunchKernelGGL(cullSetupKernel, dim3(1), dim3(256), 0, s, jobs, numJobs, splitTiles, ws->firstWork,
-	                   ws->statusBase, ws->ctl);
+	                   ws->statusBase);
 	CADR_CHECK_HIP(hipGetLastError(), "cullSetupKernel launch");
 	if (totalWork == 0) CADR_RETURN_NO_LAUNCH(s);
 	if (grid > totalWork) grid = totalWork;
@@ -1674,6 +1733,7 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 	p.numJobs = numJobs;
 	p.totalWork = uint32_t(totalWork);
 	p.splitTiles = splitTiles;
+	p.shardShift = shardShiftFor(ke.block * ke.items, grid, totalWork, bytes);
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
 	p.leaves = leaves;
@@ -1739,10 +1799,10 @@ CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, cons
 	// (grid = resident workgroups); else one tile per workgroup, which saves
 	// the loop's extra ticket and barrier on a launch-bound view
 	const int resident = ke->viewLoop ? residentWorkgroups(ke->viewLoop, ke->block) : 0;
-	if (resident > 0 && hostJob->numTiles > uint32_t(resident))
-		launchKernel(ke->viewLoop, dim3(uint32_t(resident)), dim3(ke->block), hipStream_t(stream), p);
-	else
-		launchKernel(ke->view, dim3(hostJob->numTiles), dim3(ke->block), hipStream_t(stream), p);
+	const bool loop = resident > 0 && hostJob->numTiles > uint32_t(resident);
+	const uint32_t grid = loop ? uint32_t(resident) : hostJob->numTiles;
+	p.shardShift = shardShiftFor(ke->block * ke->items, grid, hostJob->numTiles, jobBytes(*hostJob, false));
+	launchKernel(loop ? ke->viewLoop : ke->view, dim3(grid), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "cullViewKernel launch");
 	return ok();
 }
@@ -1776,6 +1836,8 @@ CADR_API int cadrPropagateCullView(const cadrTransformLevel* leaf, const cadrCul
 	p.waitLimit = ws->waitLimit;
 	p.leaf = LeafParams{leaf->localMatrices, leaf->parentIndex, leaf->parentWorld, leaf->worldMatrices, leaf->spheres,
 	                    leaf->parentWorld ? leaf->parentCount : 0u};
+	p.shardShift = shardShiftFor(ke->block * ke->items, hostJob->numTiles, hostJob->numTiles,
+	                             jobBytes(*hostJob, true));
 	launchKernel(ke->fused, dim3(hostJob->numTiles), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "fused cullViewKernel launch");
 	return ok();
