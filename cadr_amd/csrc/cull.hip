@@ -735,10 +735,113 @@ __device__ __forceinline__ void propagateTileItems(const LeafParams& Lf, const c
 
 // ---------------------------------------------------------------- one view
 
+// A wave's visible items as a compact list in its own LDS, in drawable order:
+// item index in the wave's run (10 bits), the LOD its projected radius
+// selects before the mesh's own limit (2 bits) and, for a staged mesh table,
+// the mesh (6 bits).  The command stores then run with full lanes: in
+// drawable order a wave stored its items one by one, each with the few lanes
+// that are visible, and the CU's address path, which takes a store
+// instruction's 64 lanes whether they are active or not, bound the views that
+// see a part of everything (10M drawables, 25% visible in every item: 49 MB
+// of commands cost 57 of 85 us).
+constexpr uint32_t kRunLodShift = 10, kRunMeshShift = 12;
+
+// LOD index by projected radius alone (lodAtDepth before the mesh's limit).
+__device__ __forceinline__ uint32_t lodByRadius(float r, float vz, const ViewC& v)
+{
+	const float p = r * v.lodScale;
+	return uint32_t(p < v.th0 * vz) + uint32_t(p < v.th1 * vz) + uint32_t(p < v.th2 * vz);
+}
+
+// Tests the wave's items (first item `base` of the tile) and lists the
+// visible ones; returns their number (the same in every lane).
+template <int ITEMS, bool LDS>
+__device__ __forceinline__ uint32_t listVisible(const float4 (&sp)[ITEMS], const uint32_t (&mi)[ITEMS],
+                                                const TileDesc& T, uint32_t numMeshes, const ViewC& V, uint32_t base,
+                                                uint32_t lane, uint32_t* run)
+{
+	static_assert(64 * ITEMS <= (1 << kRunLodShift), "item index bits");
+	waveSync();  // the list may lie where the wave's matrices were staged
+	uint32_t n = 0;
+#pragma unroll
+	for (int j = 0; j < ITEMS; j++) {
+		const bool vis = base + j * 64 + lane < T.count && mi[j] < numMeshes && sphereVisible(sp[j], V);
+		const uint64_t mask = __ballot(vis);
+		if (vis) {
+			const uint32_t lod = lodByRadius(sp[j].w, viewCoord(V.r2, sp[j]), V);
+			run[n + maskRank(mask)] = (j * 64 + lane) | (lod << kRunLodShift) | (LDS ? mi[j] << kRunMeshShift : 0u);
+		}
+		n = uniform(n + uint32_t(__builtin_popcountll(mask)));
+	}
+	return n;
+}
+
+// Stores the commands of a wave's n listed items from output slot pos on, 64
+// consecutive commands per pair of stores.  first: drawable index of the
+// wave's item 0.
+template <bool LDS>
+__device__ __forceinline__ void storeListed(const uint32_t* run, uint32_t n, uint32_t pos, uint32_t first,
+                                            const MeshTable& M, gptr<uint32_t> meshIndex, gmut<uint32_t> out,
+                                            uint32_t stride, uint32_t lane)
+{
+	waveSync();  // the list is written by other lanes
+	for (uint32_t c = 0; c < n; c += 64u) {
+		const uint32_t i = c + lane;
+		if (i >= n || pos + i >= stride) continue;
+		const uint32_t e = run[i];
+		const uint32_t drawable = first + (e & ((1u << kRunLodShift) - 1u)), raw = (e >> kRunLodShift) & 3u;
+		uint32_t count, firstIndex, vofs;
+		if constexpr (LDS) {
+			const uint32_t m = e >> kRunMeshShift;
+			const uint32_t lod = min(raw, M.field(4, m));
+			count = M.field(8 + lod, m);
+			firstIndex = M.field(12 + lod, m);
+			vofs = M.field(5, m);
+		} else {
+			const gptr<cadrMesh> mesh = M.mem + meshIndex[drawable];
+			const uint32_t lod = min(raw, maxLodOf(mesh->lodCount));
+			count = mesh->indexCount[lod];
+			firstIndex = mesh->firstIndex[lod];
+			vofs = uint32_t(mesh->vertexOffset);
+		}
+		const gmut<uint32_t> o = out + uint64_t(pos + i) * 5ull;
+		o[0] = count;
+		o[1] = 1u;
+		o[2] = firstIndex;
+		o[3] = vofs;
+		o[4] = drawable;
+	}
+	waveSync();  // read before the next tile's list replaces it
+}
+
+// Look-back of a tile by wave 0, from the waves' counts; the exclusive prefix
+// goes to *sExclP and a StateSet's last tile writes its count.
+template <int WAVES>
+__device__ __forceinline__ void tileOffset(const CullParams& P, const cadrCullJob& J, const TileDesc& T, uint32_t epoch,
+                                           const uint32_t* sCnt, uint32_t* sExclP, uint32_t lane)
+{
+	uint32_t total = 0;
+#pragma unroll
+	for (int q = 0; q < WAVES; q++) total += sCnt[q];
+	uint64_t* chain = P.status;
+	uint32_t excl = 0;
+	if (T.first) {
+		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
+	} else {
+		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
+		excl = lookBackWave(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch}, lane);
+		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
+	}
+	if (lane == 0) {
+		*sExclP = excl;
+		if (T.last && T.k < J.numStateSets) globalMut<uint32_t>(J.counts)[T.k] = excl + total;
+	}
+}
+
 template <int BLOCK, int ITEMS, bool LDS, bool FUSED>
 __device__ __forceinline__ void cullViewTile(const CullParams& P, const cadrCullJob& J, uint32_t t, uint32_t epoch,
-                                             const MeshTable& meshes, uint32_t (*sCnt)[ITEMS], uint32_t* sExclP,
-                                             float4* sMat, uint32_t tid, uint32_t lane, uint32_t wave)
+                                             Shard shard, const MeshTable& meshes, uint32_t* sCnt, uint32_t* sExclP,
+                                             float4* sMat, uint32_t* run, uint32_t lane, uint32_t wave)
 {
 	constexpr int WAVES = BLOCK / 64, WAVE_ITEMS = 64 * ITEMS;
 	const TileDesc T = loadTile(J, t, BLOCK * ITEMS);
@@ -755,72 +858,30 @@ __device__ __forceinline__ void cullViewTile(const CullParams& P, const cadrCull
 		propagateTileItems<ITEMS, LDS>(P.leaf, J, T, wave * WAVE_ITEMS, lane, sMat, meshes, sp, mi);
 	else
 		loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
-	float vz[ITEMS];
-	uint64_t mask[ITEMS];
-#pragma unroll
-	for (int j = 0; j < ITEMS; j++) {
-		const uint32_t e = wave * WAVE_ITEMS + j * 64 + lane;
-		const bool vis = e < T.count && mi[j] < J.numMeshes && sphereVisible(sp[j], V);
-		vz[j] = viewCoord(V.r2, sp[j]);
-		mask[j] = __ballot(vis);
-		if (lane == 0) sCnt[wave][j] = uint32_t(__builtin_popcountll(mask[j]));
-	}
+	const uint32_t n = listVisible<ITEMS, LDS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
+	if (lane == 0) sCnt[wave] = n;
 	__syncthreads();
-
-	if (wave == 0) {
-		uint32_t total = 0;
-		for (int q = 0; q < WAVES; q++)
-			for (int j = 0; j < ITEMS; j++) total += sCnt[q][j];
-		uint64_t* chain = P.status;
-		uint32_t excl = 0;
-		if (T.first) {
-			if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
-		} else {
-			if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
-			excl = lookBackWave(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch}, lane);
-			if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
-		}
-		if (lane == 0) {
-			*sExclP = excl;
-			if (T.last && T.k < J.numStateSets) globalMut<uint32_t>(J.counts)[T.k] = excl + total;
-		}
-	}
+	if (wave == 0) tileOffset<WAVES>(P, J, T, epoch, sCnt, sExclP, lane);
 	__syncthreads();
+	// the workgroup is done with the launch's tickets and status words: the
+	// last wave signs off while the others store, so that no wave waits for
+	// its stores behind the atomics
+	if (wave == WAVES - 1 && lane == 0) leaveLaunch(P, shard, epoch);
 
 	uint32_t pos = T.segBase + *sExclP;
-	for (uint32_t q = 0; q < wave; q++)
-		for (int j = 0; j < ITEMS; j++) pos += sCnt[q][j];
-	pos = uniform(pos);
-	const gmut<uint32_t> out = globalMut<uint32_t>(J.commands);
-#pragma unroll
-	for (int j = 0; j < ITEMS; j++) {
-		const uint32_t n = uint32_t(__builtin_popcountll(mask[j]));
-		if (n == 0) continue;
-		if ((mask[j] >> lane) & 1ull) {
-			uint32_t count, first, vofs;
-			meshCommand<LDS>(meshes, mi[j], sp[j].w, vz[j], V, count, first, vofs);
-			const uint32_t r = maskRank(mask[j]);
-			if (pos + r < J.commandStride) {
-				const gmut<uint32_t> o = out + uint64_t(pos) * 5ull + uint64_t(r * 5u);
-				o[0] = count;
-				o[1] = 1u;
-				o[2] = first;
-				o[3] = vofs;
-				o[4] = T.start + wave * WAVE_ITEMS + j * 64 + lane;
-			}
-		}
-		pos = uniform(pos + n);
-	}
+	for (uint32_t q = 0; q < wave; q++) pos += sCnt[q];
+	storeListed<LDS>(run, n, uniform(pos), T.start + wave * WAVE_ITEMS, meshes, meshIndex,
+	                 globalMut<uint32_t>(J.commands), J.commandStride, lane);
 }
-
 
 template <int BLOCK, int ITEMS, bool FUSED>
 __device__ __forceinline__ void cullViewBody(const CullParams& P)
 {
 	constexpr int WAVES = BLOCK / 64;
-	__shared__ float4 sMat[FUSED ? WAVES : 1][FUSED ? 256 : 1];
+	// a wave's 4-KiB matrix staging, done with before its list is written
+	__shared__ float4 sMat[WAVES][FUSED ? 256 : 16 * ITEMS];
 	__shared__ uint32_t sTicket;
-	__shared__ uint32_t sCnt[WAVES][ITEMS];
+	__shared__ uint32_t sCnt[WAVES];
 	__shared__ uint32_t sExcl;
 	__shared__ uint32_t sMeshes[16 * kLdsMeshes];
 
@@ -833,16 +894,16 @@ __device__ __forceinline__ void cullViewBody(const CullParams& P)
 	__syncthreads();
 	const uint32_t t = uniform(sTicket);
 	const MeshTable meshes{sMeshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
-	if (t < P.totalWork) {
-		float4* mat = &sMat[FUSED ? wave : 0][0];
-		if (ldsMeshes)
-			cullViewTile<BLOCK, ITEMS, true, FUSED>(P, J, t, epoch, meshes, sCnt, &sExcl, mat, tid, lane, wave);
-		else
-			cullViewTile<BLOCK, ITEMS, false, FUSED>(P, J, t, epoch, meshes, sCnt, &sExcl, mat, tid, lane, wave);
+	if (t >= P.totalWork) {
+		if (tid == 0) leaveLaunch(P, shard, epoch);
+		return;
 	}
-
-	__syncthreads();
-	if (tid == 0) leaveLaunch(P, shard, epoch);
+	float4* mat = sMat[wave];
+	uint32_t* run = reinterpret_cast<uint32_t*>(mat);
+	if (ldsMeshes)
+		cullViewTile<BLOCK, ITEMS, true, FUSED>(P, J, t, epoch, shard, meshes, sCnt, &sExcl, mat, run, lane, wave);
+	else
+		cullViewTile<BLOCK, ITEMS, false, FUSED>(P, J, t, epoch, shard, meshes, sCnt, &sExcl, mat, run, lane, wave);
 }
 
 template <int BLOCK, int ITEMS>
@@ -854,20 +915,18 @@ __global__ __launch_bounds__(BLOCK) void cullViewKernel(CullParams P)
 // The one-view cull as a persistent loop: each workgroup stages the mesh
 // table once and then takes tiles by ticket until none is left.  The next
 // tile's ticket and its loads are issued right after the current tile's
-// counts, so they are in flight during the current tile's look-back and
-// stores instead of after them.  Counts and the wave offsets alternate
-// between two LDS buffers, so two barriers per tile suffice.  Results are
-// those of cullViewTile: the same tests, the same compaction order.
-// Launched with one workgroup per resident slot when a view has more tiles
-// than that (10M drawables, 1024 x 8: 45 against 52 µs); a view of fewer
-// tiles takes one tile per workgroup (cullViewKernel), which saves the
-// loop's extra ticket and barrier.
+// items are listed, into the same registers, so they are in flight during
+// the current tile's look-back and stores.  Counts and the exclusive prefix
+// alternate between two LDS buffers, so two barriers per tile suffice.
+// Results are those of cullViewTile: the same tests, the same compaction
+// order.  Launched with one workgroup per resident slot when a view has more
+// tiles than that; a view of fewer tiles takes one tile per workgroup
+// (cullViewKernel), which saves the loop's extra ticket and barrier.
 template <int BLOCK, int ITEMS, bool LDS>
 __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCullJob& J, uint32_t t, uint32_t epoch,
-                                              Shard shard,
-                                              const MeshTable& meshes, uint32_t* sTicket,
-                                              uint32_t (*sCnt)[BLOCK / 64][ITEMS], uint32_t* sExcl, uint32_t tid,
-                                              uint32_t lane, uint32_t wave)
+                                              Shard shard, const MeshTable& meshes, uint32_t* sTicket,
+                                              uint32_t (*sCnt)[BLOCK / 64], uint32_t* sExcl, uint32_t* run,
+                                              uint32_t tid, uint32_t lane, uint32_t wave)
 {
 	constexpr int WAVES = BLOCK / 64, WAVE_ITEMS = 64 * ITEMS;
 	const ViewC V = loadView(J.views, 0);
@@ -879,80 +938,29 @@ __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCul
 	uint32_t mi[ITEMS];
 	loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
 	for (uint32_t b = 0;; b ^= 1u) {
-		float vz[ITEMS];
-		uint64_t mask[ITEMS];
-#pragma unroll
-		for (int j = 0; j < ITEMS; j++) {
-			const uint32_t e = wave * WAVE_ITEMS + j * 64 + lane;
-			const bool vis = e < T.count && mi[j] < J.numMeshes && sphereVisible(sp[j], V);
-			vz[j] = viewCoord(V.r2, sp[j]);
-			mask[j] = __ballot(vis);
-			if (lane == 0) sCnt[b][wave][j] = uint32_t(__builtin_popcountll(mask[j]));
-		}
+		const uint32_t n = listVisible<ITEMS, LDS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
+		if (lane == 0) sCnt[b][wave] = n;
 		if (tid == 0) *sTicket = takeTicket(P, shard);
 		__syncthreads();
 
 		// the next tile's loads, in flight through this tile's look-back and stores
 		const uint32_t tn = uniform(*sTicket);
 		const bool more = tn < P.totalWork;
-		TileDesc Tn{};
-		float4 spN[ITEMS];
-		uint32_t miN[ITEMS];
+		const TileDesc Tc = T;
 		if (more) {
-			Tn = loadTile(J, tn, BLOCK * ITEMS);
-			loadTileItems<ITEMS>(spheres, meshIndex, Tn, wave * WAVE_ITEMS + lane, spN, miN);
+			T = loadTile(J, tn, BLOCK * ITEMS);
+			loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
 		}
-
-		if (wave == 0) {
-			uint32_t total = 0;
-			for (int q = 0; q < WAVES; q++)
-				for (int j = 0; j < ITEMS; j++) total += sCnt[b][q][j];
-			uint64_t* chain = P.status;
-			uint32_t excl = 0;
-			if (T.first) {
-				if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
-			} else {
-				if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
-				excl = lookBackWave(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch}, lane);
-				if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
-			}
-			if (lane == 0) {
-				sExcl[b] = excl;
-				if (T.last && T.k < J.numStateSets) globalMut<uint32_t>(J.counts)[T.k] = excl + total;
-			}
-		}
+		if (wave == 0) tileOffset<WAVES>(P, J, Tc, epoch, sCnt[b], &sExcl[b], lane);
 		__syncthreads();
 
-		uint32_t pos = T.segBase + sExcl[b];
-		for (uint32_t q = 0; q < wave; q++)
-			for (int j = 0; j < ITEMS; j++) pos += sCnt[b][q][j];
-		pos = uniform(pos);
-#pragma unroll
-		for (int j = 0; j < ITEMS; j++) {
-			const uint32_t n = uint32_t(__builtin_popcountll(mask[j]));
-			if (n == 0) continue;
-			if ((mask[j] >> lane) & 1ull) {
-				uint32_t count, first, vofs;
-				meshCommand<LDS>(meshes, mi[j], sp[j].w, vz[j], V, count, first, vofs);
-				const uint32_t r = maskRank(mask[j]);
-				if (pos + r < J.commandStride) {
-					const gmut<uint32_t> o = out + uint64_t(pos) * 5ull + uint64_t(r * 5u);
-					o[0] = count;
-					o[1] = 1u;
-					o[2] = first;
-					o[3] = vofs;
-					o[4] = T.start + wave * WAVE_ITEMS + j * 64 + lane;
-				}
-			}
-			pos = uniform(pos + n);
-		}
+		if (!more && wave == WAVES - 1 && lane == 0) leaveLaunch(P, shard, epoch);  // as in cullViewTile
+
+		uint32_t pos = Tc.segBase + sExcl[b];
+		for (uint32_t q = 0; q < wave; q++) pos += sCnt[b][q];
+		storeListed<LDS>(run, n, uniform(pos), Tc.start + wave * WAVE_ITEMS, meshes, meshIndex, out, J.commandStride,
+		                 lane);
 		if (!more) break;
-		T = Tn;
-#pragma unroll
-		for (int j = 0; j < ITEMS; j++) {
-			sp[j] = spN[j];
-			mi[j] = miN[j];
-		}
 	}
 }
 
@@ -961,7 +969,8 @@ __global__ __launch_bounds__(BLOCK) void cullViewLoopKernel(CullParams P)
 {
 	constexpr int WAVES = BLOCK / 64;
 	__shared__ uint32_t sTicket;
-	__shared__ uint32_t sCnt[2][WAVES][ITEMS];
+	__shared__ uint32_t sRun[WAVES][64 * ITEMS];
+	__shared__ uint32_t sCnt[2][WAVES];
 	__shared__ uint32_t sExcl[2];
 	__shared__ uint32_t sMeshes[16 * kLdsMeshes];
 
@@ -975,15 +984,16 @@ __global__ __launch_bounds__(BLOCK) void cullViewLoopKernel(CullParams P)
 	const uint32_t t = uniform(sTicket);
 	__syncthreads();  // every wave has read the first ticket before the loop rewrites it
 	const MeshTable meshes{sMeshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
-	if (t < P.totalWork) {
-		if (ldsMeshes)
-			cullViewTiles<BLOCK, ITEMS, true>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, tid, lane, wave);
-		else
-			cullViewTiles<BLOCK, ITEMS, false>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, tid, lane, wave);
+	if (t >= P.totalWork) {
+		if (tid == 0) leaveLaunch(P, shard, epoch);
+		return;
 	}
-
-	__syncthreads();
-	if (tid == 0) leaveLaunch(P, shard, epoch);
+	if (ldsMeshes)
+		cullViewTiles<BLOCK, ITEMS, true>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, sRun[wave], tid, lane,
+		                                  wave);
+	else
+		cullViewTiles<BLOCK, ITEMS, false>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, sRun[wave], tid, lane,
+		                                   wave);
 }
 
 // The fused kernel is latency-bound (a chain of dependent loads per item), so
@@ -1451,18 +1461,21 @@ struct KernelEntry {
 	KernelFn viewLoop;    // one view, persistent (cullViewLoopKernel), or nullptr where it is not faster
 };
 
-// viewLoop where it measured faster at 10M drawables (one view of the full10m
-// scene): not at 512 x 2/8/16, and 1024 x 16's loop form spills registers.
+// viewLoop where it measured faster than one tile per workgroup (10M
+// drawables, 64 StateSets, one view, 18% visible): 1024 x 2 / 4 / 8 74.0 / 62.5
+// / 58.8 against 94.6 / 67.0 / 59.6 us; not at 256 x 4 / 8 / 16 (67.5 / 65.0 /
+// 63.3 against 63.9 / 61.5 / 63.0) nor 512 x 4 (61.7 against 62.0, no more than
+// runs differ), where several workgroups of a CU overlap each other's phases.
 // fusedBatch reads parents whole (COOP) at 256 x 8 and 512 x 4, where it
 // measured faster on uneven64 (2.39 -> 2.32 and 2.93 -> 2.84 ms); at 256 x 4
 // its registers cost a wave per SIMD (2.38 -> 2.60 ms)
 const KernelEntry kKernels[] = {
-    {256, 2, cullKernel<256, 2, false>, cullViewKernel<256, 2>, cullFusedKernel<256, 2, 4>, nullptr, cullViewLoopKernel<256, 2>},
-    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true>, cullViewLoopKernel<256, 4>},
-    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true>, cullViewLoopKernel<256, 8>},
-    {256, 16, cullKernel<256, 16, false>, cullViewKernel<256, 16>, cullFusedKernel<256, 16, 1>, nullptr, cullViewLoopKernel<256, 16>},
+    {256, 2, cullKernel<256, 2, false>, cullViewKernel<256, 2>, cullFusedKernel<256, 2, 4>, nullptr, nullptr},
+    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true>, nullptr},
+    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true>, nullptr},
+    {256, 16, cullKernel<256, 16, false>, cullViewKernel<256, 16>, cullFusedKernel<256, 16, 1>, nullptr, nullptr},
     {512, 2, cullKernel<512, 2, false>, cullViewKernel<512, 2>, cullFusedKernel<512, 2, 1>, nullptr, nullptr},
-    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, true>, cullViewLoopKernel<512, 4>},
+    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, true>, nullptr},
     {512, 8, nullptr, cullViewKernel<512, 8>, nullptr, nullptr, nullptr},
     {512, 16, nullptr, cullViewKernel<512, 16>, nullptr, nullptr, nullptr},
     {1024, 1, nullptr, cullViewKernel<1024, 1>, cullFusedKernel<1024, 1, 1>, nullptr, cullViewLoopKernel<1024, 1>},

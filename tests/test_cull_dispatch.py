@@ -61,3 +61,26 @@ def test_ticket_shards(gpu, tiles, K, block, items):
     print(f"{n} drawables, {K} StateSets, {block}x{items}", flush=True)
     _run([(n, K, 64, 1)], block, items, lambda b: b.run_view())
     _run([(n, K, 64, 1)], block, items, lambda b: b.run())
+
+
+# a wave's list of visible items: empty, full, one over a chunk of 64 commands; mesh tables on both sides of the
+# staged size; the persistent loop (1024 x 8 past 256 tiles)
+@pytest.mark.parametrize("block,items,n,K", [(256, 2, 1, 1), (256, 4, 1023, 1), (256, 4, 1025, 2), (512, 16, 8193, 1),
+                                             (1024, 1, 4097, 3), (1024, 8, 8191, 1), (1024, 8, 2_200_003, 5)])
+@pytest.mark.parametrize("meshes", [64, 65])
+def test_one_view_lists(gpu, block, items, n, K, meshes):
+    print(f"{n} drawables, {K} StateSets, {meshes} meshes, {block}x{items}", flush=True)
+    eye, up = (0.0, 0.0, 2500.0), (0.0, 1.0, 0.0)
+    views = cull.make_views([scenes.Camera(eye, (0.0, 0.0, d), up, 1.2, 1.0, 0.1, 6000.0, 1080.0, (40.0, 8.0, 0.5))
+                             for d in (-1.0, 1.0)] + scenes.random_cameras(5, 20, 0, 2, 100.0))
+    (ds, _, out, spheres, scene), = _jobs([(n, K, meshes, 1)])
+    for v in range(len(views)):  # everything, nothing, and two parts
+        view = views[v:v + 1].copy()
+        batch = cull.CullBatch(cull.make_config(block, items), [(ds, view, out)])
+        batch.run_view()
+        synchronize()
+        batch.workspace.check()
+        _check([(ds, view, out, spheres, scene)], f"{block}x{items} view {v}")
+        batch.close()
+    out.close()
+    ds.close()
