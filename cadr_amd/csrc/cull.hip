@@ -80,8 +80,8 @@ struct LeafParams {
 
 struct CullParams {
 	const cadrCullJob* jobs;
-	const uint32_t* firstWork;   // [numJobs+1] prefix of numTiles
-	const uint64_t* statusBase;  // [numJobs] prefix of numViews*numTiles
+	const uint32_t* firstWork;   // [numJobs+1] prefix of the jobs' work items, more than kInlineJobs jobs only
+	const uint64_t* statusBase;  // [numJobs] prefix of numViews*numTiles, likewise
 	uint64_t* status;
 	uint32_t* ctl;
 	uint32_t shardShift;  // log2 of the ticket shards; beside ctl, so that the first ticket waits for one load
@@ -1008,6 +1008,103 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 
 // ------------------------------------------------------- many views, jobs
 
+// Work items of a job in a batched launch: its tiles, plus one more per
+// extra view group for each of its last splitTiles tiles (the kernel's rule).
+// The host checks that a launch's total fits 32 bits.
+__host__ __device__ __forceinline__ uint64_t jobWorkItems(uint32_t numTiles, uint32_t numViews, uint32_t splitTiles)
+{
+	const uint64_t groups = (uint64_t(numViews) + kViewGroup - 1) / kViewGroup;
+	const uint64_t split = groups > 1 ? (numTiles < splitTiles ? numTiles : splitTiles) : 0u;
+	return numTiles + split * (groups - 1);
+}
+
+// Where each job's work items and status words begin.  Up to kInlineJobs jobs
+// every workgroup works the offsets out for itself at its start, one wave
+// with lanes as jobs, from the same descriptors: about 1 us of a workgroup's
+// time, where a kernel of its own before the batched one cost 4-5 us of every
+// launch.  More jobs take that kernel (cullSetupKernel).
+constexpr uint32_t kInlineJobs = 256;
+
+struct JobOffsets {
+	uint32_t firstWork[kInlineJobs];
+	uint64_t statusBase[kInlineJobs];
+};
+
+// Fills O (wave 0; a barrier must follow before it is read).
+__device__ __forceinline__ void findJobOffsets(const CullParams& P, JobOffsets& O, uint32_t lane)
+{
+	uint32_t runW = 0;
+	uint64_t runS = 0;
+	for (uint32_t base = 0; base < P.numJobs; base += 64u) {
+		const uint32_t j = base + lane;
+		uint32_t w = 0;
+		uint64_t st = 0;
+		if (j < P.numJobs) {
+			const gptr<uint32_t> q = globalPtr<uint32_t>(addr(P.jobs) + uint64_t(j) * sizeof(cadrCullJob) + 56);
+			const uint32_t tiles = q[1], views = q[3];
+			w = uint32_t(jobWorkItems(tiles, views, P.splitTiles));
+			st = uint64_t(views) * tiles;
+		}
+		uint32_t wi = w;
+		uint64_t si = st;
+#pragma unroll
+		for (int off = 1; off < 64; off <<= 1) {
+			const uint32_t a = __shfl_up(wi, off);
+			const uint64_t b = __shfl_up(si, off);
+			if (lane >= uint32_t(off)) {
+				wi += a;
+				si += b;
+			}
+		}
+		if (j < P.numJobs) {
+			O.firstWork[j] = runW + wi - w;
+			O.statusBase[j] = runS + si - st;
+		}
+		runW += __shfl(wi, 63);
+		runS += __shfl(si, 63);
+	}
+}
+
+// The job of work item w, the last one whose items begin at or before it:
+// with lanes as jobs where the offsets are inline, else by bisection upward
+// from `job` (a workgroup's tickets only grow).
+__device__ __forceinline__ uint32_t jobOfWork(const CullParams& P, const JobOffsets& O, uint32_t w, uint32_t job,
+                                              uint32_t lane)
+{
+	if (P.numJobs == 1) return 0;
+	if (P.numJobs <= kInlineJobs) {
+		uint32_t n = 0;
+		for (uint32_t base = 0; base < P.numJobs; base += 64u) {
+			const uint32_t j = base + lane;
+			n += uint32_t(__builtin_popcountll(__ballot(j < P.numJobs && O.firstWork[j] <= w)));
+		}
+		return uniform(n - 1u);
+	}
+	uint32_t lo = job, hi = P.numJobs - 1;
+	while (lo < hi) {
+		const uint32_t mid = (lo + hi + 1) / 2;
+		if (constPtr<uint32_t>(addr(P.firstWork))[mid] <= w) lo = mid; else hi = mid - 1;
+	}
+	return uniform(lo);
+}
+
+__device__ __forceinline__ uint32_t firstWorkOf(const CullParams& P, const JobOffsets& O, uint32_t job)
+{
+	if (P.numJobs == 1) return 0;
+	if (P.numJobs <= kInlineJobs) return uniform(O.firstWork[job]);
+	return constPtr<uint32_t>(addr(P.firstWork))[job];
+}
+
+__device__ __forceinline__ uint64_t statusBaseOf(const CullParams& P, const JobOffsets& O, uint32_t job)
+{
+	if (P.numJobs == 1) return 0;
+	if (P.numJobs <= kInlineJobs) {
+		const uint64_t v = O.statusBase[job];
+		return uint64_t(uniform(uint32_t(v))) | (uint64_t(uniform(uint32_t(v >> 32))) << 32);
+	}
+	return constPtr<uint64_t>(addr(P.statusBase))[job];
+}
+
 template <int BLOCK, int ITEMS>
 struct CullShared {
 	static constexpr int WAVES = BLOCK / 64;
@@ -1021,6 +1118,7 @@ struct CullShared {
 	float red2[WAVES];
 	uint32_t bad[WAVES];
 	uint32_t ticket;
+	JobOffsets offsets;
 };
 
 // COOP (fused form only): parent matrices read whole, 16 per instruction
@@ -1041,6 +1139,8 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	const Shard shard = homeShard<S::TILE>(P);
 	uint32_t job = 0, stagedJob = ~0u;
+	// the first ticket's barrier stands between this and the first use
+	if (wave == 0 && P.numJobs > 1 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
 
 	for (;;) {
 		if (tid == 0) sh.ticket = takeTicket(P, shard);
@@ -1048,20 +1148,12 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		const uint32_t w = uniform(sh.ticket);
 		if (w >= P.totalWork) break;
 
-		// job of this ticket: tickets only grow, so search upward from the last job
-		{
-			uint32_t lo = job, hi = P.numJobs - 1;
-			while (lo < hi) {
-				const uint32_t mid = (lo + hi + 1) / 2;
-				if (constPtr<uint32_t>(addr(P.firstWork))[mid] <= w) lo = mid; else hi = mid - 1;
-			}
-			job = uniform(lo);
-		}
+		job = jobOfWork(P, sh.offsets, w, job, lane);
 		const cadrCullJob J = loadJob(P.jobs, job);
 		// the work item: a whole tile for every view, or, among the job's last
 		// split tiles, one tile for one group of views (tile-major, so a
 		// tile's look-back predecessors still hold earlier tickets)
-		const uint32_t u = w - constPtr<uint32_t>(addr(P.firstWork))[job];
+		const uint32_t u = w - firstWorkOf(P, sh.offsets, job);
 		const uint32_t groups = J.numViews / kViewGroup + (J.numViews % kViewGroup != 0u ? 1u : 0u);
 		const uint32_t split = groups > 1 ? min(J.numTiles, P.splitTiles) : 0u;
 		const uint32_t whole = J.numTiles - split;
@@ -1196,7 +1288,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		const bool emptyTile = T.count == 0;
 
 		const uint64_t views = J.views;
-		uint64_t* chain0 = P.status + constPtr<uint64_t>(addr(P.statusBase))[job];
+		uint64_t* chain0 = P.status + statusBaseOf(P, sh.offsets, job);
 
 		for (uint32_t g0 = gBegin; g0 < gEnd; g0 += kViewGroup) {
 			const uint32_t vg = uniform(min(kViewGroup, J.numViews - g0));
@@ -1355,18 +1447,8 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 	if (tid == 0) leaveLaunch(P, shard, epoch);
 }
 
-// Work items of a job in a batched launch: its tiles, plus one more per
-// extra view group for each of its last splitTiles tiles (the kernel's rule).
-// The host checks that a launch's total fits 32 bits.
-__host__ __device__ __forceinline__ uint64_t jobWorkItems(uint32_t numTiles, uint32_t numViews, uint32_t splitTiles)
-{
-	const uint64_t groups = (uint64_t(numViews) + kViewGroup - 1) / kViewGroup;
-	const uint64_t split = groups > 1 ? (numTiles < splitTiles ? numTiles : splitTiles) : 0u;
-	return numTiles + split * (groups - 1);
-}
-
-// Job offsets for a batched launch (prefix sums over jobs); one block, before
-// the cull kernel on the same stream.
+// Job offsets of a batched launch of more than kInlineJobs jobs (prefix sums
+// over jobs); one block, before the cull kernel on the same stream.
 __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __restrict__ jobs, uint32_t numJobs,
                                                        uint32_t splitTiles, uint32_t* __restrict__ firstWork,
                                                        uint64_t* __restrict__ statusBase)
@@ -1732,10 +1814,12 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 
 	hipStream_t s = hipStream_t(stream);
 	const auto* jobs = reinterpret_cast<const cadrCullJob*>(deviceJobs);
-	hipLaunchKernelGGL(cullSetupKernel, dim3(1), dim3(256), 0, s, jobs, numJobs, splitTiles, ws->firstWork,
-	                   ws->statusBase);
-	CADR_CHECK_HIP(hipGetLastError(), "cullSetupKernel launch");
 	if (totalWork == 0) CADR_RETURN_NO_LAUNCH(s);
+	if (numJobs > kInlineJobs) {
+		hipLaunchKernelGGL(cullSetupKernel, dim3(1), dim3(256), 0, s, jobs, numJobs, splitTiles, ws->firstWork,
+		                   ws->statusBase);
+		CADR_CHECK_HIP(hipGetLastError(), "cullSetupKernel launch");
+	}
 	if (grid > totalWork) grid = totalWork;
 	CullParams p{};
 	p.jobs = jobs;

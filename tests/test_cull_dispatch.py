@@ -84,3 +84,12 @@ def test_one_view_lists(gpu, block, items, n, K, meshes):
         batch.close()
     out.close()
     ds.close()
+
+
+# job offsets: worked out by the workgroups in chunks of 64 jobs, by a kernel of their own past 256
+@pytest.mark.parametrize("jobs", [2, 64, 65, 256, 257])
+def test_job_offsets(gpu, jobs):
+    print(f"{jobs} jobs", flush=True)
+    specs = [(1 + (j * 37) % 90 + (600 if j % 50 == 3 else 0), 1 + j % 3, 8, 1 + (67 if j == 1 else j % 4))
+             for j in range(jobs)]
+    _run(specs, 256, 2, lambda b: b.run())
