@@ -88,6 +88,7 @@ struct CullParams {
 	uint32_t numJobs;
 	uint32_t totalWork;
 	uint32_t splitTiles;  // batched: a job's last tiles handed out per view group
+	uint32_t groupShift;  // batched: log2 of the views of such a group
 	uint32_t flags;
 	uint64_t waitLimit;                 // steady-counter ticks a look-back may wait
 	LeafParams leaf;                    // one-view fused kernel
@@ -439,10 +440,15 @@ __device__ __forceinline__ Shard homeShard(const CullParams& P)
 	return Shard{P.shardShift, (blockIdx.x >> 3) & ((1u << P.shardShift) - 1u)};
 }
 
+// Work item of ticket r of a shard.
+__device__ __forceinline__ uint32_t itemOfTicket(Shard s, uint32_t r)
+{
+	return ((((r >> 3) << s.shift) + s.g) << 3) + (r & 7u);
+}
+
 __device__ __forceinline__ uint32_t takeTicket(const CullParams& P, Shard s)
 {
-	const uint32_t r = atomicAdd(&P.ctl[kCtlShard + 64u * s.g], 1u);
-	return ((((r >> 3) << s.shift) + s.g) << 3) + (r & 7u);
+	return itemOfTicket(s, atomicAdd(&P.ctl[kCtlShard + 64u * s.g], 1u));
 }
 
 // Called by one thread of each workgroup when it leaves: the last one of the
@@ -532,6 +538,42 @@ __device__ uint32_t lookBackWave(const uint64_t* chain, uint32_t c, const WaitBo
 		excl += v;
 		if (f < 64u) break;
 		p -= 64;
+	}
+	return excl;
+}
+
+// lookBackWave for 64 / W chains at once: each run of W lanes walks its own
+// chain with a window of W predecessors.  c is the lane's chain's position
+// (0: nothing before it); returns the lane's chain's prefix.
+template <uint32_t W>
+__device__ uint32_t lookBackGroups(const uint64_t* chain, uint32_t c, const WaitBound& B, uint32_t lane)
+{
+	static_assert(W >= 2 && W <= 32 && (W & (W - 1)) == 0, "lanes a chain");
+	constexpr uint32_t kAll = W == 32 ? ~0u : (1u << (W & 31u)) - 1u;
+	const uint32_t l = lane & (W - 1u), shift = lane & ~(W - 1u);
+	uint32_t excl = 0;
+	int64_t p = c;
+	uint64_t start = 0;
+	while (__ballot(p > 0) != 0ull) {
+		const int64_t idx = p - 1 - int64_t(l);
+		const uint64_t s = idx >= 0 ? readStatus(chain + idx) : packStatus(B.epoch, kStatePrefix, 0);
+		const bool ready = statusReady(s, B.epoch);
+		const uint32_t pmask = uint32_t(__ballot(ready && (uint32_t(s) >> 30) == kStatePrefix) >> shift) & kAll;
+		const uint32_t nmask = uint32_t(__ballot(!ready) >> shift) & kAll;
+		const uint32_t f = pmask ? uint32_t(__builtin_ctz(pmask)) : W;
+		const uint32_t need = f + 1u >= W ? kAll : ((2u << f) - 1u);
+		const bool wait = p > 0 && (nmask & need) != 0u;
+		uint32_t v = l <= f ? (uint32_t(s) & kValueMask) : 0u;
+#pragma unroll
+		for (uint32_t off = W / 2; off >= 1; off >>= 1) v += __shfl_xor(v, int(off));
+		if (!wait && p > 0) {
+			excl += v;
+			p = f < W ? 0 : p - int64_t(W);
+		}
+		if (__ballot(wait) != 0ull) {
+			if (uniform(uint32_t(waitGiveUp(B, start)))) return excl;
+			__builtin_amdgcn_s_sleep(1);
+		}
 	}
 	return excl;
 }
@@ -736,15 +778,16 @@ __device__ __forceinline__ void propagateTileItems(const LeafParams& Lf, const c
 // ---------------------------------------------------------------- one view
 
 // A wave's visible items as a compact list in its own LDS, in drawable order:
-// item index in the wave's run (10 bits), the LOD its projected radius
-// selects before the mesh's own limit (2 bits) and, for a staged mesh table,
-// the mesh (6 bits).  The command stores then run with full lanes: in
+// item index in the wave's run (11 bits), the LOD its projected radius
+// selects before the mesh's own limit (2 bits) and the mesh (19 bits; the
+// meshes of a larger table are read again).  The command stores then run with full lanes: in
 // drawable order a wave stored its items one by one, each with the few lanes
 // that are visible, and the CU's address path, which takes a store
 // instruction's 64 lanes whether they are active or not, bound the views that
 // see a part of everything (10M drawables, 25% visible in every item: 49 MB
 // of commands cost 57 of 85 us).
-constexpr uint32_t kRunLodShift = 10, kRunMeshShift = 12;
+constexpr uint32_t kRunLodShift = 11, kRunMeshShift = 13;
+constexpr uint32_t kRunMeshes = 1u << (32 - kRunMeshShift);
 
 // LOD index by projected radius alone (lodAtDepth before the mesh's limit).
 __device__ __forceinline__ uint32_t lodByRadius(float r, float vz, const ViewC& v)
@@ -755,7 +798,7 @@ __device__ __forceinline__ uint32_t lodByRadius(float r, float vz, const ViewC& 
 
 // Tests the wave's items (first item `base` of the tile) and lists the
 // visible ones; returns their number (the same in every lane).
-template <int ITEMS, bool LDS>
+template <int ITEMS>
 __device__ __forceinline__ uint32_t listVisible(const float4 (&sp)[ITEMS], const uint32_t (&mi)[ITEMS],
                                                 const TileDesc& T, uint32_t numMeshes, const ViewC& V, uint32_t base,
                                                 uint32_t lane, uint32_t* run)
@@ -769,7 +812,7 @@ __device__ __forceinline__ uint32_t listVisible(const float4 (&sp)[ITEMS], const
 		const uint64_t mask = __ballot(vis);
 		if (vis) {
 			const uint32_t lod = lodByRadius(sp[j].w, viewCoord(V.r2, sp[j]), V);
-			run[n + maskRank(mask)] = (j * 64 + lane) | (lod << kRunLodShift) | (LDS ? mi[j] << kRunMeshShift : 0u);
+			run[n + maskRank(mask)] = (j * 64 + lane) | (lod << kRunLodShift) | (mi[j] << kRunMeshShift);
 		}
 		n = uniform(n + uint32_t(__builtin_popcountll(mask)));
 	}
@@ -781,8 +824,8 @@ __device__ __forceinline__ uint32_t listVisible(const float4 (&sp)[ITEMS], const
 // wave's item 0.
 template <bool LDS>
 __device__ __forceinline__ void storeListed(const uint32_t* run, uint32_t n, uint32_t pos, uint32_t first,
-                                            const MeshTable& M, gptr<uint32_t> meshIndex, gmut<uint32_t> out,
-                                            uint32_t stride, uint32_t lane)
+                                            const MeshTable& M, uint32_t numMeshes, gptr<uint32_t> meshIndex,
+                                            gmut<uint32_t> out, uint32_t stride, uint32_t lane)
 {
 	waveSync();  // the list is written by other lanes
 	for (uint32_t c = 0; c < n; c += 64u) {
@@ -798,11 +841,15 @@ __device__ __forceinline__ void storeListed(const uint32_t* run, uint32_t n, uin
 			firstIndex = M.field(12 + lod, m);
 			vofs = M.field(5, m);
 		} else {
-			const gptr<cadrMesh> mesh = M.mem + meshIndex[drawable];
-			const uint32_t lod = min(raw, maxLodOf(mesh->lodCount));
-			count = mesh->indexCount[lod];
-			firstIndex = mesh->firstIndex[lod];
-			vofs = uint32_t(mesh->vertexOffset);
+			// the whole record at once, so that one round trip serves the LOD limit and its fields
+			const uint32_t m = numMeshes <= kRunMeshes ? e >> kRunMeshShift : meshIndex[drawable];
+			const gptr<uint4> q = reinterpret_cast<gptr<uint4>>(M.mem + m);
+			const uint4 head = make_uint4(q[1].x, q[1].y, q[1].z, q[1].w);  // lodCount, vertexOffset
+			const uint4 c4 = make_uint4(q[2].x, q[2].y, q[2].z, q[2].w), f4 = make_uint4(q[3].x, q[3].y, q[3].z, q[3].w);
+			const uint32_t lod = min(raw, maxLodOf(head.x));
+			count = lod == 0u ? c4.x : lod == 1u ? c4.y : lod == 2u ? c4.z : c4.w;
+			firstIndex = lod == 0u ? f4.x : lod == 1u ? f4.y : lod == 2u ? f4.z : f4.w;
+			vofs = head.y;
 		}
 		const gmut<uint32_t> o = out + uint64_t(pos + i) * 5ull;
 		o[0] = count;
@@ -858,7 +905,7 @@ __device__ __forceinline__ void cullViewTile(const CullParams& P, const cadrCull
 		propagateTileItems<ITEMS, LDS>(P.leaf, J, T, wave * WAVE_ITEMS, lane, sMat, meshes, sp, mi);
 	else
 		loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
-	const uint32_t n = listVisible<ITEMS, LDS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
+	const uint32_t n = listVisible<ITEMS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
 	if (lane == 0) sCnt[wave] = n;
 	__syncthreads();
 	if (wave == 0) tileOffset<WAVES>(P, J, T, epoch, sCnt, sExclP, lane);
@@ -870,7 +917,7 @@ __device__ __forceinline__ void cullViewTile(const CullParams& P, const cadrCull
 
 	uint32_t pos = T.segBase + *sExclP;
 	for (uint32_t q = 0; q < wave; q++) pos += sCnt[q];
-	storeListed<LDS>(run, n, uniform(pos), T.start + wave * WAVE_ITEMS, meshes, meshIndex,
+	storeListed<LDS>(run, n, uniform(pos), T.start + wave * WAVE_ITEMS, meshes, J.numMeshes, meshIndex,
 	                 globalMut<uint32_t>(J.commands), J.commandStride, lane);
 }
 
@@ -938,7 +985,7 @@ __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCul
 	uint32_t mi[ITEMS];
 	loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
 	for (uint32_t b = 0;; b ^= 1u) {
-		const uint32_t n = listVisible<ITEMS, LDS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
+		const uint32_t n = listVisible<ITEMS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
 		if (lane == 0) sCnt[b][wave] = n;
 		if (tid == 0) *sTicket = takeTicket(P, shard);
 		__syncthreads();
@@ -958,8 +1005,8 @@ __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCul
 
 		uint32_t pos = Tc.segBase + sExcl[b];
 		for (uint32_t q = 0; q < wave; q++) pos += sCnt[b][q];
-		storeListed<LDS>(run, n, uniform(pos), Tc.start + wave * WAVE_ITEMS, meshes, meshIndex, out, J.commandStride,
-		                 lane);
+		storeListed<LDS>(run, n, uniform(pos), Tc.start + wave * WAVE_ITEMS, meshes, J.numMeshes, meshIndex, out,
+		                 J.commandStride, lane);
 		if (!more) break;
 	}
 }
@@ -1009,13 +1056,40 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 // ------------------------------------------------------- many views, jobs
 
 // Work items of a job in a batched launch: its tiles, plus one more per
-// extra view group for each of its last splitTiles tiles (the kernel's rule).
+// extra view group for each of its last splitTiles tiles (workItem's rule).
 // The host checks that a launch's total fits 32 bits.
-__host__ __device__ __forceinline__ uint64_t jobWorkItems(uint32_t numTiles, uint32_t numViews, uint32_t splitTiles)
+__host__ __device__ __forceinline__ uint64_t jobWorkItems(uint32_t numTiles, uint32_t numViews, uint32_t splitTiles,
+                                                          uint32_t groupShift)
 {
-	const uint64_t groups = (uint64_t(numViews) + kViewGroup - 1) / kViewGroup;
+	const uint64_t groups = (uint64_t(numViews) + (1u << groupShift) - 1) >> groupShift;
 	const uint64_t split = groups > 1 ? (numTiles < splitTiles ? numTiles : splitTiles) : 0u;
 	return numTiles + split * (groups - 1);
+}
+
+// Item u of a job: a whole tile for every view, or, among the job's last
+// split tiles, one tile for one group of views (tile-major, so a tile's
+// look-back predecessors still hold earlier tickets).
+// Every field is made explicitly uniform: view constants loaded by an index
+// that the compiler cannot prove uniform go to vector registers (measured:
+// 216 against 159 registers, 2.5M drawables x 256 views 600 against 397 us).
+struct WorkItem {
+	uint32_t tile, viewBegin, viewEnd;
+};
+
+__device__ __forceinline__ WorkItem workItem(const CullParams& P, const cadrCullJob& J, uint32_t u)
+{
+	const uint32_t g = 1u << P.groupShift;
+	const uint32_t groups = (J.numViews >> P.groupShift) + ((J.numViews & (g - 1u)) != 0u ? 1u : 0u);
+	const uint32_t split = groups > 1 ? min(J.numTiles, P.splitTiles) : 0u;
+	const uint32_t whole = J.numTiles - split;
+	uint32_t t = u, begin = 0, end = J.numViews;
+	if (u >= whole) {
+		const uint32_t q = u - whole;
+		t = whole + q / groups;
+		begin = (q % groups) << P.groupShift;
+		end = begin + min(J.numViews - begin, g);
+	}
+	return WorkItem{uniform(t), uniform(begin), uniform(end)};
 }
 
 // Where each job's work items and status words begin.  Up to kInlineJobs jobs
@@ -1042,7 +1116,7 @@ __device__ __forceinline__ void findJobOffsets(const CullParams& P, JobOffsets& 
 		if (j < P.numJobs) {
 			const gptr<uint32_t> q = globalPtr<uint32_t>(addr(P.jobs) + uint64_t(j) * sizeof(cadrCullJob) + 56);
 			const uint32_t tiles = q[1], views = q[3];
-			w = uint32_t(jobWorkItems(tiles, views, P.splitTiles));
+			w = uint32_t(jobWorkItems(tiles, views, P.splitTiles, P.groupShift));
 			st = uint64_t(views) * tiles;
 		}
 		uint32_t wi = w;
@@ -1105,6 +1179,116 @@ __device__ __forceinline__ uint64_t statusBaseOf(const CullParams& P, const JobO
 	return constPtr<uint64_t>(addr(P.statusBase))[job];
 }
 
+// Jobs of few views: the batched kernel without what only many views pay
+// for.  No tile sphere, no visibility bits kept per view: the workgroup lists
+// its visible items for CH views at a time, wave 0 looks all CH chains back
+// at once, and the commands are stored from the lists.  It holds half the
+// batched kernel's registers, so twice its workgroups are resident to overlap
+// their chains of round trips.  Persistent, like the batched kernel; a mesh
+// table is staged only where the launch has one job.
+template <int BLOCK, int ITEMS, int CH>
+struct FewShared {
+	static constexpr int WAVES = BLOCK / 64;
+	uint32_t run[WAVES][CH][64 * ITEMS];
+	uint32_t meshes[16 * kLdsMeshes];
+	JobOffsets offsets;
+	uint32_t cnt[2][CH][WAVES];
+	uint32_t excl[2][CH];
+	uint32_t ticket[2];
+};
+
+template <int BLOCK, int ITEMS, int CH, bool LDS>
+__device__ __forceinline__ void cullFewTile(const CullParams& P, const cadrCullJob& J, const TileDesc& T,
+                                            uint32_t viewBegin, uint32_t viewEnd, uint64_t* chain0, uint32_t epoch, const MeshTable& meshes, FewShared<BLOCK, ITEMS, CH>& sh,
+                                            uint32_t& b, uint32_t lane, uint32_t wave)
+{
+	constexpr int WAVES = BLOCK / 64, WAVE_ITEMS = 64 * ITEMS;
+	constexpr uint32_t W = 64 / CH;  // lanes of a view in the look-back
+	const gptr<uint32_t> meshIndex = globalPtr<uint32_t>(J.meshIndex);
+	float4 sp[ITEMS];
+	uint32_t mi[ITEMS];
+	loadTileItems<ITEMS>(globalPtr<float4>(J.spheres), meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
+	for (uint32_t v0 = viewBegin; v0 < viewEnd; v0 += CH, b ^= 1u) {
+		uint32_t n[CH];
+#pragma unroll
+		for (int c = 0; c < CH; c++) {
+			n[c] = 0;
+			if (v0 + c < viewEnd) {
+				n[c] = listVisible<ITEMS>(sp, mi, T, J.numMeshes, loadView(J.views, v0 + c), wave * WAVE_ITEMS, lane,
+				                          sh.run[wave][c]);
+				if (lane == 0) sh.cnt[b][c][wave] = n[c];
+			}
+		}
+		__syncthreads();
+		if (wave == 0) {
+			const uint32_t c = lane / W, view = v0 + c;  // the lane's view
+			const bool on = view < viewEnd, lead = on && lane % W == 0u;
+			uint32_t total = 0;
+			if (on)
+				for (int q = 0; q < WAVES; q++) total += sh.cnt[b][c][q];
+			uint64_t* chain = chain0 + uint64_t(on ? view : v0) * J.numTiles;
+			uint32_t excl = 0;
+			if (T.first) {
+				if (lead) publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
+			} else {
+				if (lead) publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
+				const WaitBound B{P.ctl, P.waitLimit, epoch};
+				if constexpr (CH == 1)
+					excl = lookBackWave(chain, T.chain, B, lane);
+				else
+					excl = lookBackGroups<W>(chain, on ? T.chain : 0u, B, lane);
+				if (lead) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
+			}
+			if (lead) {
+				sh.excl[b][c] = excl;
+				if (T.last && T.k < J.numStateSets)
+					globalMut<uint32_t>(J.counts)[uint64_t(view) * J.numStateSets + T.k] = excl + total;
+			}
+		}
+		__syncthreads();
+#pragma unroll
+		for (int c = 0; c < CH; c++) {
+			if (n[c] == 0) continue;
+			uint32_t pos = T.segBase + sh.excl[b][c];
+			for (uint32_t q = 0; q < wave; q++) pos += sh.cnt[b][c][q];
+			storeListed<LDS>(sh.run[wave][c], n[c], uniform(pos), T.start + wave * WAVE_ITEMS, meshes, J.numMeshes,
+			                 meshIndex, globalMut<uint32_t>(J.commands) + uint64_t(v0 + c) * J.commandStride * 5ull,
+			                 J.commandStride, lane);
+		}
+	}
+}
+
+template <int BLOCK, int ITEMS, int CH>
+__global__ __launch_bounds__(BLOCK) void cullFewKernel(CullParams P)
+{
+	__shared__ FewShared<BLOCK, ITEMS, CH> sh;
+	const uint32_t tid = threadIdx.x, lane = laneId(), wave = uniform(tid / 64);
+	const Shard shard = homeShard<BLOCK * ITEMS>(P);
+	uint32_t job = 0, b = 0;
+	if (tid == 0) sh.ticket[0] = takeTicket(P, shard);
+	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	if (wave == 0 && P.numJobs > 1 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
+	bool ldsMeshes = false;
+	if (P.numJobs == 1) ldsMeshes = stageMeshes<BLOCK>(sh.meshes, loadJob(P.jobs, 0), tid);
+	for (uint32_t k = 0;; k ^= 1u) {
+		__syncthreads();
+		const uint32_t t = uniform(sh.ticket[k]);
+		if (t >= P.totalWork) break;
+		job = jobOfWork(P, sh.offsets, t, job, lane);
+		const cadrCullJob J = loadJob(P.jobs, job);
+		const WorkItem item = workItem(P, J, t - firstWorkOf(P, sh.offsets, job));
+		const TileDesc T = loadTile(J, item.tile, BLOCK * ITEMS);
+		uint64_t* chain0 = P.status + statusBaseOf(P, sh.offsets, job);
+		const MeshTable meshes{sh.meshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
+		if (ldsMeshes)
+			cullFewTile<BLOCK, ITEMS, CH, true>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane, wave);
+		else
+			cullFewTile<BLOCK, ITEMS, CH, false>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane, wave);
+		if (tid == 0) sh.ticket[k ^ 1u] = takeTicket(P, shard);
+	}
+	if (tid == 0) leaveLaunch(P, shard, epoch);
+}
+
 template <int BLOCK, int ITEMS>
 struct CullShared {
 	static constexpr int WAVES = BLOCK / 64;
@@ -1150,22 +1334,10 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 
 		job = jobOfWork(P, sh.offsets, w, job, lane);
 		const cadrCullJob J = loadJob(P.jobs, job);
-		// the work item: a whole tile for every view, or, among the job's last
-		// split tiles, one tile for one group of views (tile-major, so a
-		// tile's look-back predecessors still hold earlier tickets)
-		const uint32_t u = w - firstWorkOf(P, sh.offsets, job);
-		const uint32_t groups = J.numViews / kViewGroup + (J.numViews % kViewGroup != 0u ? 1u : 0u);
-		const uint32_t split = groups > 1 ? min(J.numTiles, P.splitTiles) : 0u;
-		const uint32_t whole = J.numTiles - split;
-		uint32_t t = u, gBegin = 0, gEnd = J.numViews;
-		if (u >= whole) {
-			const uint32_t q = u - whole;
-			t = uniform(whole + q / groups);
-			gBegin = uniform((q % groups) * kViewGroup);
-			gEnd = gBegin + min(J.numViews - gBegin, kViewGroup);
-		}
+		const WorkItem item = workItem(P, J, w - firstWorkOf(P, sh.offsets, job));
+		const uint32_t gBegin = item.viewBegin, gEnd = item.viewEnd;
 		const bool storeLeaf = gBegin == 0;
-		const TileDesc T = loadTile(J, t, S::TILE);
+		const TileDesc T = loadTile(J, item.tile, S::TILE);
 		// the job's mesh table is staged once per run of tickets of one job
 		// (every wave left the previous tile's last barrier, so no wave still
 		// reads the old table)
@@ -1291,7 +1463,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		uint64_t* chain0 = P.status + statusBaseOf(P, sh.offsets, job);
 
 		for (uint32_t g0 = gBegin; g0 < gEnd; g0 += kViewGroup) {
-			const uint32_t vg = uniform(min(kViewGroup, J.numViews - g0));
+			const uint32_t vg = uniform(min(kViewGroup, gEnd - g0));
 
 			// tile classes of the group's views, lane v holding view g0+v, and
 			// the views that see part of the tile (every wave computes the same
@@ -1450,7 +1622,8 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 // Job offsets of a batched launch of more than kInlineJobs jobs (prefix sums
 // over jobs); one block, before the cull kernel on the same stream.
 __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __restrict__ jobs, uint32_t numJobs,
-                                                       uint32_t splitTiles, uint32_t* __restrict__ firstWork,
+                                                       uint32_t splitTiles, uint32_t groupShift,
+                                                       uint32_t* __restrict__ firstWork,
                                                        uint64_t* __restrict__ statusBase)
 {
 	__shared__ uint32_t sT[256];
@@ -1463,7 +1636,7 @@ __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __rest
 		uint32_t nt = 0;
 		uint64_t ns = 0;
 		if (j < numJobs) {
-			nt = uint32_t(jobWorkItems(jobs[j].numTiles, jobs[j].numViews, splitTiles));
+			nt = uint32_t(jobWorkItems(jobs[j].numTiles, jobs[j].numViews, splitTiles, groupShift));
 			ns = uint64_t(jobs[j].numViews) * jobs[j].numTiles;
 		}
 		sT[tid] = nt;
@@ -1541,6 +1714,7 @@ struct KernelEntry {
 	KernelFn fused;       // leaf propagation + one view, or nullptr
 	KernelFn fusedBatch;  // leaf propagation + many views / jobs, or nullptr
 	KernelFn viewLoop;    // one view, persistent (cullViewLoopKernel), or nullptr where it is not faster
+	KernelFn few[3];      // few views per job, 1, 2 or 4 at a time (cullFewKernel), or nullptr
 };
 
 // viewLoop where it measured faster than one tile per workgroup (10M
@@ -1552,12 +1726,12 @@ struct KernelEntry {
 // measured faster on uneven64 (2.39 -> 2.32 and 2.93 -> 2.84 ms); at 256 x 4
 // its registers cost a wave per SIMD (2.38 -> 2.60 ms)
 const KernelEntry kKernels[] = {
-    {256, 2, cullKernel<256, 2, false>, cullViewKernel<256, 2>, cullFusedKernel<256, 2, 4>, nullptr, nullptr},
-    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true>, nullptr},
-    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true>, nullptr},
+    {256, 2, cullKernel<256, 2, false>, cullViewKernel<256, 2>, cullFusedKernel<256, 2, 4>, nullptr, nullptr, {cullFewKernel<256, 2, 1>, cullFewKernel<256, 2, 2>, cullFewKernel<256, 2, 4>}},
+    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true>, nullptr, {cullFewKernel<256, 4, 1>, cullFewKernel<256, 4, 2>, cullFewKernel<256, 4, 4>}},
+    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true>, nullptr, {cullFewKernel<256, 8, 1>, cullFewKernel<256, 8, 2>, cullFewKernel<256, 8, 4>}},
     {256, 16, cullKernel<256, 16, false>, cullViewKernel<256, 16>, cullFusedKernel<256, 16, 1>, nullptr, nullptr},
     {512, 2, cullKernel<512, 2, false>, cullViewKernel<512, 2>, cullFusedKernel<512, 2, 1>, nullptr, nullptr},
-    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, true>, nullptr},
+    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, true>, nullptr, {cullFewKernel<512, 4, 1>, cullFewKernel<512, 4, 2>, cullFewKernel<512, 4, 4>}},
     {512, 8, nullptr, cullViewKernel<512, 8>, nullptr, nullptr, nullptr},
     {512, 16, nullptr, cullViewKernel<512, 16>, nullptr, nullptr, nullptr},
     {1024, 1, nullptr, cullViewKernel<1024, 1>, cullFusedKernel<1024, 1, 1>, nullptr, cullViewLoopKernel<1024, 1>},
@@ -1780,6 +1954,29 @@ int checkLeaf(const cadrTransformLevel& L, const cadrCullJob& J, const std::stri
 	return CADR_SUCCESS;
 }
 
+// The few-view kernel for a launch, or nullptr where the many-view kernel
+// (cullKernel) is the faster one.  That one reads a tile once for 64 views and
+// skips the views that see none of it or all of it, but keeps its workgroups
+// long on a tile; the few-view kernel tests every drawable, four views at a
+// time, in many more work items.  Measured at 256 x 8, trees of clustered
+// drawables, few against many: 12 views 4M drawables 93 / 107 us, 2M 53 / 59;
+// 37 views 100k 19 / 39, 333k 33 / 45, 1M 68 / 62; 64 views 333k 43 / 64, 1M
+// 105 / 86; 128 views 100k 33 / 64, 333k 75 / 75.  So few wins up to about 16
+// views a drawable, and for more views up to about 2^25 tests in the launch.
+KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t numJobs, uint32_t flags)
+{
+	uint64_t drawables = 0, tests = 0;
+	uint32_t mostViews = 0;
+	for (uint32_t j = 0; j < numJobs; j++) {
+		drawables += jobs[j].numDrawables;
+		tests += uint64_t(jobs[j].numDrawables) * jobs[j].numViews;
+		mostViews = std::max(mostViews, jobs[j].numViews);
+	}
+	const bool split = (flags & CADR_CULL_WHOLE_TILES) == 0;
+	if (split ? tests > 16 * drawables && tests > (1ull << 25) : mostViews > 4) return nullptr;
+	return ke.few[mostViews <= 1 ? 0 : mostViews == 2 ? 1 : 2];
+}
+
 // One persistent launch of a batched kernel over numJobs jobs; leaves: the
 // fused form's leaf levels (device memory), else null.
 int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config, uint64_t deviceJobs,
@@ -1797,12 +1994,21 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 	uint32_t perCU = config->workgroupsPerCU;
 	if (perCU == 0) perCU = ke.block >= 512 ? 2 : 4;
 	uint64_t grid = uint64_t(cu > 0 ? cu : 256) * perCU;
-	const uint32_t splitTiles = (config->flags & CADR_CULL_WHOLE_TILES) ? 0u : uint32_t(std::min<uint64_t>(grid, 1u << 20));
+	const KernelFn few = leaves ? nullptr : fewKernelFor(ke, hostJobs, numJobs, config->flags);
+	uint32_t splitTiles = uint32_t(std::min<uint64_t>(grid, 1u << 20)), groupShift = 6;
+	if (few) {
+		fn = few;
+		splitTiles = 0xffffffffu;
+		groupShift = 2;
+		if (config->workgroupsPerCU == 0)
+			if (const int resident = residentWorkgroups(few, ke.block)) grid = uint64_t(resident);
+	}
+	if (config->flags & CADR_CULL_WHOLE_TILES) splitTiles = 0;
 	uint64_t totalWork = 0, statusNeed = 0, bytes = 0;
 	for (uint32_t j = 0; j < numJobs; j++) {
 		const int rc = checkJob(hostJobs[j]);
 		if (rc != CADR_SUCCESS) return rc;
-		totalWork += jobWorkItems(hostJobs[j].numTiles, hostJobs[j].numViews, splitTiles);
+		totalWork += jobWorkItems(hostJobs[j].numTiles, hostJobs[j].numViews, splitTiles, groupShift);
 		statusNeed += uint64_t(hostJobs[j].numViews) * hostJobs[j].numTiles;
 		bytes += jobBytes(hostJobs[j], leaves != nullptr);
 	}
@@ -1816,8 +2022,8 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 	const auto* jobs = reinterpret_cast<const cadrCullJob*>(deviceJobs);
 	if (totalWork == 0) CADR_RETURN_NO_LAUNCH(s);
 	if (numJobs > kInlineJobs) {
-		hipLaunchKernelGGL(cullSetupKernel, dim3(1), dim3(256), 0, s, jobs, numJobs, splitTiles, ws->firstWork,
-		                   ws->statusBase);
+		hipLaunchKernelGGL(cullSetupKernel, dim3(1), dim3(256), 0, s, jobs, numJobs, splitTiles,
+		                   groupShift, ws->firstWork, ws->statusBase);
 		CADR_CHECK_HIP(hipGetLastError(), "cullSetupKernel launch");
 	}
 	if (grid > totalWork) grid = totalWork;
@@ -1830,6 +2036,7 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 	p.numJobs = numJobs;
 	p.totalWork = uint32_t(totalWork);
 	p.splitTiles = splitTiles;
+	p.groupShift = groupShift;
 	p.shardShift = shardShiftFor(ke.block * ke.items, grid, totalWork, bytes);
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;

@@ -35,9 +35,9 @@ def _check(jobs, what):
                 assert got[v][k].tobytes() == exp[v][k].tobytes(), f"{what}: view {v} StateSet {k}"
 
 
-def _run(specs, block, items, run):
+def _run(specs, block, items, run, flags=0):
     jobs = _jobs(specs)
-    batch = cull.CullBatch(cull.make_config(block, items), [j[:3] for j in jobs])
+    batch = cull.CullBatch(cull.make_config(block, items, flags=flags), [j[:3] for j in jobs])
     for k in range(2):
         for _, _, out, _, _ in jobs:
             out.counts.fill_u32(0xDEADBEEF)
@@ -93,3 +93,35 @@ def test_job_offsets(gpu, jobs):
     specs = [(1 + (j * 37) % 90 + (600 if j % 50 == 3 else 0), 1 + j % 3, 8, 1 + (67 if j == 1 else j % 4))
              for j in range(jobs)]
     _run(specs, 256, 2, lambda b: b.run())
+
+
+# few views: 1, 2 and 4 at a time, the last group cut off, mesh tables staged (one job) and not; CULL_WHOLE_TILES
+# takes more than four views to the many-view kernel, whose view groups end at 32 and 64
+@pytest.mark.parametrize("block,items", [(256, 2), (256, 4), (256, 8), (512, 4)])
+@pytest.mark.parametrize("flags", [0, N.CULL_WHOLE_TILES])
+@pytest.mark.parametrize("specs", [[(5000, 3, 64, 1)], [(5000, 2, 65, 2), (1, 1, 9, 1), (2049, 4, 300, 2)],
+                                   [(4097, 1, 64, 3)], [(900, 5, 7, 4), (3000, 1, 64, 1)], [(3001, 2, 64, 5)],
+                                   [(2500, 3, 80, 33), (2500, 1, 64, 2)], [(1025, 1, 64, 65)]])
+def test_few_and_many_views(gpu, block, items, flags, specs):
+    print(f"{specs} {block}x{items} flags {flags}", flush=True)
+    _run(specs, block, items, lambda b: b.run(), flags)
+
+
+def test_many_views_boundary_spheres(gpu):
+    """Spheres within ulps of every plane, through the many-view kernel's estimate."""
+    from test_cull import _boundary_spheres
+    rng = np.random.default_rng(3)
+    views = cull.make_views(scenes.random_cameras(11, 20, 0, 8, 100.0))
+    spheres = _boundary_spheres(views, 40, rng)
+    n = spheres.shape[0]
+    scene = scenes.plain_scene(n, num_statesets=1)
+    ds = cull.DeviceScene(scene)
+    ds.upload_spheres(spheres)
+    out = cull.CullOutputs(len(views), n, 1)
+    batch = cull.CullBatch(cull.make_config(256, 8, flags=N.CULL_WHOLE_TILES), [(ds, views, out)])
+    batch.run()
+    synchronize()
+    _check([(ds, views, out, spheres, scene)], "boundary spheres")
+    batch.close()
+    out.close()
+    ds.close()
