@@ -20,7 +20,7 @@
 // over StateSets, so the walks stay short.  Status words are tagged with a
 // launch epoch and never cleared.
 //
-// Four kernels:
+// Five kernels:
 //   cullViewKernel - one view: one workgroup per tile, visibility kept in
 //     registers, a 64-lane parallel look-back in wave 0, each visible
 //     drawable's lane storing its command at its compacted slot.  It resets
@@ -35,10 +35,12 @@
 //     a tile is read from HBM once into registers and tested against all
 //     views of its job, 64 views at a time; lane v of wave 0 walks the chain
 //     of view v; each visible drawable's lane stores its command directly at
-//     its compacted slot.  A conservative bounding sphere of the tile, classified
-//     per view with lanes as views, lets whole (tile, view) pairs skip the
-//     per-drawable test when the tile is wholly outside or inside the
-//     frustum.
+//     its compacted slot.  A conservative bounding sphere of a wave's items,
+//     classified per view with lanes as views, lets whole (wave, view) pairs
+//     skip the per-drawable test when the items are wholly outside or inside
+//     the frustum.
+//   cullFewKernel - jobs of few views, or small launches: work items of one
+//     tile and up to four views, visible items listed per view.
 #include "internal.h"
 #include "launch.h"
 #include "fp32.h"
@@ -267,16 +269,17 @@ __device__ __forceinline__ uint32_t lodAtDepth(float r, float vz, const ViewC& v
 	return lod < maxLod ? lod : maxLod;
 }
 
-// Tile-vs-view class: 0 = test each drawable, 1 = all outside, 2 = all inside.
+// Class of a wave's items in a view: 0 = test each drawable, 1 = all outside,
+// 2 = all inside.
 //
-// ts is a sphere containing every drawable sphere of the tile
-// (|c_i - C| + r_i <= R).  Each quantity the drawable test compares, v.z and
+// ts is a sphere containing every drawable sphere of the wave's part of a
+// tile (|c_i - C| + r_i <= R).  Each quantity the drawable test compares, v.z and
 // g(c) = |v.x|*sideX[0] - v.z*sideX[1] (the larger of two linear plane
 // functions), is Lipschitz in the sphere centre with constant L_P = the
 // largest gradient norm among its linear pieces: |row2| for v.z, and
 // |sideX[0]*row0 -+ sideX[1]*row2| for g (likewise for y), taken at least 1.
-// A drawable's quantity then differs from the tile centre's by at most
-// L*|c_i - C| <= L*(R - r_i), so the tile is wholly outside a plane when the
+// A drawable's quantity then differs from the sphere centre's by at most
+// L*|c_i - C| <= L*(R - r_i), so the items are wholly outside a plane when the
 // centre is outside by more than L*R, and wholly inside when inside by more
 // than L*R.  The norms are rounded up by a relative 2^-12; the margin m,
 // about 2^-14 of the magnitudes involved, is some thousand times the FP32
@@ -289,7 +292,7 @@ __device__ __forceinline__ float norm3(float x, float y, float z)
 	return __builtin_amdgcn_sqrtf((x * x + y * y) + z * z);
 }
 
-__device__ __forceinline__ uint32_t classifyTile(float4 ts, const ViewC& v)
+__device__ __forceinline__ uint32_t classifyItems(float4 ts, const ViewC& v)
 {
 	const float vx = viewCoord(v.r0, ts);
 	const float vy = viewCoord(v.r1, ts);
@@ -1298,9 +1301,6 @@ struct CullShared {
 	uint32_t base[kViewGroup][WAVES];  // a wave's first output slot in its view's StateSet segment
 
 	uint32_t meshes[16 * kLdsMeshes];
-	float red[WAVES][6];
-	float red2[WAVES];
-	uint32_t bad[WAVES];
 	uint32_t ticket;
 	JobOffsets offsets;
 };
@@ -1388,7 +1388,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 			mi[j] = m;
 
 			// a sphere other than a finite one with r >= 0 or the empty sphere
-			// (r = -inf, never visible) disables the tile sphere for this tile
+			// (r = -inf, never visible) disables the wave's sphere
 			if (e < T.count && s.w != -__builtin_inff() &&
 			    !(__builtin_isfinite(s.x) && __builtin_isfinite(s.y) && __builtin_isfinite(s.z) &&
 			      __builtin_isfinite(s.w) && s.w >= 0.f))
@@ -1399,8 +1399,16 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 				mn[2] = fminf(mn[2], s.z - s.w); mx[2] = fmaxf(mx[2], s.z + s.w);
 			}
 		}
-		const bool useTileSphere = (P.flags & CADR_CULL_NO_TILE_SPHERES) == 0u;
-		if (useTileSphere) {
+		// a sphere around the wave's items: centre the middle of their bounding
+		// box, radius the largest |c_i - C| + r_i (a second reduction), which for
+		// scattered drawables is up to sqrt(3) times tighter than the box's half
+		// diagonal.  Each wave bounds its own items: it needs no block barrier,
+		// and its sphere is smaller than the tile's (2.5M drawables x 256 views,
+		// 256 x 8: 421 -> 413 us; 64 uneven scenes fused, 256 x 4: 866 -> 837).
+		bool usable = false;
+		float4 bound = make_float4(0.f, 0.f, 0.f, -1.f);
+		float maxCoord = 0.f;  // bound on |centre component|
+		if ((P.flags & CADR_CULL_NO_TILE_SPHERES) == 0u) {
 #pragma unroll
 			for (int off = 32; off >= 1; off >>= 1) {
 #pragma unroll
@@ -1409,55 +1417,26 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 					mx[a] = fmaxf(mx[a], __shfl_xor(mx[a], off));
 				}
 			}
-			const bool waveIrregular = __ballot(irregular) != 0ull;
-			if (lane == 0) {
-				sh.bad[wave] = waveIrregular ? 1u : 0u;
-				sh.red[wave][0] = mn[0]; sh.red[wave][1] = mn[1]; sh.red[wave][2] = mn[2];
-				sh.red[wave][3] = mx[0]; sh.red[wave][4] = mx[1]; sh.red[wave][5] = mx[2];
-			}
-		}
-		__syncthreads();
-		bool tileUsable = false;
-		float4 tileSphere = make_float4(0.f, 0.f, 0.f, -1.f);
-		float tileCoord = 0.f;  // bound on |centre component| over the tile
-		if (useTileSphere) {
-			uint32_t anyBad = 0;
-#pragma unroll
-			for (int q = 0; q < WAVES; q++) {
-				anyBad |= sh.bad[q];
-				for (int a = 0; a < 3; a++) {
-					mn[a] = fminf(mn[a], sh.red[q][a]);
-					mx[a] = fmaxf(mx[a], sh.red[q][3 + a]);
-				}
-			}
-			// centre: the middle of the tile's bounding box; radius: the largest
-			// |c_i - C| + r_i over the tile (a second reduction), which for
-			// scattered drawables is up to sqrt(3) times tighter than the box's
-			// half diagonal
+			const bool anyBad = __ballot(irregular) != 0ull;
 			const float cx = (mn[0] + mx[0]) * 0.5f, cy = (mn[1] + mx[1]) * 0.5f, cz = (mn[2] + mx[2]) * 0.5f;
-			float rad = 0.f;
+			float R = 0.f;
 #pragma unroll
 			for (int j = 0; j < ITEMS; j++) {
 				const float4 q = sp[j];
-				if (q.w >= 0.f) rad = fmaxf(rad, norm3(q.x - cx, q.y - cy, q.z - cz) + q.w);
+				if (q.w >= 0.f) R = fmaxf(R, norm3(q.x - cx, q.y - cy, q.z - cz) + q.w);
 			}
 #pragma unroll
-			for (int off = 32; off >= 1; off >>= 1) rad = fmaxf(rad, __shfl_xor(rad, off));
-			if (lane == 0) sh.red2[wave] = rad;
-			__syncthreads();
-			float R = 0.f;
-#pragma unroll
-			for (int q = 0; q < WAVES; q++) R = fmaxf(R, sh.red2[q]);
+			for (int off = 32; off >= 1; off >>= 1) R = fmaxf(R, __shfl_xor(R, off));
 			R *= 1.0f + 1.0f / 4096.0f;
-			tileUsable = anyBad == 0u && __builtin_isfinite(R) && __builtin_isfinite(cx) &&
-			             __builtin_isfinite(cy) && __builtin_isfinite(cz);
+			usable = !anyBad && __builtin_isfinite(R) && __builtin_isfinite(cx) && __builtin_isfinite(cy) &&
+			         __builtin_isfinite(cz);
 			// inflate against rounding of the centre and radius above
 			const float slack = (fabsf(cx) + fabsf(cy) + fabsf(cz) + R) * (1.0f / 65536.0f);
-			tileSphere = make_float4(cx, cy, cz, R + slack);
-			tileCoord = fmaxf(fmaxf(fmaxf(fabsf(mn[0]), fabsf(mx[0])), fmaxf(fabsf(mn[1]), fabsf(mx[1]))),
-			                  fmaxf(fabsf(mn[2]), fabsf(mx[2])));
+			bound = make_float4(cx, cy, cz, R + slack);
+			maxCoord = fmaxf(fmaxf(fmaxf(fabsf(mn[0]), fabsf(mx[0])), fmaxf(fabsf(mn[1]), fabsf(mx[1]))),
+			                 fmaxf(fabsf(mn[2]), fabsf(mx[2])));
 		}
-		const bool emptyTile = T.count == 0;
+		const bool emptyWave = wave * WAVE_ITEMS >= T.count;  // none of the wave's items lies in the tile
 
 		const uint64_t views = J.views;
 		uint64_t* chain0 = P.status + statusBaseOf(P, sh.offsets, job);
@@ -1465,21 +1444,21 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		for (uint32_t g0 = gBegin; g0 < gEnd; g0 += kViewGroup) {
 			const uint32_t vg = uniform(min(kViewGroup, gEnd - g0));
 
-			// tile classes of the group's views, lane v holding view g0+v, and
-			// the views that see part of the tile (every wave computes the same
-			// classes, so the mask is the same in every wave); the others
-			// contribute nothing and are skipped by all three phases
-			// (and the bound of the FMA estimate for the view; NaN: not used)
+			// classes of the wave's items in the group's views, lane v holding
+			// view g0+v, and the views that see some of them; the others
+			// contribute nothing and are skipped (and the bound of the FMA
+			// estimate for the view; NaN: not used)
 			uint32_t cls = 0;
 			float margin = __builtin_nanf("");
-			if (emptyTile) {
+			if (emptyWave) {
 				cls = 1;
-			} else if (tileUsable && lane < vg) {
+			} else if (usable && lane < vg) {
 				const ViewC Vl = loadView(views, g0 + lane);
-				cls = classifyTile(tileSphere, Vl);
-				margin = prefilterMargin(Vl, tileCoord, tileSphere.w);
+				cls = classifyItems(bound, Vl);
+				margin = prefilterMargin(Vl, maxCoord, bound.w);
 			}
 			const uint64_t active = __ballot(lane < vg && cls != 1u);
+			if (lane < vg) sh.cnt[lane][wave] = 0;
 
 			// 1. visibility bits and per-wave counts.  Lanes past the tile and
 			// invalid meshes hold the empty sphere, which no test passes.  Each
@@ -1529,12 +1508,9 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 
 			// 2. look-back, one view per lane of wave 0
 			if (wave == 0 && lane < vg) {
-				const bool act = (active >> lane) & 1ull;
 				uint32_t total = 0;
-				if (act) {
 #pragma unroll
-					for (int q = 0; q < WAVES; q++) total += sh.cnt[lane][q];
-				}
+				for (int q = 0; q < WAVES; q++) total += sh.cnt[lane][q];
 				uint64_t* chain = chain0 + uint64_t(g0 + lane) * J.numTiles;
 				uint32_t excl = 0;
 				if (T.first) {
@@ -1544,13 +1520,11 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 					excl = lookBackSerial(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch});
 					publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
 				}
-				if (act) {
-					uint32_t b = T.segBase + excl;
+				uint32_t b = T.segBase + excl;
 #pragma unroll
-					for (int q = 0; q < WAVES; q++) {
-						sh.base[lane][q] = b;
-						b += sh.cnt[lane][q];
-					}
+				for (int q = 0; q < WAVES; q++) {
+					sh.base[lane][q] = b;
+					b += sh.cnt[lane][q];
 				}
 				if (T.last && T.k < J.numStateSets)
 					globalMut<uint32_t>(J.counts)[uint64_t(g0 + lane) * J.numStateSets + T.k] = excl + total;
