@@ -449,9 +449,15 @@ __device__ __forceinline__ uint32_t itemOfTicket(Shard s, uint32_t r)
 	return ((((r >> 3) << s.shift) + s.g) << 3) + (r & 7u);
 }
 
-__device__ __forceinline__ uint32_t takeTicket(const CullParams& P, Shard s)
+// The add's result is not waited for here (the address is kept from being
+// known uniform, or the compiler turns the add into a wave reduction that
+// waits for it), so other loads can be in flight beside it; itemOfTicket of
+// the result is.
+__device__ __forceinline__ uint32_t askTicket(const CullParams& P, Shard s)
 {
-	return itemOfTicket(s, atomicAdd(&P.ctl[kCtlShard + 64u * s.g], 1u));
+	uint64_t a = addr(P.ctl + kCtlShard + 64u * s.g);
+	asm volatile("" : "+v"(a));
+	return __hip_atomic_fetch_add(globalMut<uint32_t>(a), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Called by one thread of each workgroup when it leaves: the last one of the
@@ -631,18 +637,32 @@ __device__ __forceinline__ float4 meshSphere(const MeshTable& M, uint32_t m)
 }
 
 // Mesh table of a job staged in LDS, field-major (see MeshTable), when it is
-// small; returns whether the LDS copy is in use.
+// small: loads first, LDS stores when the caller has nothing else to start.
 template <int BLOCK>
-__device__ __forceinline__ bool stageMeshes(uint32_t* sMeshes, const cadrCullJob& J, uint32_t tid)
-{
-	if (J.numMeshes > kLdsMeshes) return false;
-	const gptr<uint32_t> src = globalPtr<uint32_t>(J.meshes);
-	for (uint32_t i = tid; i < J.numMeshes * 16u; i += BLOCK) {
-		const uint32_t x = src[i];
-		sMeshes[(i % 16u) * kLdsMeshes + i / 16u] = i % 16u == 4u ? maxLodOf(x) : x;
+struct MeshStaging {
+	static constexpr int N = (16 * kLdsMeshes + BLOCK - 1) / BLOCK;
+	uint32_t x[N];
+	uint32_t words;  // 0: not staged
+
+	__device__ __forceinline__ bool load(const cadrCullJob& J, uint32_t tid)
+	{
+		words = J.numMeshes <= kLdsMeshes ? J.numMeshes * 16u : 0u;
+		if (words != 0u) {
+			const gptr<uint32_t> src = globalPtr<uint32_t>(J.meshes);
+#pragma unroll
+			for (int k = 0; k < N; k++) x[k] = src[min(tid + uint32_t(k) * BLOCK, words - 1u)];
+		}
+		return J.numMeshes <= kLdsMeshes;
 	}
-	return true;
-}
+	__device__ __forceinline__ void store(uint32_t* sMeshes, uint32_t tid) const
+	{
+#pragma unroll
+		for (int k = 0; k < N; k++) {
+			const uint32_t i = tid + uint32_t(k) * BLOCK;
+			if (i < words) sMeshes[(i % 16u) * kLdsMeshes + i / 16u] = i % 16u == 4u ? maxLodOf(x[k]) : x[k];
+		}
+	}
+};
 
 // The fused form of loadTileItems: the wave's items are computed from the
 // leaf level instead of read, exactly as cadrPropagateTransforms computes
@@ -937,10 +957,15 @@ __device__ __forceinline__ void cullViewBody(const CullParams& P)
 
 	const uint32_t tid = threadIdx.x, lane = laneId(), wave = tid / 64;
 	const Shard shard = homeShard<BLOCK * ITEMS>(P);
-	if (tid == 0) sTicket = takeTicket(P, shard);
+	// ticket, epoch and mesh table in flight together
+	uint32_t ticket = 0;
+	if (tid == 0) ticket = askTicket(P, shard);
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	const cadrCullJob J = loadJob(P.jobs, 0);
-	const bool ldsMeshes = stageMeshes<BLOCK>(sMeshes, J, tid);
+	MeshStaging<BLOCK> staging;
+	const bool ldsMeshes = staging.load(J, tid);
+	if (tid == 0) sTicket = itemOfTicket(shard, ticket);
+	staging.store(sMeshes, tid);
 	__syncthreads();
 	const uint32_t t = uniform(sTicket);
 	const MeshTable meshes{sMeshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
@@ -990,7 +1015,7 @@ __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCul
 	for (uint32_t b = 0;; b ^= 1u) {
 		const uint32_t n = listVisible<ITEMS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
 		if (lane == 0) sCnt[b][wave] = n;
-		if (tid == 0) *sTicket = takeTicket(P, shard);
+		if (tid == 0) *sTicket = itemOfTicket(shard, askTicket(P, shard));
 		__syncthreads();
 
 		// the next tile's loads, in flight through this tile's look-back and stores
@@ -1026,10 +1051,15 @@ __global__ __launch_bounds__(BLOCK) void cullViewLoopKernel(CullParams P)
 
 	const uint32_t tid = threadIdx.x, lane = laneId(), wave = tid / 64;
 	const Shard shard = homeShard<BLOCK * ITEMS>(P);
-	if (tid == 0) sTicket = takeTicket(P, shard);
+	// ticket, epoch and mesh table in flight together
+	uint32_t ticket = 0;
+	if (tid == 0) ticket = askTicket(P, shard);
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	const cadrCullJob J = loadJob(P.jobs, 0);
-	const bool ldsMeshes = stageMeshes<BLOCK>(sMeshes, J, tid);
+	MeshStaging<BLOCK> staging;
+	const bool ldsMeshes = staging.load(J, tid);
+	if (tid == 0) sTicket = itemOfTicket(shard, ticket);
+	staging.store(sMeshes, tid);
 	__syncthreads();
 	const uint32_t t = uniform(sTicket);
 	__syncthreads();  // every wave has read the first ticket before the loop rewrites it
@@ -1202,8 +1232,9 @@ struct FewShared {
 
 template <int BLOCK, int ITEMS, int CH, bool LDS>
 __device__ __forceinline__ void cullFewTile(const CullParams& P, const cadrCullJob& J, const TileDesc& T,
-                                            uint32_t viewBegin, uint32_t viewEnd, uint64_t* chain0, uint32_t epoch, const MeshTable& meshes, FewShared<BLOCK, ITEMS, CH>& sh,
-                                            uint32_t& b, uint32_t lane, uint32_t wave)
+                                            uint32_t viewBegin, uint32_t viewEnd, uint64_t* chain0, uint32_t epoch,
+                                            const MeshTable& meshes, FewShared<BLOCK, ITEMS, CH>& sh, uint32_t& b,
+                                            uint32_t lane, uint32_t wave)
 {
 	constexpr int WAVES = BLOCK / 64, WAVE_ITEMS = 64 * ITEMS;
 	constexpr uint32_t W = 64 / CH;  // lanes of a view in the look-back
@@ -1268,11 +1299,17 @@ __global__ __launch_bounds__(BLOCK) void cullFewKernel(CullParams P)
 	const uint32_t tid = threadIdx.x, lane = laneId(), wave = uniform(tid / 64);
 	const Shard shard = homeShard<BLOCK * ITEMS>(P);
 	uint32_t job = 0, b = 0;
-	if (tid == 0) sh.ticket[0] = takeTicket(P, shard);
+	uint32_t ticket = 0;
+	if (tid == 0) ticket = askTicket(P, shard);
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	if (wave == 0 && P.numJobs > 1 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
 	bool ldsMeshes = false;
-	if (P.numJobs == 1) ldsMeshes = stageMeshes<BLOCK>(sh.meshes, loadJob(P.jobs, 0), tid);
+	if (P.numJobs == 1) {
+		MeshStaging<BLOCK> staging;
+		ldsMeshes = staging.load(loadJob(P.jobs, 0), tid);
+		staging.store(sh.meshes, tid);
+	}
+	if (tid == 0) sh.ticket[0] = itemOfTicket(shard, ticket);
 	for (uint32_t k = 0;; k ^= 1u) {
 		__syncthreads();
 		const uint32_t t = uniform(sh.ticket[k]);
@@ -1284,10 +1321,14 @@ __global__ __launch_bounds__(BLOCK) void cullFewKernel(CullParams P)
 		uint64_t* chain0 = P.status + statusBaseOf(P, sh.offsets, job);
 		const MeshTable meshes{sh.meshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
 		if (ldsMeshes)
-			cullFewTile<BLOCK, ITEMS, CH, true>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane, wave);
+			cullFewTile<BLOCK, ITEMS, CH, true>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane,
+			                                    wave);
 		else
-			cullFewTile<BLOCK, ITEMS, CH, false>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane, wave);
-		if (tid == 0) sh.ticket[k ^ 1u] = takeTicket(P, shard);
+			cullFewTile<BLOCK, ITEMS, CH, false>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane,
+			                                     wave);
+		// not earlier: a ticket held during the stores keeps its tile's followers
+		// waiting in their look-backs (24 served scenes: 98 -> 103 us)
+		if (tid == 0) sh.ticket[k ^ 1u] = itemOfTicket(shard, askTicket(P, shard));
 	}
 	if (tid == 0) leaveLaunch(P, shard, epoch);
 }
@@ -1327,7 +1368,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 	if (wave == 0 && P.numJobs > 1 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
 
 	for (;;) {
-		if (tid == 0) sh.ticket = takeTicket(P, shard);
+		if (tid == 0) sh.ticket = itemOfTicket(shard, askTicket(P, shard));
 		__syncthreads();
 		const uint32_t w = uniform(sh.ticket);
 		if (w >= P.totalWork) break;
@@ -1343,7 +1384,9 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		// reads the old table)
 		bool ldsMeshes = J.numMeshes <= kLdsMeshes;
 		if (job != stagedJob) {
-			ldsMeshes = stageMeshes<BLOCK>(sh.meshes, J, tid);
+			MeshStaging<BLOCK> staging;
+			ldsMeshes = staging.load(J, tid);
+			staging.store(sh.meshes, tid);
 			stagedJob = job;
 		}
 
@@ -1747,6 +1790,22 @@ const KernelEntry* findKernel(const cadrCullConfig* c)
 	return nullptr;
 }
 
+// The shape that runs a one-view launch of numTiles tiles given in shape ke:
+// where the tiles do not fill the compute units once, the one of the same
+// tile size with the most threads, so that each wave's chain of round trips is
+// shorter (100k drawables, 256 x 4 against 1024 x 1: 7.4 / 6.8 us; a tree frame
+// of 41k leaves 19.0 / 17.7 us, of 400k leaves, 391 tiles, 29.6 / 31.0 us).
+// The fused kernel is kept at 512 threads: 41k leaves 20.4 / 20.6 us.
+const KernelEntry* shapeFor(const KernelEntry* ke, uint32_t numTiles, KernelFn KernelEntry::*path)
+{
+	const int cu = computeUnitCount();
+	if (numTiles > uint32_t(cu > 0 ? cu : 256)) return ke;
+	const KernelEntry* best = ke;
+	for (const KernelEntry& k : kKernels)
+		if (k.block * k.items == ke->block * ke->items && k.block > best->block && k.*path) best = &k;
+	return best;
+}
+
 }  // namespace
 
 bool cadr::cullHasKernel(const cadrCullConfig* c, CullPath path)
@@ -2080,6 +2139,7 @@ CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, cons
 	const bool loop = resident > 0 && hostJob->numTiles > uint32_t(resident);
 	const uint32_t grid = loop ? uint32_t(resident) : hostJob->numTiles;
 	p.shardShift = shardShiftFor(ke->block * ke->items, grid, hostJob->numTiles, jobBytes(*hostJob, false));
+	if (!loop) ke = shapeFor(ke, hostJob->numTiles, &KernelEntry::view);
 	launchKernel(loop ? ke->viewLoop : ke->view, dim3(grid), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "cullViewKernel launch");
 	return ok();
@@ -2116,6 +2176,7 @@ CADR_API int cadrPropagateCullView(const cadrTransformLevel* leaf, const cadrCul
 	                    leaf->parentWorld ? leaf->parentCount : 0u};
 	p.shardShift = shardShiftFor(ke->block * ke->items, hostJob->numTiles, hostJob->numTiles,
 	                             jobBytes(*hostJob, true));
+	if (ke->block < 512) ke = shapeFor(ke, hostJob->numTiles, &KernelEntry::fused);
 	launchKernel(ke->fused, dim3(hostJob->numTiles), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "fused cullViewKernel launch");
 	return ok();

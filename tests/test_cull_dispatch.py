@@ -125,3 +125,28 @@ def test_many_views_boundary_spheres(gpu):
     batch.close()
     out.close()
     ds.close()
+
+
+# one-view launches of at most one tile a compute unit run the widest shape of their tile size
+@pytest.mark.parametrize("block,items,fanouts", [(256, 4, (4, 256, 256)), (256, 4, (4, 256, 257)),
+                                                 (256, 8, (8, 256, 256)), (256, 8, (8, 256, 257)), (512, 2, (3, 7, 11))])
+def test_fused_shape_by_tiles(gpu, block, items, fanouts):
+    print(f"{fanouts} {block}x{items}", flush=True)
+    scene = scenes.tree_scene(fanouts, seed=scenes.SEED_BASE + 950, num_statesets=1, lod_count=3)
+    worlds, spheres = oracle.propagate_scene(scene)
+    ds = cull.DeviceScene(scene)
+    descs = ds.level_descs(spheres=False)
+    views = cull.make_views(scenes.random_cameras(9, 20, 0, 1, 100.0))
+    out = cull.CullOutputs(1, ds.n, ds.K)
+    batch = cull.CullBatch(cull.make_config(block, items), [(ds, views, out)])
+    for lv in descs[:-1]:
+        N.check(N.load().cadrPropagateTransforms(N.ptr(lv), None))
+    for k in range(2):
+        batch.run_fused(descs[-1])
+        synchronize()
+        batch.workspace.check()
+        _check([(ds, views, out, spheres, scene)], f"fused {block}x{items} launch {k}")
+    assert ds.world_matrices(-1).tobytes() == worlds[-1].tobytes()
+    batch.close()
+    out.close()
+    ds.close()
