@@ -713,17 +713,18 @@ __device__ __forceinline__ void issueItemLoads(const LeafParams& Lf, uint64_t fi
 
 // store: write the world matrices (and spheres); a tile that several work
 // items of one launch share is written by one of them.
-template <int ITEMS, bool LDS, bool PREFETCH = true, bool COOP = false>
+// sphere(j, s) receives the lane's world sphere of item j, in order of j.
+template <int ITEMS, bool LDS, bool PREFETCH = true, bool COOP = false, class Sink>
 __device__ __forceinline__ void propagateTileItems(const LeafParams& Lf, const cadrCullJob& J, const TileDesc& T,
                                                    uint32_t base, uint32_t lane, float4* stage,
-                                                   const MeshTable& meshes, float4 (&sp)[ITEMS],
-                                                   uint32_t (&mi)[ITEMS], bool store = true)
+                                                   const MeshTable& meshes, Sink sphere, uint32_t (&mi)[ITEMS],
+                                                   bool store = true)
 {
 	const float4 empty = make_float4(0.f, 0.f, 0.f, -__builtin_inff());
 	if (T.count == 0) {
 #pragma unroll
 		for (int j = 0; j < ITEMS; j++) {
-			sp[j] = empty;
+			sphere(j, empty);
 			mi[j] = 0;
 		}
 		return;
@@ -748,7 +749,7 @@ __device__ __forceinline__ void propagateTileItems(const LeafParams& Lf, const c
 #pragma unroll
 	for (int j = 0; j < ITEMS; j++) {
 		if (uint32_t(j) >= items) {
-			sp[j] = empty;
+			sphere(j, empty);
 			continue;
 		}
 		const uint64_t first = uint64_t(T.start) + base + uint32_t(j) * 64u;
@@ -791,7 +792,7 @@ __device__ __forceinline__ void propagateTileItems(const LeafParams& Lf, const c
 		float4 s = empty;
 		if (live && mi[j] < J.numMeshes) s = sphereTransform(W, meshSphere<LDS>(meshes, mi[j]));
 		if (store && Lf.spheres && live) storeF4(globalMut<float4>(Lf.spheres) + i, s);
-		sp[j] = s;
+		sphere(j, s);
 		// without the prefetch, keep the scheduler from hoisting later items'
 		// loads above this one (every item's 32 registers of loads at once)
 		if constexpr (!PREFETCH) __builtin_amdgcn_sched_barrier(0);
@@ -925,7 +926,8 @@ __device__ __forceinline__ void cullViewTile(const CullParams& P, const cadrCull
 	float4 sp[ITEMS];
 	uint32_t mi[ITEMS];
 	if constexpr (FUSED)
-		propagateTileItems<ITEMS, LDS>(P.leaf, J, T, wave * WAVE_ITEMS, lane, sMat, meshes, sp, mi);
+		propagateTileItems<ITEMS, LDS>(P.leaf, J, T, wave * WAVE_ITEMS, lane, sMat, meshes,
+		                               [&](int j, float4 q) __attribute__((always_inline)) { sp[j] = q; }, mi);
 	else
 		loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
 	const uint32_t n = listVisible<ITEMS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
@@ -1348,19 +1350,24 @@ struct CullShared {
 
 // COOP (fused form only): parent matrices read whole, 16 per instruction
 // (issueParentLoads), for leaves whose parents are scattered; it holds more
-// registers, so it is chosen per shape (see the kernel table).
-template <int BLOCK, int ITEMS, bool FUSED, bool COOP = false>
-__global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
+// registers, so it is chosen per shape, like WPE, the waves per SIMD asked of
+// the register allocator (see the kernel table).
+template <int BLOCK, int ITEMS, bool FUSED, bool COOP = false, int WPE = 1>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void cullKernel(CullParams P)
 {
 	using S = CullShared<BLOCK, ITEMS>;
 	constexpr int WAVES = S::WAVES;
 	constexpr int WAVE_ITEMS = 64 * ITEMS;
 	__shared__ S sh;
-	__shared__ float4 sMat[FUSED ? WAVES : 1][FUSED ? 256 : 1];  // local-matrix staging of the fused form
+	// the fused form keeps its spheres here instead of in registers, which
+	// computing them needs: with the spheres in registers it held 237 (256 x 8)
+	// and ran 2 waves per SIMD, its view loop at half the VALU's rate (64 uneven
+	// scenes 977 us, now 867 with 3 waves; 512 x 4 1238 and 881 with 4)
+	__shared__ float4 sSpheres[FUSED ? WAVES : 1][FUSED ? WAVE_ITEMS : 1];
 
 	const uint32_t tid = threadIdx.x;
-	const uint32_t lane = laneId();
-	const uint32_t wave = tid / 64;
+	uint32_t lane = laneId();
+	const uint32_t wave = uniform(tid / 64);
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	const Shard shard = homeShard<S::TILE>(P);
 	uint32_t job = 0, stagedJob = ~0u;
@@ -1372,6 +1379,9 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		__syncthreads();
 		const uint32_t w = uniform(sh.ticket);
 		if (w >= P.totalWork) break;
+		// a lane index of its own for each tile: the compiler otherwise keeps
+		// dozens of addresses derived from it in registers across tiles
+		if constexpr (FUSED) asm volatile("" : "+v"(lane));
 
 		job = jobOfWork(P, sh.offsets, w, job, lane);
 		const cadrCullJob J = loadJob(P.jobs, job);
@@ -1395,30 +1405,50 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 		// load the tile into registers (wave-contiguous runs) and bound it for
 		// the tile sphere; the fused form computes the spheres from the job's
 		// leaf level instead, writing its world matrices on the way
-		float4 sp[ITEMS];
+		float4 sp[FUSED ? 1 : ITEMS];
 		uint32_t mi[ITEMS];
+		float4* own = sSpheres[FUSED ? wave : 0];
 		if constexpr (FUSED) {
 			__syncthreads();  // the sphere transforms read the LDS mesh table
 			const LeafParams Lf = loadLeaf(P.leaves, job);
 			constexpr bool PREFETCH = ITEMS >= 8;
-			float4* stage = &sMat[wave][0];
+			// the matrices are staged in the last 4 KiB of the wave's spheres;
+			// spheres that belong there wait in registers until the last item
+			static_assert(ITEMS >= 4, "4 KiB of spheres a wave");
+			constexpr int EARLY = ITEMS - 4;
+			float4* stage = own + 64 * EARLY;
+			float4 late[4];
+			auto sink = [&](int j, float4 q) __attribute__((always_inline)) {
+				if (j < EARLY)
+					own[j * 64 + lane] = q;
+				else
+					late[j - EARLY] = q;
+			};
 			if (ldsMeshes)
-				propagateTileItems<ITEMS, true, PREFETCH, COOP>(Lf, J, T, wave * WAVE_ITEMS, lane, stage, meshes, sp,
+				propagateTileItems<ITEMS, true, PREFETCH, COOP>(Lf, J, T, wave * WAVE_ITEMS, lane, stage, meshes, sink,
 				                                                mi, storeLeaf);
 			else
-				propagateTileItems<ITEMS, false, PREFETCH, COOP>(Lf, J, T, wave * WAVE_ITEMS, lane, stage, meshes, sp,
+				propagateTileItems<ITEMS, false, PREFETCH, COOP>(Lf, J, T, wave * WAVE_ITEMS, lane, stage, meshes, sink,
 				                                                 mi, storeLeaf);
+			waveSync();  // the staging is read before its place is taken
+#pragma unroll
+			for (int k = 0; k < 4; k++) stage[k * 64 + lane] = late[k];
+			waveSync();
+			asm volatile("" : "+v"(lane));
 		} else {
 			loadTileItems<ITEMS>(globalPtr<float4>(J.spheres), globalPtr<uint32_t>(J.meshIndex), T,
 			                     wave * WAVE_ITEMS + lane, sp, mi);
 		}
+		auto sphereAt = [&](int j) __attribute__((always_inline)) {
+			if constexpr (FUSED) return own[j * 64 + lane]; else return sp[j];
+		};
 		bool irregular = false;
 		float mn[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
 		float mx[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
 #pragma unroll
 		for (int j = 0; j < ITEMS; j++) {
 			const uint32_t e = wave * WAVE_ITEMS + j * 64 + lane;
-			float4 s = sp[j];
+			float4 s = sphereAt(j);
 			uint32_t m = mi[j];
 			if (e >= T.count) {
 				s = make_float4(0.f, 0.f, 0.f, -__builtin_inff());
@@ -1427,7 +1457,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 				s = make_float4(0.f, 0.f, 0.f, -__builtin_inff());  // invalid mesh: never visible
 				m = 0;
 			}
-			sp[j] = s;
+			if constexpr (FUSED) own[j * 64 + lane] = s; else sp[j] = s;
 			mi[j] = m;
 
 			// a sphere other than a finite one with r >= 0 or the empty sphere
@@ -1465,7 +1495,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 			float R = 0.f;
 #pragma unroll
 			for (int j = 0; j < ITEMS; j++) {
-				const float4 q = sp[j];
+				const float4 q = sphereAt(j);
 				if (q.w >= 0.f) R = fmaxf(R, norm3(q.x - cx, q.y - cy, q.z - cz) + q.w);
 			}
 #pragma unroll
@@ -1512,27 +1542,29 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 			for (int j = 0; j < ITEMS; j++) vlo[j] = vhi[j] = 0u;
 			for (uint64_t am = active; am != 0ull; am &= am - 1ull) {
 				const uint32_t v = uint32_t(__builtin_ctzll(am));
+				if constexpr (FUSED) asm volatile("" ::: "memory");  // the spheres are read again for each view
 				const uint32_t c = uniform(__builtin_amdgcn_readlane(cls, v));
 				const float mg = __uint_as_float(uniform(__builtin_amdgcn_readlane(__float_as_uint(margin), v)));
 				const ViewC V = loadView(views, g0 + v);
 				bool vis[ITEMS];
 				if (c == 2u) {
 #pragma unroll
-					for (int j = 0; j < ITEMS; j++) vis[j] = sp[j].w >= 0.f;
+					for (int j = 0; j < ITEMS; j++) vis[j] = sphereAt(j).w >= 0.f;
 				} else if (mg <= 0x1p100f) {
 					// the translation column in vector registers once per view
 					float w0 = V.r0.w, w1 = V.r1.w, w2 = V.r2.w;
 					asm volatile("" : "+v"(w0), "+v"(w1), "+v"(w2));
 #pragma unroll
 					for (int j = 0; j < ITEMS; j++) {
-						const float p = planeMin(sp[j], V, w0, w1, w2);
+						const float4 q = sphereAt(j);
+						const float p = planeMin(q, V, w0, w1, w2);
 						vis[j] = p > 0.f;
 						const bool unsure = !(fabsf(p) > mg);
-						if (__ballot(unsure) != 0ull) vis[j] = unsure ? sphereVisible(sp[j], V) : vis[j];
+						if (__ballot(unsure) != 0ull) vis[j] = unsure ? sphereVisible(q, V) : vis[j];
 					}
 				} else {
 #pragma unroll
-					for (int j = 0; j < ITEMS; j++) vis[j] = sphereVisible(sp[j], V);
+					for (int j = 0; j < ITEMS; j++) vis[j] = sphereVisible(sphereAt(j), V);
 				}
 				uint32_t n = 0;
 				const uint32_t bit = 1u << (v & 31u);
@@ -1584,6 +1616,7 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 			                     const uint32_t (&bits)[ITEMS]) __attribute__((always_inline)) {
 				for (; am != 0ull; am &= am - 1ull) {
 					const uint32_t v = v0 + uint32_t(__builtin_ctzll(am));
+					if constexpr (FUSED) asm volatile("" ::: "memory");
 					const uint32_t run = uniform(sh.cnt[v][wave]);
 					if (run == 0) continue;
 					const ViewC V = loadView(views, g0 + v);
@@ -1599,9 +1632,10 @@ __global__ __launch_bounds__(BLOCK) void cullKernel(CullParams P)
 							const uint32_t n = uint32_t(__builtin_popcountll(m));
 							if (n == 0) continue;
 							if (vis) {
+								const float4 q = sphereAt(j);
 								uint32_t count, first, vofs;
-								meshCommand<decltype(lds)::value>(meshes, mi[j], sp[j].w, viewCoord(V.r2, sp[j]), V,
-								                                  count, first, vofs);
+								meshCommand<decltype(lds)::value>(meshes, mi[j], q.w, viewCoord(V.r2, q), V, count,
+								                                  first, vofs);
 								const uint32_t r = maskRank(m);
 								if (!decltype(checked)::value || pos + r < J.commandStride) {
 									const gmut<uint32_t> o = out + uint64_t(pos) * 5ull + uint64_t(r * 5u);
@@ -1739,16 +1773,18 @@ struct KernelEntry {
 // / 58.8 against 94.6 / 67.0 / 59.6 us; not at 256 x 4 / 8 / 16 (67.5 / 65.0 /
 // 63.3 against 63.9 / 61.5 / 63.0) nor 512 x 4 (61.7 against 62.0, no more than
 // runs differ), where several workgroups of a CU overlap each other's phases.
-// fusedBatch reads parents whole (COOP) at 256 x 8 and 512 x 4, where it
-// measured faster on uneven64 (2.39 -> 2.32 and 2.93 -> 2.84 ms); at 256 x 4
-// its registers cost a wave per SIMD (2.38 -> 2.60 ms)
+// fusedBatch: parents read whole (COOP) and the items prefetched at 256 x 8,
+// held to 3 waves per SIMD (4 registers spilled); neither at 256 x 4 and 512 x
+// 4, held to 4.  64 uneven scenes, 1-32 views: 256 x 8 867 us (no prefetch 881,
+// neither 879, registers unbounded 1002), 256 x 4 855 (COOP 923, 3 waves 910),
+// 512 x 4 881 (3 waves with COOP 1255).
 const KernelEntry kKernels[] = {
     {256, 2, cullKernel<256, 2, false>, cullViewKernel<256, 2>, cullFusedKernel<256, 2, 4>, nullptr, nullptr, {cullFewKernel<256, 2, 1>, cullFewKernel<256, 2, 2>, cullFewKernel<256, 2, 4>}},
-    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true>, nullptr, {cullFewKernel<256, 4, 1>, cullFewKernel<256, 4, 2>, cullFewKernel<256, 4, 4>}},
-    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true>, nullptr, {cullFewKernel<256, 8, 1>, cullFewKernel<256, 8, 2>, cullFewKernel<256, 8, 4>}},
+    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true, false, 4>, nullptr, {cullFewKernel<256, 4, 1>, cullFewKernel<256, 4, 2>, cullFewKernel<256, 4, 4>}},
+    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true, 3>, nullptr, {cullFewKernel<256, 8, 1>, cullFewKernel<256, 8, 2>, cullFewKernel<256, 8, 4>}},
     {256, 16, cullKernel<256, 16, false>, cullViewKernel<256, 16>, cullFusedKernel<256, 16, 1>, nullptr, nullptr},
     {512, 2, cullKernel<512, 2, false>, cullViewKernel<512, 2>, cullFusedKernel<512, 2, 1>, nullptr, nullptr},
-    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, true>, nullptr, {cullFewKernel<512, 4, 1>, cullFewKernel<512, 4, 2>, cullFewKernel<512, 4, 4>}},
+    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, false, 4>, nullptr, {cullFewKernel<512, 4, 1>, cullFewKernel<512, 4, 2>, cullFewKernel<512, 4, 4>}},
     {512, 8, nullptr, cullViewKernel<512, 8>, nullptr, nullptr, nullptr},
     {512, 16, nullptr, cullViewKernel<512, 16>, nullptr, nullptr, nullptr},
     {1024, 1, nullptr, cullViewKernel<1024, 1>, cullFusedKernel<1024, 1, 1>, nullptr, cullViewLoopKernel<1024, 1>},
