@@ -1215,16 +1215,26 @@ __device__ __forceinline__ uint64_t statusBaseOf(const CullParams& P, const JobO
 }
 
 // Jobs of few views: the batched kernel without what only many views pay
-// for.  No tile sphere, no visibility bits kept per view: the workgroup lists
-// its visible items for CH views at a time, wave 0 looks all CH chains back
-// at once, and the commands are stored from the lists.  It holds half the
-// batched kernel's registers, so twice its workgroups are resident to overlap
-// their chains of round trips.  Persistent, like the batched kernel; a mesh
-// table is staged only where the launch has one job.
-template <int BLOCK, int ITEMS, int CH>
+// for.  No bounding sphere, no visibility bits kept per view: the workgroup
+// lists the visible items of a work item's views (up to CH), wave 0 looks
+// their chains back at once, and the commands are stored from the lists.  It
+// holds less than half the batched kernel's registers, so more workgroups are
+// resident to overlap their chains of round trips.  Persistent, like the
+// batched kernel; the mesh table is staged where the launch has one job.
+//
+// With DEFER (one or two views) the look-back runs one item behind: a
+// workgroup publishes an item's totals as soon as they are known, starts the
+// next item's loads and only then looks back and stores the item before.  No
+// published total ever waits for a look-back, so look-backs find their
+// predecessors published and the loads are in flight all the time; without
+// it, a next ticket held that early keeps its followers waiting (24 served
+// scenes, 256 x 4: 118 us against 96.6, and 99.4 with the ticket taken last;
+// 256 x 2: 179 / 121 / 139).  Four views take the ticket last: two lists of
+// four views would halve the workgroups a CU holds.
+template <int BLOCK, int ITEMS, int CH, bool DEFER>
 struct FewShared {
 	static constexpr int WAVES = BLOCK / 64;
-	uint32_t run[WAVES][CH][64 * ITEMS];
+	uint32_t run[DEFER ? 2 : 1][WAVES][CH][64 * ITEMS];
 	uint32_t meshes[16 * kLdsMeshes];
 	JobOffsets offsets;
 	uint32_t cnt[2][CH][WAVES];
@@ -1232,107 +1242,216 @@ struct FewShared {
 	uint32_t ticket[2];
 };
 
-template <int BLOCK, int ITEMS, int CH, bool LDS>
-__device__ __forceinline__ void cullFewTile(const CullParams& P, const cadrCullJob& J, const TileDesc& T,
-                                            uint32_t viewBegin, uint32_t viewEnd, uint64_t* chain0, uint32_t epoch,
-                                            const MeshTable& meshes, FewShared<BLOCK, ITEMS, CH>& sh, uint32_t& b,
-                                            uint32_t lane, uint32_t wave)
+// A work item as its workgroup holds it: the job, the tile, the views and
+// where their chains begin.
+struct FewItem {
+	cadrCullJob J;
+	TileDesc T;
+	uint32_t viewBegin, viewEnd;
+	uint64_t* chain0;
+};
+
+template <bool JOBS>
+__device__ __forceinline__ FewItem fewItem(const CullParams& P, const JobOffsets& offsets, const cadrCullJob& only,
+                                           uint32_t t, uint32_t tile, uint32_t& job, uint32_t lane)
 {
-	constexpr int WAVES = BLOCK / 64, WAVE_ITEMS = 64 * ITEMS;
-	constexpr uint32_t W = 64 / CH;  // lanes of a view in the look-back
-	const gptr<uint32_t> meshIndex = globalPtr<uint32_t>(J.meshIndex);
-	float4 sp[ITEMS];
-	uint32_t mi[ITEMS];
-	loadTileItems<ITEMS>(globalPtr<float4>(J.spheres), meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
-	for (uint32_t v0 = viewBegin; v0 < viewEnd; v0 += CH, b ^= 1u) {
-		uint32_t n[CH];
-#pragma unroll
-		for (int c = 0; c < CH; c++) {
-			n[c] = 0;
-			if (v0 + c < viewEnd) {
-				n[c] = listVisible<ITEMS>(sp, mi, T, J.numMeshes, loadView(J.views, v0 + c), wave * WAVE_ITEMS, lane,
-				                          sh.run[wave][c]);
-				if (lane == 0) sh.cnt[b][c][wave] = n[c];
-			}
-		}
-		__syncthreads();
-		if (wave == 0) {
-			const uint32_t c = lane / W, view = v0 + c;  // the lane's view
-			const bool on = view < viewEnd, lead = on && lane % W == 0u;
-			uint32_t total = 0;
-			if (on)
-				for (int q = 0; q < WAVES; q++) total += sh.cnt[b][c][q];
-			uint64_t* chain = chain0 + uint64_t(on ? view : v0) * J.numTiles;
-			uint32_t excl = 0;
-			if (T.first) {
-				if (lead) publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
-			} else {
-				if (lead) publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
-				const WaitBound B{P.ctl, P.waitLimit, epoch};
-				if constexpr (CH == 1)
-					excl = lookBackWave(chain, T.chain, B, lane);
-				else
-					excl = lookBackGroups<W>(chain, on ? T.chain : 0u, B, lane);
-				if (lead) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
-			}
-			if (lead) {
-				sh.excl[b][c] = excl;
-				if (T.last && T.k < J.numStateSets)
-					globalMut<uint32_t>(J.counts)[uint64_t(view) * J.numStateSets + T.k] = excl + total;
-			}
-		}
-		__syncthreads();
-#pragma unroll
-		for (int c = 0; c < CH; c++) {
-			if (n[c] == 0) continue;
-			uint32_t pos = T.segBase + sh.excl[b][c];
-			for (uint32_t q = 0; q < wave; q++) pos += sh.cnt[b][c][q];
-			storeListed<LDS>(sh.run[wave][c], n[c], uniform(pos), T.start + wave * WAVE_ITEMS, meshes, J.numMeshes,
-			                 meshIndex, globalMut<uint32_t>(J.commands) + uint64_t(v0 + c) * J.commandStride * 5ull,
-			                 J.commandStride, lane);
-		}
+	FewItem f;
+	if constexpr (JOBS) {
+		job = jobOfWork(P, offsets, t, job, lane);
+		f.J = loadJob(P.jobs, job);
+		t -= firstWorkOf(P, offsets, job);
+		f.chain0 = P.status + statusBaseOf(P, offsets, job);
+	} else {
+		f.J = only;
+		f.chain0 = P.status;
+	}
+	const WorkItem item = workItem(P, f.J, t);
+	f.T = loadTile(f.J, item.tile, tile);
+	f.viewBegin = item.viewBegin;
+	f.viewEnd = item.viewEnd;
+	return f;
+}
+
+// The lane's view of an item in wave 0's look-back: 64 / CH lanes a view.
+template <int CH>
+struct FewChain {
+	uint64_t* chain;
+	uint32_t view;
+	bool on, lead;
+	__device__ __forceinline__ FewChain(const FewItem& f, uint32_t lane)
+	{
+		constexpr uint32_t W = 64 / CH;
+		view = f.viewBegin + lane / W;
+		on = view < f.viewEnd;
+		lead = on && lane % W == 0u;
+		chain = f.chain0 + uint64_t(on ? view : f.viewBegin) * f.J.numTiles + f.T.chain;
+	}
+};
+
+// Wave 0: publishes an item's totals (per lane: its view's).
+template <int CH>
+__device__ __forceinline__ void fewPublish(const FewItem& f, uint32_t total, uint32_t epoch, uint32_t lane)
+{
+	const FewChain<CH> c(f, lane);
+	if (c.lead) publish(c.chain, packStatus(epoch, f.T.first ? kStatePrefix : kStateAggregate, total));
+}
+
+// Wave 0: an item's exclusive prefixes, published as inclusive ones, to excl[].
+template <int CH>
+__device__ __forceinline__ void fewLookBack(const CullParams& P, const FewItem& f, uint32_t total, uint32_t epoch,
+                                            uint32_t* excl, uint32_t lane)
+{
+	const FewChain<CH> c(f, lane);
+	uint32_t e = 0;
+	if (!f.T.first) {
+		const WaitBound B{P.ctl, P.waitLimit, epoch};
+		if constexpr (CH == 1)
+			e = lookBackWave(c.chain - f.T.chain, f.T.chain, B, lane);
+		else
+			e = lookBackGroups<64 / CH>(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane);
+		if (c.lead) publish(c.chain, packStatus(epoch, kStatePrefix, e + total));
+	}
+	if (c.lead) {
+		excl[lane / (64 / CH)] = e;
+		if (f.T.last && f.T.k < f.J.numStateSets)
+			globalMut<uint32_t>(f.J.counts)[uint64_t(c.view) * f.J.numStateSets + f.T.k] = e + total;
 	}
 }
 
-template <int BLOCK, int ITEMS, int CH>
+// Every wave: its commands of an item, n[c] of them per view from slot off[c]
+// of the tile's run on.
+template <int CH, bool LDS, int N>
+__device__ __forceinline__ void fewStore(const FewItem& f, const MeshTable& staged, const uint32_t (*run)[N],
+                                         const uint32_t (&n)[CH], const uint32_t (&off)[CH], const uint32_t* excl,
+                                         uint32_t wave, uint32_t lane)
+{
+	const MeshTable meshes{staged.lds, globalPtr<cadrMesh>(f.J.meshes), LDS};
+#pragma unroll
+	for (int c = 0; c < CH; c++) {
+		if (n[c] == 0) continue;
+		const uint32_t pos = uniform(f.T.segBase + excl[c] + off[c]);
+		storeListed<LDS>(run[c], n[c], pos, f.T.start + wave * N, meshes, f.J.numMeshes, globalPtr<uint32_t>(f.J.meshIndex),
+		                 globalMut<uint32_t>(f.J.commands) + uint64_t(f.viewBegin + c) * f.J.commandStride * 5ull,
+		                 f.J.commandStride, lane);
+	}
+}
+
+template <int BLOCK, int ITEMS, int CH, bool DEFER, bool JOBS, bool LDS>
+__device__ __forceinline__ void cullFewItems(const CullParams& P, FewShared<BLOCK, ITEMS, CH, DEFER>& sh,
+                                             const cadrCullJob& only, uint32_t t, Shard shard, uint32_t epoch, uint32_t tid,
+                                             uint32_t lane, uint32_t wave)
+{
+	constexpr int WAVES = BLOCK / 64, WAVE_ITEMS = 64 * ITEMS;
+	const MeshTable staged{sh.meshes, nullptr, LDS};
+	uint32_t job = 0;
+	FewItem cur = fewItem<JOBS>(P, sh.offsets, only, t, BLOCK * ITEMS, job, lane), prev = cur;
+	float4 sp[ITEMS];
+	uint32_t mi[ITEMS], nPrev[CH], offPrev[CH], totalPrev = 0;
+	loadTileItems<ITEMS>(globalPtr<float4>(cur.J.spheres), globalPtr<uint32_t>(cur.J.meshIndex), cur.T,
+	                     wave * WAVE_ITEMS + lane, sp, mi);
+	bool pending = false;
+	for (uint32_t b = 0;; b ^= 1u) {
+		asm volatile("" : "+v"(lane));  // nothing derived from it stays in registers across tiles
+		uint32_t n[CH], off[CH];
+#pragma unroll
+		for (int c = 0; c < CH; c++) {
+			n[c] = 0;
+			if (cur.viewBegin + c < cur.viewEnd)
+				n[c] = listVisible<ITEMS>(sp, mi, cur.T, cur.J.numMeshes, loadView(cur.J.views, cur.viewBegin + c),
+				                          wave * WAVE_ITEMS, lane, sh.run[DEFER ? b : 0][wave][c]);
+			if (lane == 0) sh.cnt[b][c][wave] = n[c];
+		}
+		if (DEFER && tid == 0) sh.ticket[b] = itemOfTicket(shard, askTicket(P, shard));
+		__syncthreads();
+		FewItem next;
+		bool more = false;
+		auto takeNext = [&](FewItem& f) __attribute__((always_inline)) {
+			const uint32_t tn = uniform(sh.ticket[b]);
+			more = tn < P.totalWork;
+			if (more) {
+				f = fewItem<JOBS>(P, sh.offsets, only, tn, BLOCK * ITEMS, job, lane);
+				loadTileItems<ITEMS>(globalPtr<float4>(f.J.spheres), globalPtr<uint32_t>(f.J.meshIndex), f.T,
+				                     wave * WAVE_ITEMS + lane, sp, mi);
+			}
+		};
+		// the next item's loads, in flight through the look-back and the stores
+		if constexpr (DEFER) takeNext(next);
+#pragma unroll
+		for (int c = 0; c < CH; c++) {
+			off[c] = 0;
+			for (uint32_t q = 0; q < wave; q++) off[c] += sh.cnt[b][c][q];
+			off[c] = uniform(off[c]);
+		}
+		uint32_t total = 0;
+		if (wave == 0) {
+			for (int q = 0; q < WAVES; q++) total += sh.cnt[b][lane / (64 / CH)][q];
+			fewPublish<CH>(cur, total, epoch, lane);
+			if constexpr (DEFER) {
+				if (pending) fewLookBack<CH>(P, prev, totalPrev, epoch, sh.excl[b], lane);
+			} else {
+				fewLookBack<CH>(P, cur, total, epoch, sh.excl[b], lane);
+			}
+		}
+		__syncthreads();
+		if constexpr (DEFER) {
+			if (pending) fewStore<CH, LDS, WAVE_ITEMS>(prev, staged, sh.run[b ^ 1u][wave], nPrev, offPrev, sh.excl[b], wave, lane);
+			if (!more) {
+				if (wave == 0) fewLookBack<CH>(P, cur, total, epoch, sh.excl[b ^ 1u], lane);
+				__syncthreads();
+				if (wave == WAVES - 1 && lane == 0) leaveLaunch(P, shard, epoch);
+				fewStore<CH, LDS, WAVE_ITEMS>(cur, staged, sh.run[b][wave], n, off, sh.excl[b ^ 1u], wave, lane);
+				return;
+			}
+			prev = cur;
+			totalPrev = total;
+			pending = true;
+#pragma unroll
+			for (int c = 0; c < CH; c++) {
+				nPrev[c] = n[c];
+				offPrev[c] = off[c];
+			}
+			cur = next;
+		} else {
+			fewStore<CH, LDS, WAVE_ITEMS>(cur, staged, sh.run[0][wave], n, off, sh.excl[b], wave, lane);
+			if (tid == 0) sh.ticket[b] = itemOfTicket(shard, askTicket(P, shard));
+			__syncthreads();
+			takeNext(cur);
+			if (!more) break;
+		}
+	}
+	if (tid == 0) leaveLaunch(P, shard, epoch);
+}
+
+template <int BLOCK, int ITEMS, int CH, bool DEFER, bool JOBS>
 __global__ __launch_bounds__(BLOCK) void cullFewKernel(CullParams P)
 {
-	__shared__ FewShared<BLOCK, ITEMS, CH> sh;
+	__shared__ FewShared<BLOCK, ITEMS, CH, DEFER> sh;
 	const uint32_t tid = threadIdx.x, lane = laneId(), wave = uniform(tid / 64);
 	const Shard shard = homeShard<BLOCK * ITEMS>(P);
-	uint32_t job = 0, b = 0;
 	uint32_t ticket = 0;
 	if (tid == 0) ticket = askTicket(P, shard);
 	const uint32_t epoch = __hip_atomic_load(&P.ctl[kCtlEpoch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-	if (wave == 0 && P.numJobs > 1 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
 	bool ldsMeshes = false;
-	if (P.numJobs == 1) {
+	cadrCullJob only{};
+	if constexpr (JOBS) {
+		if (wave == 0 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
+	} else {
+		only = loadJob(P.jobs, 0);
 		MeshStaging<BLOCK> staging;
-		ldsMeshes = staging.load(loadJob(P.jobs, 0), tid);
+		ldsMeshes = staging.load(only, tid);
 		staging.store(sh.meshes, tid);
 	}
-	if (tid == 0) sh.ticket[0] = itemOfTicket(shard, ticket);
-	for (uint32_t k = 0;; k ^= 1u) {
-		__syncthreads();
-		const uint32_t t = uniform(sh.ticket[k]);
-		if (t >= P.totalWork) break;
-		job = jobOfWork(P, sh.offsets, t, job, lane);
-		const cadrCullJob J = loadJob(P.jobs, job);
-		const WorkItem item = workItem(P, J, t - firstWorkOf(P, sh.offsets, job));
-		const TileDesc T = loadTile(J, item.tile, BLOCK * ITEMS);
-		uint64_t* chain0 = P.status + statusBaseOf(P, sh.offsets, job);
-		const MeshTable meshes{sh.meshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
-		if (ldsMeshes)
-			cullFewTile<BLOCK, ITEMS, CH, true>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane,
-			                                    wave);
-		else
-			cullFewTile<BLOCK, ITEMS, CH, false>(P, J, T, item.viewBegin, item.viewEnd, chain0, epoch, meshes, sh, b, lane,
-			                                     wave);
-		// not earlier: a ticket held during the stores keeps its tile's followers
-		// waiting in their look-backs (24 served scenes: 98 -> 103 us)
-		if (tid == 0) sh.ticket[k ^ 1u] = itemOfTicket(shard, askTicket(P, shard));
+	if (tid == 0) sh.ticket[1] = itemOfTicket(shard, ticket);
+	__syncthreads();
+	const uint32_t t = uniform(sh.ticket[1]);
+	if (t >= P.totalWork) {
+		if (tid == 0) leaveLaunch(P, shard, epoch);
+		return;
 	}
-	if (tid == 0) leaveLaunch(P, shard, epoch);
+	if (!JOBS && ldsMeshes)
+		cullFewItems<BLOCK, ITEMS, CH, DEFER, JOBS, true>(P, sh, only, t, shard, epoch, tid, lane, wave);
+	else
+		cullFewItems<BLOCK, ITEMS, CH, DEFER, JOBS, false>(P, sh, only, t, shard, epoch, tid, lane, wave);
 }
 
 template <int BLOCK, int ITEMS>
@@ -1765,26 +1884,33 @@ struct KernelEntry {
 	KernelFn fused;       // leaf propagation + one view, or nullptr
 	KernelFn fusedBatch;  // leaf propagation + many views / jobs, or nullptr
 	KernelFn viewLoop;    // one view, persistent (cullViewLoopKernel), or nullptr where it is not faster
-	KernelFn few[3];      // few views per job, 1, 2 or 4 at a time (cullFewKernel), or nullptr
+	KernelFn few[2][3];   // few views per job, 1, 2 or 4 at a time (cullFewKernel): one job, many; or nullptr
 };
 
 // viewLoop where it measured faster than one tile per workgroup (10M
 // drawables, 64 StateSets, one view, 18% visible): 1024 x 2 / 4 / 8 74.0 / 62.5
 // / 58.8 against 94.6 / 67.0 / 59.6 us; not at 256 x 4 / 8 / 16 (67.5 / 65.0 /
-// 63.3 against 63.9 / 61.5 / 63.0) nor 512 x 4 (61.7 against 62.0, no more than
-// runs differ), where several workgroups of a CU overlap each other's phases.
+// 63.3 against 63.9 / 61.5 / 63.0), where several workgroups of a CU overlap
+// each other's phases (viewLoopOf has another kernel for the smaller tiles).
 // fusedBatch: parents read whole (COOP) and the items prefetched at 256 x 8,
 // held to 3 waves per SIMD (4 registers spilled); neither at 256 x 4 and 512 x
 // 4, held to 4.  64 uneven scenes, 1-32 views: 256 x 8 867 us (no prefetch 881,
 // neither 879, registers unbounded 1002), 256 x 4 855 (COOP 923, 3 waves 910),
 // 512 x 4 881 (3 waves with COOP 1255).
+#define FEW(B, I)                                                                                              \
+	{                                                                                                       \
+		{cullFewKernel<B, I, 1, true, false>, cullFewKernel<B, I, 2, true, false>,                        \
+		 cullFewKernel<B, I, 4, false, false>},                                                           \
+		{cullFewKernel<B, I, 1, true, true>, cullFewKernel<B, I, 2, true, true>,                          \
+		 cullFewKernel<B, I, 4, false, true>},                                                            \
+	}
 const KernelEntry kKernels[] = {
-    {256, 2, cullKernel<256, 2, false>, cullViewKernel<256, 2>, cullFusedKernel<256, 2, 4>, nullptr, nullptr, {cullFewKernel<256, 2, 1>, cullFewKernel<256, 2, 2>, cullFewKernel<256, 2, 4>}},
-    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true, false, 4>, nullptr, {cullFewKernel<256, 4, 1>, cullFewKernel<256, 4, 2>, cullFewKernel<256, 4, 4>}},
-    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true, 3>, nullptr, {cullFewKernel<256, 8, 1>, cullFewKernel<256, 8, 2>, cullFewKernel<256, 8, 4>}},
+    {256, 2, cullKernel<256, 2, false>, cullViewKernel<256, 2>, cullFusedKernel<256, 2, 4>, nullptr, nullptr, FEW(256, 2)},
+    {256, 4, cullKernel<256, 4, false>, cullViewKernel<256, 4>, cullFusedKernel<256, 4, 4>, cullKernel<256, 4, true, false, 4>, nullptr, FEW(256, 4)},
+    {256, 8, cullKernel<256, 8, false>, cullViewKernel<256, 8>, cullFusedKernel<256, 8, 1>, cullKernel<256, 8, true, true, 3>, nullptr, FEW(256, 8)},
     {256, 16, cullKernel<256, 16, false>, cullViewKernel<256, 16>, cullFusedKernel<256, 16, 1>, nullptr, nullptr},
     {512, 2, cullKernel<512, 2, false>, cullViewKernel<512, 2>, cullFusedKernel<512, 2, 1>, nullptr, nullptr},
-    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, false, 4>, nullptr, {cullFewKernel<512, 4, 1>, cullFewKernel<512, 4, 2>, cullFewKernel<512, 4, 4>}},
+    {512, 4, cullKernel<512, 4, false>, cullViewKernel<512, 4>, cullFusedKernel<512, 4, 1>, cullKernel<512, 4, true, false, 4>, nullptr, FEW(512, 4)},
     {512, 8, nullptr, cullViewKernel<512, 8>, nullptr, nullptr, nullptr},
     {512, 16, nullptr, cullViewKernel<512, 16>, nullptr, nullptr, nullptr},
     {1024, 1, nullptr, cullViewKernel<1024, 1>, cullFusedKernel<1024, 1, 1>, nullptr, cullViewLoopKernel<1024, 1>},
@@ -2023,6 +2149,15 @@ int checkLeaf(const cadrTransformLevel& L, const cadrCullJob& J, const std::stri
 	return CADR_SUCCESS;
 }
 
+// The persistent kernel of one view, or nullptr where one tile per workgroup
+// is faster: cullFewKernel at 256 x 2 and 256 / 512 x 4 (10M drawables, 64
+// StateSets 62.7 / 57.0 / 55.6 against 73.8 / 58.2 / 57.6 us, one StateSet 256
+// x 4 68.7 against 91.1), not at 256 x 8 (60.4 against 57.3).
+KernelFn viewLoopOf(const KernelEntry& ke)
+{
+	return ke.viewLoop ? ke.viewLoop : ke.items <= 4 ? ke.few[0][0] : nullptr;
+}
+
 // The few-view kernel for a launch, or nullptr where the many-view kernel
 // (cullKernel) is the faster one.  That one reads a tile once for 64 views and
 // skips the views that see none of it or all of it, but keeps its workgroups
@@ -2043,7 +2178,7 @@ KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t n
 	}
 	const bool split = (flags & CADR_CULL_WHOLE_TILES) == 0;
 	if (split ? tests > 16 * drawables && tests > (1ull << 25) : mostViews > 4) return nullptr;
-	return ke.few[mostViews <= 1 ? 0 : mostViews == 2 ? 1 : 2];
+	return ke.few[numJobs > 1][mostViews <= 1 ? 0 : mostViews == 2 ? 1 : 2];
 }
 
 // One persistent launch of a batched kernel over numJobs jobs; leaves: the
@@ -2171,12 +2306,14 @@ CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, cons
 	// more tiles than workgroups fit on the GPU at once: the persistent kernel
 	// (grid = resident workgroups); else one tile per workgroup, which saves
 	// the loop's extra ticket and barrier on a launch-bound view
-	const int resident = ke->viewLoop ? residentWorkgroups(ke->viewLoop, ke->block) : 0;
+	const KernelFn viewLoop = viewLoopOf(*ke);
+	const int resident = viewLoop ? residentWorkgroups(viewLoop, ke->block) : 0;
 	const bool loop = resident > 0 && hostJob->numTiles > uint32_t(resident);
 	const uint32_t grid = loop ? uint32_t(resident) : hostJob->numTiles;
 	p.shardShift = shardShiftFor(ke->block * ke->items, grid, hostJob->numTiles, jobBytes(*hostJob, false));
 	if (!loop) ke = shapeFor(ke, hostJob->numTiles, &KernelEntry::view);
-	launchKernel(loop ? ke->viewLoop : ke->view, dim3(grid), dim3(ke->block), hipStream_t(stream), p);
+	p.groupShift = 2;
+	launchKernel(loop ? viewLoop : ke->view, dim3(grid), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "cullViewKernel launch");
 	return ok();
 }

@@ -150,3 +150,9 @@ def test_fused_shape_by_tiles(gpu, block, items, fanouts):
     batch.close()
     out.close()
     ds.close()
+
+
+def test_deferred_look_back_over_many_tiles(gpu):
+    """Jobs of more tiles than workgroups, one and two views: each workgroup stores an item after it has taken the next."""
+    _run([(2_000_003, 3, 64, 2), (500_001, 5, 64, 1), (70, 1, 3, 2)], 256, 2, lambda b: b.run())
+    _run([(2_500_003, 1, 64, 1)], 256, 4, lambda b: b.run_view())
