@@ -79,4 +79,32 @@ __device__ __forceinline__ uint64_t lookupHandle(const uint64_t* __restrict__ ro
 	}
 }
 
+// lookupHandle of N handles at once, one table level after the other, so that
+// N loads are in flight at each level.  A handle that resolves to 0 on the
+// way loads the root table's first entry from there on, and its result is 0.
+template <int LEVEL, int N>
+__device__ __forceinline__ void lookupHandles(const uint64_t* __restrict__ rootTable, const uint64_t (&handle)[N],
+                                              uint64_t (&address)[N])
+{
+	const uint64_t root = reinterpret_cast<uint64_t>(rootTable);
+	bool ok[N];
+#pragma unroll
+	for (int k = 0; k < N; k++) {
+		const uint32_t i = LEVEL == 1 ? uint32_t(handle[k]) : uint32_t(handle[k] >> ((LEVEL - 1) * CADR_HANDLE_LEVEL_SHIFT));
+		ok[k] = i < CADR_HANDLES_PER_TABLE;
+		address[k] = globalAt<uint64_t>(root)[ok[k] ? i : 0u];
+	}
+#pragma unroll
+	for (int l = LEVEL - 2; l >= 0; l--) {
+#pragma unroll
+		for (int k = 0; k < N; k++) {
+			const uint32_t i = uint32_t(handle[k] >> (l * CADR_HANDLE_LEVEL_SHIFT)) & CADR_HANDLE_LEVEL_MASK;
+			ok[k] = ok[k] && address[k] != 0;
+			address[k] = globalAt<uint64_t>(ok[k] ? address[k] + 8ull * i : root)[0];
+		}
+	}
+#pragma unroll
+	for (int k = 0; k < N; k++) address[k] = ok[k] ? address[k] : 0;
+}
+
 }  // namespace cadr
