@@ -153,6 +153,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void p
 	__shared__ float4 stage[4][256];
 	__shared__ uint64_t firstUnit[kMaxBatchLevels + 1];
 	const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	if (numLevels <= 2u) {
+		// one or two levels (a frame's inner depths): both descriptors are loaded
+		// at once, which saves the scan's round trip
+		const cadrTransformLevel A = levels[0], B = levels[numLevels - 1u];
+		const uint64_t ua = (A.count + 63u) / 64u, total = ua + (numLevels == 2u ? (B.count + 63u) / 64u : 0u);
+		for (uint64_t unit = uint64_t(blockIdx.x) * 4u + wave; unit < total; unit += uint64_t(gridDim.x) * 4u) {
+			const bool first = unit < ua;
+			propagateUnit<SPHERES>(first ? A : B, (first ? unit : unit - ua) * 64u, stage[wave], lane);
+		}
+		return;
+	}
 	// firstUnit[l] = units of levels 0..l-1: loaded in parallel, then an
 	// in-place Hillis-Steele scan over the (at most 1024) levels
 	for (uint32_t i = threadIdx.x; i < numLevels; i += 256u) firstUnit[i + 1] = (levels[i].count + 63u) / 64u;
