@@ -220,21 +220,23 @@ __global__ __launch_bounds__(256) void worldSpheresKernel(const float4* __restri
 	spheres[i] = nodeSphere(W, meshes, numMeshes, meshIndex[i]);
 }
 
-// A transform plan's launch: one unit (level, first node) per wave, in the
-// plan's order; workgroups are dispatched in index order, so the waves in
-// flight at any time hold consecutive units of that order.
+// A transform plan's launch: one unit per wave, in the plan's order;
+// workgroups are dispatched in index order, so the waves in flight at any time
+// hold consecutive units of that order.  A unit is a level of its own, the
+// caller's level cut down to the unit's nodes, so a wave reads one descriptor
+// and not a unit and then its level: the chain of round trips, not the bytes,
+// is what a wave's time goes to.
 template <bool SPHERES>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void propagatePlanKernel(const cadrTransformLevel* __restrict__ levels,
-                                                           const uint2* __restrict__ units, uint64_t numUnits)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void propagatePlanKernel(const cadrTransformLevel* __restrict__ units,
+                                                           uint64_t numUnits)
 {
 	__shared__ float4 stage[4][256];
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const uint64_t u = uint64_t(blockIdx.x) * 4u + wave;
 	if (u >= numUnits) return;  // whole wave past the end (waves are independent)
-	const uint2 unit = units[u];
-	const cadrTransformLevel L = levels[unit.x];
-	propagateUnit<SPHERES>(L, uint64_t(unit.y), stage[wave], lane);
+	const cadrTransformLevel L = units[u];
+	propagateUnit<SPHERES>(L, 0u, stage[wave], lane);
 }
 
 // The sort key of each unit of a plan: the parent index of its first node
@@ -250,12 +252,31 @@ __global__ __launch_bounds__(256) void planKeysKernel(const cadrTransformLevel* 
 	keys[u] = L.parentWorld ? reinterpret_cast<const uint32_t*>(L.parentIndex)[unit.y] : 0u;
 }
 
+// A plan's units from (level, first node) pairs: each a level of at most 64
+// nodes, its arrays moved on to the first of them.
+__global__ __launch_bounds__(256) void planUnitsKernel(const cadrTransformLevel* __restrict__ levels,
+                                                       const uint2* __restrict__ order, uint64_t numUnits,
+                                                       cadrTransformLevel* __restrict__ units)
+{
+	const uint64_t u = uint64_t(blockIdx.x) * 256u + threadIdx.x;
+	if (u >= numUnits) return;
+	const uint2 unit = order[u];
+	cadrTransformLevel L = levels[unit.x];
+	const uint64_t first = unit.y;
+	L.localMatrices += 64 * first;
+	L.worldMatrices += 64 * first;
+	L.parentIndex += 4 * first;
+	L.meshIndex += 4 * first;
+	if (L.spheres) L.spheres += 16 * first;
+	L.count = min(L.count - first, uint64_t(64));
+	units[u] = L;
+}
+
 }  // namespace cadr
 
 struct cadrTransformPlan {
 	int device = 0;
-	cadrTransformLevel* levels = nullptr;  // device copy of the descriptors
-	uint2* units = nullptr;                // (level, first node), in launch order
+	cadrTransformLevel* units = nullptr;   // 64 nodes of a level each, in launch order
 	uint64_t numUnits = 0;
 	bool spheres = false;                  // some level writes world spheres
 };
@@ -366,24 +387,33 @@ CADR_API int cadrTransformPlanCreate(const cadrTransformLevel* hostLevels, uint3
 	CADR_CHECK_HIP(hipGetDevice(&p->device), "hipGetDevice");
 	p->numUnits = units.size();
 	hipStream_t s = hipStream_t(stream);
+	cadrTransformLevel* dLevels = nullptr;  // what the units are made from, until they are
+	uint2* dOrder = nullptr;
 	uint32_t* dKeys = nullptr;
-	auto fail = [&](hipError_t e, const char* what) {
+	auto release = [&]() {
+		(void)hipFree(dLevels);
+		(void)hipFree(dOrder);
 		(void)hipFree(dKeys);
+	};
+	auto fail = [&](hipError_t e, const char* what) {
+		release();
 		cadrTransformPlanDestroy(p);
 		return setHipError(e, what);
 	};
-	hipError_t e = hipMalloc(&p->levels, std::max<size_t>(numLevels, 1) * sizeof(cadrTransformLevel));
-	if (e != hipSuccess) return fail(e, "hipMalloc(plan levels)");
-	e = hipMalloc(&p->units, std::max<size_t>(units.size(), 1) * sizeof(uint2));
-	if (e != hipSuccess) return fail(e, "hipMalloc(plan units)");
 	if (!units.empty()) {
+		hipError_t e = hipMalloc(&p->units, units.size() * sizeof(cadrTransformLevel));
+		if (e != hipSuccess) return fail(e, "hipMalloc(plan units)");
+		e = hipMalloc(&dLevels, numLevels * sizeof(cadrTransformLevel));
+		if (e != hipSuccess) return fail(e, "hipMalloc(plan levels)");
+		e = hipMalloc(&dOrder, units.size() * sizeof(uint2));
+		if (e != hipSuccess) return fail(e, "hipMalloc(plan order)");
 		e = hipMalloc(&dKeys, units.size() * sizeof(uint32_t));
 		if (e != hipSuccess) return fail(e, "hipMalloc(plan keys)");
-		e = hipMemcpyAsync(p->levels, hostLevels, numLevels * sizeof(cadrTransformLevel), hipMemcpyHostToDevice, s);
-		if (e == hipSuccess) e = hipMemcpyAsync(p->units, units.data(), units.size() * sizeof(uint2), hipMemcpyHostToDevice, s);
+		e = hipMemcpyAsync(dLevels, hostLevels, numLevels * sizeof(cadrTransformLevel), hipMemcpyHostToDevice, s);
+		if (e == hipSuccess) e = hipMemcpyAsync(dOrder, units.data(), units.size() * sizeof(uint2), hipMemcpyHostToDevice, s);
 		if (e != hipSuccess) return fail(e, "hipMemcpyAsync(plan)");
-		hipLaunchKernelGGL(planKeysKernel, dim3(uint32_t((units.size() + 255) / 256)), dim3(256), 0, s, p->levels,
-		                   p->units, uint64_t(units.size()), dKeys);
+		const dim3 grid(uint32_t((units.size() + 255) / 256));
+		hipLaunchKernelGGL(planKeysKernel, grid, dim3(256), 0, s, dLevels, dOrder, uint64_t(units.size()), dKeys);
 		e = hipGetLastError();
 		if (e != hipSuccess) return fail(e, "planKeysKernel launch");
 		std::vector<uint32_t> keys(units.size());
@@ -401,10 +431,13 @@ CADR_API int cadrTransformPlanCreate(const cadrTransformLevel* hostLevels, uint3
 		});
 		std::vector<uint2> sorted(units.size());
 		for (size_t i = 0; i < order.size(); i++) sorted[i] = units[order[i]];
-		e = hipMemcpy(p->units, sorted.data(), sorted.size() * sizeof(uint2), hipMemcpyHostToDevice);
-		if (e != hipSuccess) return fail(e, "hipMemcpy(plan units)");
-		(void)hipFree(dKeys);
-		dKeys = nullptr;
+		e = hipMemcpyAsync(dOrder, sorted.data(), sorted.size() * sizeof(uint2), hipMemcpyHostToDevice, s);
+		if (e != hipSuccess) return fail(e, "hipMemcpyAsync(plan order)");
+		hipLaunchKernelGGL(planUnitsKernel, grid, dim3(256), 0, s, dLevels, dOrder, uint64_t(units.size()), p->units);
+		e = hipGetLastError();
+		if (e == hipSuccess) e = hipStreamSynchronize(s);  // the launches may come on other streams
+		if (e != hipSuccess) return fail(e, "planUnitsKernel");
+		release();
 	}
 	*plan = p;
 	return ok();
@@ -420,7 +453,7 @@ CADR_API int cadrPropagateTransformsPlanned(const cadrTransformPlan* plan, cadrS
 	const uint64_t blocks = (plan->numUnits + 3) / 4;
 	CADR_REQUIRE(blocks < (1ull << 31), "cadrPropagateTransformsPlanned: plan too large");
 	launchKernel(plan->spheres ? propagatePlanKernel<true> : propagatePlanKernel<false>, dim3(uint32_t(blocks)),
-	             dim3(256), hipStream_t(stream), plan->levels, plan->units, plan->numUnits);
+	             dim3(256), hipStream_t(stream), plan->units, plan->numUnits);
 	CADR_CHECK_HIP(hipGetLastError(), "propagatePlanKernel launch");
 	return ok();
 }
@@ -428,7 +461,6 @@ CADR_API int cadrPropagateTransformsPlanned(const cadrTransformPlan* plan, cadrS
 CADR_API void cadrTransformPlanDestroy(cadrTransformPlan* plan)
 {
 	if (!plan) return;
-	(void)hipFree(plan->levels);
 	(void)hipFree(plan->units);
 	delete plan;
 }
