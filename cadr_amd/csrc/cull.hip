@@ -1968,6 +1968,17 @@ const KernelEntry* shapeFor(const KernelEntry* ke, uint32_t numTiles, KernelFn K
 	return best;
 }
 
+// The same for a batched launch: 512 x 4 for 256 x 8, the one pair of shapes
+// that has every batched kernel (150k drawables, 4 / 20 views: 14.4 / 21.0 us at
+// 256 x 8, 11.4 / 18.4 at 512 x 4; 400k, 196 tiles, 16.1 / 29.4 and 13.1 / 28.4;
+// 12 small trees, leaves fused, 49.5 and 39.8).
+const KernelEntry* batchShapeFor(const KernelEntry* ke, uint64_t tiles, KernelFn KernelEntry::*path)
+{
+	if (tiles > 0xffffffffull) return ke;
+	const KernelEntry* wide = shapeFor(ke, uint32_t(tiles), path);
+	return ke->few[0][0] && wide->few[0][0] ? wide : ke;
+}
+
 }  // namespace
 
 bool cadr::cullHasKernel(const cadrCullConfig* c, CullPath path)
@@ -2165,25 +2176,31 @@ KernelFn viewLoopOf(const KernelEntry& ke)
 // time, in many more work items.  Measured at 256 x 8, trees of clustered
 // drawables, few against many: 12 views 4M drawables 93 / 107 us, 2M 53 / 59;
 // 37 views 100k 19 / 39, 333k 33 / 45, 1M 68 / 62; 64 views 333k 43 / 64, 1M
-// 105 / 86; 128 views 100k 33 / 64, 333k 75 / 75.  So few wins up to about 16
-// views a drawable, and for more views up to about 2^25 tests in the launch.
+// 105 / 86; 128 views 100k 33 / 64, 333k 75 / 75; 512 x 4: 16 views 865k 33 /
+// 36, 27 views 1.2M 70 / 62.  So few wins up to about 16 views a drawable, and
+// for more views where the tiles do not fill the chip twice and the launch has
+// no more than about 2^25 tests.
 KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t numJobs, uint32_t flags)
 {
-	uint64_t drawables = 0, tests = 0;
+	uint64_t drawables = 0, tests = 0, tiles = 0;
 	uint32_t mostViews = 0;
 	for (uint32_t j = 0; j < numJobs; j++) {
-		drawables += jobs[j].numDrawables;
-		tests += uint64_t(jobs[j].numDrawables) * jobs[j].numViews;
+		// (a tile of few or no drawables costs what some 256 tests do)
+		const uint64_t n = std::max<uint64_t>(jobs[j].numDrawables, 256ull * jobs[j].numTiles);
+		drawables += n;
+		tests += n * jobs[j].numViews;
+		tiles += jobs[j].numTiles;
 		mostViews = std::max(mostViews, jobs[j].numViews);
 	}
 	const bool split = (flags & CADR_CULL_WHOLE_TILES) == 0;
-	if (split ? tests > 16 * drawables && tests > (1ull << 25) : mostViews > 4) return nullptr;
+	const bool small = tiles <= 512 && tests <= (1ull << 25);
+	if (split ? tests > 16 * drawables && !small : mostViews > 4) return nullptr;
 	return ke.few[numJobs > 1][mostViews <= 1 ? 0 : mostViews == 2 ? 1 : 2];
 }
 
 // One persistent launch of a batched kernel over numJobs jobs; leaves: the
 // fused form's leaf levels (device memory), else null.
-int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config, uint64_t deviceJobs,
+int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cadrCullConfig* config, uint64_t deviceJobs,
                 const cadrCullJob* hostJobs, uint32_t numJobs, cadrCullWorkspace* ws, cadrStream stream,
                 const cadrTransformLevel* leaves, const std::string& name)
 {
@@ -2195,6 +2212,10 @@ int launchBatch(KernelFn fn, const KernelEntry& ke, const cadrCullConfig* config
 	// the persistent grid; unless CADR_CULL_WHOLE_TILES, a job's last grid
 	// tiles are handed out per view group
 	const int cu = computeUnitCount();
+	uint64_t tiles = 0;
+	for (uint32_t j = 0; j < numJobs; j++) tiles += hostJobs[j].numTiles;
+	const KernelEntry& ke = *batchShapeFor(&asked, tiles, path);
+	KernelFn fn = ke.*path;
 	uint32_t perCU = config->workgroupsPerCU;
 	if (perCU == 0) perCU = ke.block >= 512 ? 2 : 4;
 	uint64_t grid = uint64_t(cu > 0 ? cu : 256) * perCU;
@@ -2257,7 +2278,7 @@ CADR_API int cadrCullBatch(const cadrCullConfig* config, uint64_t deviceJobs, co
 {
 	const KernelEntry* ke = findKernel(config);
 	CADR_REQUIRE(ke && ke->batch, "cadrCullBatch: unsupported blockSize/itemsPerThread");
-	return launchBatch(ke->batch, *ke, config, deviceJobs, hostJobs, numJobs, ws, stream, nullptr, "cadrCullBatch");
+	return launchBatch(&KernelEntry::batch, *ke, config, deviceJobs, hostJobs, numJobs, ws, stream, nullptr, "cadrCullBatch");
 }
 
 CADR_API int cadrPropagateCullBatch(uint64_t deviceLeaves, const cadrTransformLevel* hostLeaves,
@@ -2274,7 +2295,7 @@ CADR_API int cadrPropagateCullBatch(uint64_t deviceLeaves, const cadrTransformLe
 		const int rc = checkLeaf(hostLeaves[j], hostJobs[j], "cadrPropagateCullBatch");
 		if (rc != CADR_SUCCESS) return rc;
 	}
-	return launchBatch(ke->fusedBatch, *ke, config, deviceJobs, hostJobs, numJobs, ws, stream,
+	return launchBatch(&KernelEntry::fusedBatch, *ke, config, deviceJobs, hostJobs, numJobs, ws, stream,
 	                   reinterpret_cast<const cadrTransformLevel*>(deviceLeaves), "cadrPropagateCullBatch");
 }
 
@@ -2450,6 +2471,6 @@ CADR_API int cadrCullBatchNoAlloc(const cadrCullConfig* config, uint64_t deviceJ
 	w.device = dev;
 	w.ticksPerUs = sd.ticksPerUs;
 	w.waitLimit = kDefaultWaitLimitUs * sd.ticksPerUs;
-	return launchBatch(ke->batch, *ke, config, deviceJobs, hostJobs, numJobs, &w, stream, nullptr,
+	return launchBatch(&KernelEntry::batch, *ke, config, deviceJobs, hostJobs, numJobs, &w, stream, nullptr,
 	                   "cadrCullBatchNoAlloc");
 }

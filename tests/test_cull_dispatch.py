@@ -156,3 +156,10 @@ def test_deferred_look_back_over_many_tiles(gpu):
     """Jobs of more tiles than workgroups, one and two views: each workgroup stores an item after it has taken the next."""
     _run([(2_000_003, 3, 64, 2), (500_001, 5, 64, 1), (70, 1, 3, 2)], 256, 2, lambda b: b.run())
     _run([(2_500_003, 1, 64, 1)], 256, 4, lambda b: b.run_view())
+
+
+# batched launches of at most one tile a compute unit run 256 x 8 tiles with 512 threads
+@pytest.mark.parametrize("tiles", [1, 256, 257])
+@pytest.mark.parametrize("views", [1, 3, 18])
+def test_batch_shape_by_tiles(gpu, tiles, views):
+    _run([(tiles * 2048 - 5, 1, 64, views)], 256, 8, lambda b: b.run())
