@@ -1922,6 +1922,12 @@ const KernelEntry kKernels[] = {
     {128, 16, cullKernel<128, 16, false>, nullptr, nullptr, nullptr, nullptr},
 };
 
+uint32_t computeUnits()
+{
+	const int cu = computeUnitCount();
+	return cu > 0 ? uint32_t(cu) : 256u;
+}
+
 // Workgroups of kernel fn (block threads) resident on the current device at
 // once: compute units x workgroups per CU by the occupancy calculator,
 // cached per (device, kernel).  0 if the query fails.
@@ -1958,10 +1964,9 @@ const KernelEntry* findKernel(const cadrCullConfig* c)
 // shorter (100k drawables, 256 x 4 against 1024 x 1: 7.4 / 6.8 us; a tree frame
 // of 41k leaves 19.0 / 17.7 us, of 400k leaves, 391 tiles, 29.6 / 31.0 us).
 // The fused kernel is kept at 512 threads: 41k leaves 20.4 / 20.6 us.
-const KernelEntry* shapeFor(const KernelEntry* ke, uint32_t numTiles, KernelFn KernelEntry::*path)
+const KernelEntry* shapeFor(const KernelEntry* ke, uint32_t numTiles, uint32_t cu, KernelFn KernelEntry::*path)
 {
-	const int cu = computeUnitCount();
-	if (numTiles > uint32_t(cu > 0 ? cu : 256)) return ke;
+	if (numTiles > cu) return ke;
 	const KernelEntry* best = ke;
 	for (const KernelEntry& k : kKernels)
 		if (k.block * k.items == ke->block * ke->items && k.block > best->block && k.*path) best = &k;
@@ -1972,10 +1977,10 @@ const KernelEntry* shapeFor(const KernelEntry* ke, uint32_t numTiles, KernelFn K
 // that has every batched kernel (150k drawables, 4 / 20 views: 14.4 / 21.0 us at
 // 256 x 8, 11.4 / 18.4 at 512 x 4; 400k, 196 tiles, 16.1 / 29.4 and 13.1 / 28.4;
 // 12 small trees, leaves fused, 49.5 and 39.8).
-const KernelEntry* batchShapeFor(const KernelEntry* ke, uint64_t tiles, KernelFn KernelEntry::*path)
+const KernelEntry* batchShapeFor(const KernelEntry* ke, uint64_t tiles, uint32_t cu, KernelFn KernelEntry::*path)
 {
-	if (tiles > 0xffffffffull) return ke;
-	const KernelEntry* wide = shapeFor(ke, uint32_t(tiles), path);
+	if (tiles > cu) return ke;
+	const KernelEntry* wide = shapeFor(ke, uint32_t(tiles), cu, path);
 	return ke->few[0][0] && wide->few[0][0] ? wide : ke;
 }
 
@@ -2211,14 +2216,14 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	CADR_REQUIRE(numJobs <= ws->maxJobs, name + ": more jobs than the workspace was created for");
 	// the persistent grid; unless CADR_CULL_WHOLE_TILES, a job's last grid
 	// tiles are handed out per view group
-	const int cu = computeUnitCount();
+	const uint32_t cu = computeUnits();
 	uint64_t tiles = 0;
 	for (uint32_t j = 0; j < numJobs; j++) tiles += hostJobs[j].numTiles;
-	const KernelEntry& ke = *batchShapeFor(&asked, tiles, path);
+	const KernelEntry& ke = *batchShapeFor(&asked, tiles, cu, path);
 	KernelFn fn = ke.*path;
 	uint32_t perCU = config->workgroupsPerCU;
 	if (perCU == 0) perCU = ke.block >= 512 ? 2 : 4;
-	uint64_t grid = uint64_t(cu > 0 ? cu : 256) * perCU;
+	uint64_t grid = uint64_t(cu) * perCU;
 	const KernelFn few = leaves ? nullptr : fewKernelFor(ke, hostJobs, numJobs, config->flags);
 	uint32_t splitTiles = uint32_t(std::min<uint64_t>(grid, 1u << 20)), groupShift = 6;
 	if (few) {
@@ -2227,6 +2232,13 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 		groupShift = 2;
 		if (config->workgroupsPerCU == 0)
 			if (const int resident = residentWorkgroups(few, ke.block)) grid = uint64_t(resident);
+	}
+	else if (leaves && tiles <= cu / 2) {
+		// a fused launch of few tiles: four views a work item, each item
+		// computing the tile's leaves again (12 trees, 74 tiles, 1-16 views: 40.8
+		// -> 32.2 us; 171 tiles 39.8 -> 41.9, so not there)
+		splitTiles = 0xffffffffu;
+		groupShift = 2;
 	}
 	if (config->flags & CADR_CULL_WHOLE_TILES) splitTiles = 0;
 	uint64_t totalWork = 0, statusNeed = 0, bytes = 0;
@@ -2327,12 +2339,13 @@ CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, cons
 	// more tiles than workgroups fit on the GPU at once: the persistent kernel
 	// (grid = resident workgroups); else one tile per workgroup, which saves
 	// the loop's extra ticket and barrier on a launch-bound view
-	const KernelFn viewLoop = viewLoopOf(*ke);
+	const uint32_t cu = computeUnits();
+	const KernelFn viewLoop = hostJob->numTiles > cu ? viewLoopOf(*ke) : nullptr;  // a CU holds one workgroup at least
 	const int resident = viewLoop ? residentWorkgroups(viewLoop, ke->block) : 0;
 	const bool loop = resident > 0 && hostJob->numTiles > uint32_t(resident);
 	const uint32_t grid = loop ? uint32_t(resident) : hostJob->numTiles;
 	p.shardShift = shardShiftFor(ke->block * ke->items, grid, hostJob->numTiles, jobBytes(*hostJob, false));
-	if (!loop) ke = shapeFor(ke, hostJob->numTiles, &KernelEntry::view);
+	if (!loop) ke = shapeFor(ke, hostJob->numTiles, cu, &KernelEntry::view);
 	p.groupShift = 2;
 	launchKernel(loop ? viewLoop : ke->view, dim3(grid), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "cullViewKernel launch");
@@ -2370,7 +2383,7 @@ CADR_API int cadrPropagateCullView(const cadrTransformLevel* leaf, const cadrCul
 	                    leaf->parentWorld ? leaf->parentCount : 0u};
 	p.shardShift = shardShiftFor(ke->block * ke->items, hostJob->numTiles, hostJob->numTiles,
 	                             jobBytes(*hostJob, true));
-	if (ke->block < 512) ke = shapeFor(ke, hostJob->numTiles, &KernelEntry::fused);
+	if (ke->block < 512) ke = shapeFor(ke, hostJob->numTiles, computeUnits(), &KernelEntry::fused);
 	launchKernel(ke->fused, dim3(hostJob->numTiles), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "fused cullViewKernel launch");
 	return ok();

@@ -163,3 +163,37 @@ def test_deferred_look_back_over_many_tiles(gpu):
 @pytest.mark.parametrize("views", [1, 3, 18])
 def test_batch_shape_by_tiles(gpu, tiles, views):
     _run([(tiles * 2048 - 5, 1, 64, views)], 256, 8, lambda b: b.run())
+
+
+# fused batches: few tiles are cut by four views (each item computes its leaves again, one of them stores them), more
+# tiles and CULL_WHOLE_TILES are not
+@pytest.mark.parametrize("block,items,flags,fanouts", [(256, 4, 0, (3, 50, 21)), (256, 4, N.CULL_WHOLE_TILES, (3, 50, 21)),
+                                                       (256, 8, 0, (2, 30, 40)), (512, 4, N.CULL_WHOLE_TILES, (2, 30, 40)),
+                                                       (256, 4, 0, (2, 300, 260))])
+def test_fused_batch_view_groups(gpu, block, items, flags, fanouts):
+    print(f"{fanouts} {block}x{items} flags {flags}", flush=True)
+    jobs, leaves, worlds = [], [], []
+    for j, V in enumerate((9, 2, 70)):
+        scene = scenes.tree_scene((fanouts[0] + j,) + fanouts[1:], seed=scenes.SEED_BASE + 970 + j, num_statesets=3)
+        w, spheres = oracle.propagate_scene(scene)
+        ds = cull.DeviceScene(scene)
+        descs = ds.level_descs(spheres=False)
+        for lv in descs[:-1]:
+            N.check(N.load().cadrPropagateTransforms(N.ptr(lv), None))
+        views = cull.make_views(scenes.random_cameras(13 + j, 20, 0, V, 150.0))
+        jobs.append((ds, views, cull.CullOutputs(V, ds.n, ds.K), spheres, scene))
+        leaves.append(descs[-1])
+        worlds.append(w[-1])
+    batch = cull.CullBatch(cull.make_config(block, items, flags=flags), [j[:3] for j in jobs])
+    batch.set_leaves(np.concatenate(leaves))
+    for k in range(2):
+        batch.run_fused_batch()
+        synchronize()
+        batch.workspace.check()
+        _check(jobs, f"fused batch launch {k}")
+    for (ds, _, out, _, _), w in zip(jobs, worlds):
+        assert ds.world_matrices(-1).tobytes() == w.tobytes()
+        out.close()
+    batch.close()
+    for ds, *_ in jobs:
+        ds.close()
