@@ -420,7 +420,9 @@ typedef struct cadrCullJob {
 	uint32_t numMeshes;         /* drawables with meshIndex >= numMeshes are never visible */
 } cadrCullJob;                  /* 80 B */
 
-/* Kernel shape.  tileSize = blockSize * itemsPerThread. */
+/* Kernel shape.  tileSize = blockSize * itemsPerThread.  A launch whose tiles
+ * do not fill the compute units once may run another shape of the same tile
+ * size; results do not depend on it. */
 typedef struct cadrCullConfig {
 	uint32_t blockSize;         /* 256 or 512 threads                          */
 	uint32_t itemsPerThread;    /* 2, 4, 8 or 16                               */
@@ -432,7 +434,8 @@ typedef struct cadrCullConfig {
 /* Batched launches: every work item is one tile for all of its job's views.
  * By default the last (persistent grid size) tiles of a job with more than
  * 64 views are handed out as one work item per (tile, 64-view group), so the
- * launch's last work items are short and its workgroups finish together. */
+ * launch's last work items are short and its workgroups finish together, and
+ * launches of few views or few tiles as one per (tile, four views). */
 #define CADR_CULL_WHOLE_TILES 2u
 
 /* Device workspace of the cull launches: look-back status words, tile
