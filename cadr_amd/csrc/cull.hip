@@ -9,7 +9,7 @@
 //
 // Work is split into tiles of at most blockSize*itemsPerThread drawables that
 // never cross a StateSet boundary; tiles are taken by atomic tickets in array
-// order (dealt over several counters where small tiles need it, takeTicket),
+// order (dealt over several counters where small tiles need it, askTicket),
 // so a tile only ever waits on tiles that already run or come next.  Within a
 // tile, wave w owns a contiguous run of 64*itemsPerThread drawables (item j of
 // lane l is drawable w*64*itemsPerThread + j*64 + l): loads are coalesced and
@@ -21,14 +21,15 @@
 // launch epoch and never cleared.
 //
 // Five kernels:
-//   cullViewKernel - one view: one workgroup per tile, visibility kept in
-//     registers, a 64-lane parallel look-back in wave 0, each visible
-//     drawable's lane storing its command at its compacted slot.  It resets
-//     its tickets and advances the epoch itself (the last workgroup to
-//     finish), so a view costs one launch.
+//   cullViewKernel - one view: one workgroup per tile, a 64-lane parallel
+//     look-back in wave 0; each wave lists its visible drawables in LDS and
+//     stores their commands with full lanes.  It resets its tickets and
+//     advances the epoch itself (the last workgroup to finish), so a view
+//     costs one launch.
 //   cullViewLoopKernel - the same view pass as a persistent loop over tiles,
 //     the next tile's loads in flight during the current tile's look-back
-//     and stores; used when a view has more tiles than resident workgroups.
+//     and stores; used when a view has more tiles than resident workgroups,
+//     at the shapes where it is the faster one (viewLoopOf).
 //   cullFusedKernel - the same for one view, with the tile's spheres computed
 //     from the last transform level instead of read (cadrPropagateCullView).
 //   cullKernel - many views and many scenes (jobs) in one persistent launch:
@@ -40,7 +41,8 @@
 //     skip the per-drawable test when the items are wholly outside or inside
 //     the frustum.
 //   cullFewKernel - jobs of few views, or small launches: work items of one
-//     tile and up to four views, visible items listed per view.
+//     tile and up to four views, visible items listed per view; with one view
+//     also the persistent kernel of the small tiles (viewLoopOf).
 #include "internal.h"
 #include "launch.h"
 #include "fp32.h"
@@ -677,8 +679,8 @@ struct MeshStaging {
 // loadTileItems); with PREFETCH the local block and parent matrix of item
 // j+1 are issued before item j is computed, so each item's loads overlap the
 // previous item's work.  The batched kernel prefetches only with 8 items per
-// thread: with 4, the 32 registers of the prefetch drop it from 3 to 2 waves
-// per SIMD for the whole view loop (measured slower).
+// thread (both sides measured, at kKernels): with 4 it runs 4 waves per SIMD
+// and has no registers for it.
 struct ItemLoads {
 	float4 raw[4];  // this lane's 4 float4 of the wave's 4-KiB local block
 	float4 P[4];    // this lane's parent world matrix, or with COOP its 4 float4 of the
