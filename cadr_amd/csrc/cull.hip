@@ -1465,7 +1465,7 @@ struct CullShared {
 	uint32_t base[kViewGroup][WAVES];  // a wave's first output slot in its view's StateSet segment
 
 	uint32_t meshes[16 * kLdsMeshes];
-	uint32_t ticket;
+	uint32_t ticket[2];
 	JobOffsets offsets;
 };
 
@@ -1495,10 +1495,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 	// the first ticket's barrier stands between this and the first use
 	if (wave == 0 && P.numJobs > 1 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
 
-	for (;;) {
-		if (tid == 0) sh.ticket = itemOfTicket(shard, askTicket(P, shard));
+	// Two tickets in turn: an item's body need hold no barrier (a job without
+	// views takes no view group), so a wave may still have to read one ticket
+	// when thread 0 writes the next; it has read it by that one's barrier.
+	for (uint32_t b = 0;; b ^= 1u) {
+		if (tid == 0) sh.ticket[b] = itemOfTicket(shard, askTicket(P, shard));
 		__syncthreads();
-		const uint32_t w = uniform(sh.ticket);
+		const uint32_t w = uniform(sh.ticket[b]);
 		if (w >= P.totalWork) break;
 		// a lane index of its own for each tile: the compiler otherwise keeps
 		// dozens of addresses derived from it in registers across tiles

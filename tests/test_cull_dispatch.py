@@ -197,3 +197,16 @@ def test_fused_batch_view_groups(gpu, block, items, flags, fanouts):
     batch.close()
     for ds, *_ in jobs:
         ds.close()
+
+
+# jobs without views first, in the middle and last, of one tile and of many, beside jobs of few and many views: such a
+# job has no look-back chains and no outputs, and the others' are what they are without it
+NO_VIEWS = [(70_001, 1, 64, 0), (9000, 2, 64, 70), (1, 1, 8, 0), (70_001, 3, 65, 0), (5000, 1, 64, 2), (70_001, 1, 64, 0)]
+
+
+@pytest.mark.parametrize("block,items,flags", [(256, 4, N.CULL_WHOLE_TILES), (256, 8, N.CULL_WHOLE_TILES), (256, 16, 0),
+                                               (512, 2, 0), (128, 8, 0)])
+def test_jobs_without_views_many(gpu, block, items, flags):
+    """The many-view kernel (shapes without a few-view one, or whole tiles for 70 views)."""
+    print(f"{block}x{items} flags {flags}", flush=True)
+    _run(NO_VIEWS, block, items, lambda b: b.run(), flags)
