@@ -1094,10 +1094,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 
 // Work items of a job in a batched launch: its tiles, plus one more per
 // extra view group for each of its last splitTiles tiles (workItem's rule).
+// A job without views has nothing to test and owns no status words: no items,
+// except in a fused launch (leaves), which writes its leaf level.
 // The host checks that a launch's total fits 32 bits.
 __host__ __device__ __forceinline__ uint64_t jobWorkItems(uint32_t numTiles, uint32_t numViews, uint32_t splitTiles,
-                                                          uint32_t groupShift)
+                                                          uint32_t groupShift, bool leaves)
 {
+	if (numViews == 0 && !leaves) return 0;
 	const uint64_t groups = (uint64_t(numViews) + (1u << groupShift) - 1) >> groupShift;
 	const uint64_t split = groups > 1 ? (numTiles < splitTiles ? numTiles : splitTiles) : 0u;
 	return numTiles + split * (groups - 1);
@@ -1153,7 +1156,7 @@ __device__ __forceinline__ void findJobOffsets(const CullParams& P, JobOffsets& 
 		if (j < P.numJobs) {
 			const gptr<uint32_t> q = globalPtr<uint32_t>(addr(P.jobs) + uint64_t(j) * sizeof(cadrCullJob) + 56);
 			const uint32_t tiles = q[1], views = q[3];
-			w = uint32_t(jobWorkItems(tiles, views, P.splitTiles, P.groupShift));
+			w = uint32_t(jobWorkItems(tiles, views, P.splitTiles, P.groupShift, P.leaves != nullptr));
 			st = uint64_t(views) * tiles;
 		}
 		uint32_t wi = w;
@@ -1308,7 +1311,7 @@ __device__ __forceinline__ void fewLookBack(const CullParams& P, const FewItem& 
 	if (!f.T.first) {
 		const WaitBound B{P.ctl, P.waitLimit, epoch};
 		if constexpr (CH == 1)
-			e = lookBackWave(c.chain - f.T.chain, f.T.chain, B, lane);
+			e = lookBackWave(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane);
 		else
 			e = lookBackGroups<64 / CH>(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane);
 		if (c.lead) publish(c.chain, packStatus(epoch, kStatePrefix, e + total));
@@ -1495,9 +1498,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 	// the first ticket's barrier stands between this and the first use
 	if (wave == 0 && P.numJobs > 1 && P.numJobs <= kInlineJobs) findJobOffsets(P, sh.offsets, lane);
 
-	// Two tickets in turn: an item's body need hold no barrier (a job without
-	// views takes no view group), so a wave may still have to read one ticket
-	// when thread 0 writes the next; it has read it by that one's barrier.
+	// Two tickets in turn: the barriers of an item's body are inside its view
+	// groups, so without them a wave could still have to read one ticket when
+	// thread 0 writes the next; it has read it by that one's barrier.
 	for (uint32_t b = 0;; b ^= 1u) {
 		if (tid == 0) sh.ticket[b] = itemOfTicket(shard, askTicket(P, shard));
 		__syncthreads();
@@ -1797,7 +1800,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 // Job offsets of a batched launch of more than kInlineJobs jobs (prefix sums
 // over jobs); one block, before the cull kernel on the same stream.
 __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __restrict__ jobs, uint32_t numJobs,
-                                                       uint32_t splitTiles, uint32_t groupShift,
+                                                       uint32_t splitTiles, uint32_t groupShift, bool leaves,
                                                        uint32_t* __restrict__ firstWork,
                                                        uint64_t* __restrict__ statusBase)
 {
@@ -1811,7 +1814,7 @@ __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __rest
 		uint32_t nt = 0;
 		uint64_t ns = 0;
 		if (j < numJobs) {
-			nt = uint32_t(jobWorkItems(jobs[j].numTiles, jobs[j].numViews, splitTiles, groupShift));
+			nt = uint32_t(jobWorkItems(jobs[j].numTiles, jobs[j].numViews, splitTiles, groupShift, leaves));
 			ns = uint64_t(jobs[j].numViews) * jobs[j].numTiles;
 		}
 		sT[tid] = nt;
@@ -2195,6 +2198,7 @@ KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t n
 	uint64_t drawables = 0, tests = 0, tiles = 0;
 	uint32_t mostViews = 0;
 	for (uint32_t j = 0; j < numJobs; j++) {
+		if (jobs[j].numViews == 0) continue;  // no work items
 		// (a tile of few or no drawables costs what some 256 tests do)
 		const uint64_t n = std::max<uint64_t>(jobs[j].numDrawables, 256ull * jobs[j].numTiles);
 		drawables += n;
@@ -2250,7 +2254,7 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	for (uint32_t j = 0; j < numJobs; j++) {
 		const int rc = checkJob(hostJobs[j]);
 		if (rc != CADR_SUCCESS) return rc;
-		totalWork += jobWorkItems(hostJobs[j].numTiles, hostJobs[j].numViews, splitTiles, groupShift);
+		totalWork += jobWorkItems(hostJobs[j].numTiles, hostJobs[j].numViews, splitTiles, groupShift, leaves != nullptr);
 		statusNeed += uint64_t(hostJobs[j].numViews) * hostJobs[j].numTiles;
 		bytes += jobBytes(hostJobs[j], leaves != nullptr);
 	}
@@ -2265,7 +2269,7 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	if (totalWork == 0) CADR_RETURN_NO_LAUNCH(s);
 	if (numJobs > kInlineJobs) {
 		hipLaunchKernelGGL(cullSetupKernel, dim3(1), dim3(256), 0, s, jobs, numJobs, splitTiles,
-		                   groupShift, ws->firstWork, ws->statusBase);
+		                   groupShift, leaves != nullptr, ws->firstWork, ws->statusBase);
 		CADR_CHECK_HIP(hipGetLastError(), "cullSetupKernel launch");
 	}
 	if (grid > totalWork) grid = totalWork;

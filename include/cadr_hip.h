@@ -415,7 +415,8 @@ typedef struct cadrCullJob {
 	uint32_t numDrawables;
 	uint32_t numTiles;
 	uint32_t numStateSets;
-	uint32_t numViews;
+	uint32_t numViews;          /* 0: nothing is done for the job, except that
+	                             * cadrPropagateCullBatch writes its leaf level */
 	uint32_t commandStride;     /* commands per view, >= numDrawables          */
 	uint32_t numMeshes;         /* drawables with meshIndex >= numMeshes are never visible */
 } cadrCullJob;                  /* 80 B */

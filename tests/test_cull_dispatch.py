@@ -210,3 +210,51 @@ def test_jobs_without_views_many(gpu, block, items, flags):
     """The many-view kernel (shapes without a few-view one, or whole tiles for 70 views)."""
     print(f"{block}x{items} flags {flags}", flush=True)
     _run(NO_VIEWS, block, items, lambda b: b.run(), flags)
+
+
+@pytest.mark.parametrize("block,items", [(256, 2), (256, 4), (256, 8), (512, 4)])
+@pytest.mark.parametrize("specs", [
+    [(70_001, 1, 64, 0)],                                                                   # nothing but that
+    [(70_001, 1, 64, 0), (9000, 2, 64, 1), (70_001, 3, 8, 0), (5, 1, 9, 1), (30_001, 1, 64, 0)],  # one view at a time
+    [(70_001, 1, 64, 0), (9000, 2, 64, 2), (70_001, 3, 8, 0), (5, 1, 9, 1), (30_001, 1, 64, 0)],  # two
+    NO_VIEWS])                                                                              # four
+def test_jobs_without_views_few(gpu, block, items, specs):
+    print(f"{specs} {block}x{items}", flush=True)
+    _run(specs, block, items, lambda b: b.run())
+
+
+@pytest.mark.parametrize("views", [1, 2])
+def test_jobs_without_views_past_the_inline_offsets(gpu, views):
+    """More than 256 jobs, whose offsets a kernel of its own works out: every third without views."""
+    specs = [(1 + (j * 41) % 90 + (3000 if j % 50 == 3 else 0), 1 + j % 3, 8, 0 if j % 3 == 0 else 1 + j % views)
+             for j in range(260)]
+    _run(specs, 256, 2, lambda b: b.run())
+
+
+def test_jobs_without_views_fused(gpu):
+    """Fused launches write the leaf level of such a job too."""
+    jobs, leaves, worlds = [], [], []
+    for j, V in enumerate((0, 3, 0, 70, 0)):
+        scene = scenes.tree_scene((3 + j, 50, 21), seed=scenes.SEED_BASE + 990 + j, num_statesets=2)
+        w, spheres = oracle.propagate_scene(scene)
+        ds = cull.DeviceScene(scene)
+        descs = ds.level_descs()
+        for lv in descs[:-1]:
+            N.check(N.load().cadrPropagateTransforms(N.ptr(lv), None))
+        views = cull.make_views(scenes.random_cameras(17 + j, 20, 0, V, 150.0))
+        jobs.append((ds, views, cull.CullOutputs(V, ds.n, ds.K), spheres, scene))
+        leaves.append(descs[-1])
+        worlds.append(w[-1])
+    batch = cull.CullBatch(cull.make_config(256, 4), [j[:3] for j in jobs])
+    batch.set_leaves(np.concatenate(leaves))
+    batch.run_fused_batch()
+    synchronize()
+    batch.workspace.check()
+    _check(jobs, "fused batch with jobs without views")
+    for (ds, _, out, spheres, _), w in zip(jobs, worlds):
+        assert ds.world_matrices(-1).tobytes() == w.tobytes()
+        assert ds.download_spheres().tobytes() == spheres.tobytes()
+        out.close()
+    batch.close()
+    for ds, *_ in jobs:
+        ds.close()
