@@ -2212,11 +2212,17 @@ KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t n
 	return ke.few[numJobs > 1][mostViews <= 1 ? 0 : mostViews == 2 ? 1 : 2];
 }
 
+// Whether a leaf level's world matrices are written over its local ones.
+bool inPlace(const cadrTransformLevel& L)
+{
+	return L.localMatrices < L.worldMatrices + 64 * L.count && L.worldMatrices < L.localMatrices + 64 * L.count;
+}
+
 // One persistent launch of a batched kernel over numJobs jobs; leaves: the
-// fused form's leaf levels (device memory), else null.
+// fused form's leaf levels (device memory, with their host copy), else null.
 int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cadrCullConfig* config, uint64_t deviceJobs,
                 const cadrCullJob* hostJobs, uint32_t numJobs, cadrCullWorkspace* ws, cadrStream stream,
-                const cadrTransformLevel* leaves, const std::string& name)
+                const cadrTransformLevel* leaves, const cadrTransformLevel* hostLeaves, const std::string& name)
 {
 	CADR_REQUIRE(ws, name + ": workspace is NULL");
 	if (numJobs == 0) CADR_RETURN_NO_LAUNCH(stream);
@@ -2250,6 +2256,9 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 		groupShift = 2;
 	}
 	if (config->flags & CADR_CULL_WHOLE_TILES) splitTiles = 0;
+	// every item of a tile cut by views reads the tile's local matrices, so one
+	// whose world matrices take their place is left whole
+	if (leaves && std::any_of(hostLeaves, hostLeaves + numJobs, inPlace)) splitTiles = 0;
 	uint64_t totalWork = 0, statusNeed = 0, bytes = 0;
 	for (uint32_t j = 0; j < numJobs; j++) {
 		const int rc = checkJob(hostJobs[j]);
@@ -2299,7 +2308,8 @@ CADR_API int cadrCullBatch(const cadrCullConfig* config, uint64_t deviceJobs, co
 {
 	const KernelEntry* ke = findKernel(config);
 	CADR_REQUIRE(ke && ke->batch, "cadrCullBatch: unsupported blockSize/itemsPerThread");
-	return launchBatch(&KernelEntry::batch, *ke, config, deviceJobs, hostJobs, numJobs, ws, stream, nullptr, "cadrCullBatch");
+	return launchBatch(&KernelEntry::batch, *ke, config, deviceJobs, hostJobs, numJobs, ws, stream, nullptr, nullptr,
+	                   "cadrCullBatch");
 }
 
 CADR_API int cadrPropagateCullBatch(uint64_t deviceLeaves, const cadrTransformLevel* hostLeaves,
@@ -2317,7 +2327,7 @@ CADR_API int cadrPropagateCullBatch(uint64_t deviceLeaves, const cadrTransformLe
 		if (rc != CADR_SUCCESS) return rc;
 	}
 	return launchBatch(&KernelEntry::fusedBatch, *ke, config, deviceJobs, hostJobs, numJobs, ws, stream,
-	                   reinterpret_cast<const cadrTransformLevel*>(deviceLeaves), "cadrPropagateCullBatch");
+	                   reinterpret_cast<const cadrTransformLevel*>(deviceLeaves), hostLeaves, "cadrPropagateCullBatch");
 }
 
 CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, const cadrCullJob* hostJob,
@@ -2493,6 +2503,6 @@ CADR_API int cadrCullBatchNoAlloc(const cadrCullConfig* config, uint64_t deviceJ
 	w.device = dev;
 	w.ticksPerUs = sd.ticksPerUs;
 	w.waitLimit = kDefaultWaitLimitUs * sd.ticksPerUs;
-	return launchBatch(&KernelEntry::batch, *ke, config, deviceJobs, hostJobs, numJobs, &w, stream, nullptr,
+	return launchBatch(&KernelEntry::batch, *ke, config, deviceJobs, hostJobs, numJobs, &w, stream, nullptr, nullptr,
 	                   "cadrCullBatchNoAlloc");
 }

@@ -258,3 +258,38 @@ def test_jobs_without_views_fused(gpu):
     batch.close()
     for ds, *_ in jobs:
         ds.close()
+
+
+# leaf levels whose world matrices take the local ones' place: a tile's matrices are computed by one work item, whatever
+# the views and tiles (few tiles: cut by four views otherwise; more than 64 views: by 64)
+@pytest.mark.parametrize("block,items,fanouts,views", [(256, 4, (3, 50, 21), (5, 64, 33)), (256, 4, (2, 40, 30), (9, 2, 70)),
+                                                       (512, 4, (2, 30, 40), (64, 17)), (256, 8, (4, 40, 30), (64,)),
+                                                       (256, 4, (2, 300, 260), (130,))])
+def test_fused_batch_in_place(gpu, block, items, fanouts, views):
+    print(f"{fanouts} {block}x{items} views {views}", flush=True)
+    jobs, leaves, worlds = [], [], []
+    for j, V in enumerate(views):
+        scene = scenes.tree_scene((fanouts[0] + j,) + fanouts[1:], seed=scenes.SEED_BASE + 1010 + j, num_statesets=3)
+        w, spheres = oracle.propagate_scene(scene)
+        ds = cull.DeviceScene(scene)
+        descs = ds.level_descs(spheres=False)
+        for lv in descs[:-1]:
+            N.check(N.load().cadrPropagateTransforms(N.ptr(lv), None))
+        descs[-1]["worldMatrices"] = descs[-1]["localMatrices"]
+        cams = cull.make_views(scenes.random_cameras(23 + j, 20, 0, V, 150.0))
+        jobs.append((ds, cams, cull.CullOutputs(V, ds.n, ds.K), spheres, scene))
+        leaves.append(descs[-1])
+        worlds.append(w[-1])
+    batch = cull.CullBatch(cull.make_config(block, items), [j[:3] for j in jobs])
+    batch.set_leaves(np.concatenate(leaves))
+    batch.run_fused_batch()
+    synchronize()
+    batch.workspace.check()
+    _check(jobs, "fused batch in place")
+    for (ds, _, out, _, _), w in zip(jobs, worlds):
+        n, local = ds.levels[-1][0], ds.levels[-1][1]
+        assert local.download(np.float32, n * 16).reshape(n, 16).tobytes() == w.tobytes()
+        out.close()
+    batch.close()
+    for ds, *_ in jobs:
+        ds.close()
