@@ -2239,7 +2239,16 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	uint32_t perCU = config->workgroupsPerCU;
 	if (perCU == 0) perCU = ke.block >= 512 ? 2 : 4;
 	uint64_t grid = uint64_t(cu) * perCU;
-	const KernelFn few = leaves ? nullptr : fewKernelFor(ke, hostJobs, numJobs, config->flags);
+	auto workItems = [&](uint32_t splitTiles, uint32_t groupShift) {
+		uint64_t n = 0;
+		for (uint32_t j = 0; j < numJobs; j++)
+			n += jobWorkItems(hostJobs[j].numTiles, hostJobs[j].numViews, splitTiles, groupShift, leaves != nullptr);
+		return n;
+	};
+	constexpr uint64_t kMaxWork = 0xffffffffull;  // tickets are 32 bits
+	// every tile cut by four views: only what still has its tickets
+	const bool cut = workItems(0xffffffffu, 2) < kMaxWork;
+	const KernelFn few = leaves || !cut ? nullptr : fewKernelFor(ke, hostJobs, numJobs, config->flags);
 	uint32_t splitTiles = uint32_t(std::min<uint64_t>(grid, 1u << 20)), groupShift = 6;
 	if (few) {
 		fn = few;
@@ -2248,7 +2257,7 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 		if (config->workgroupsPerCU == 0)
 			if (const int resident = residentWorkgroups(few, ke.block)) grid = uint64_t(resident);
 	}
-	else if (leaves && tiles <= cu / 2) {
+	else if (leaves && cut && tiles <= cu / 2) {
 		// a fused launch of few tiles: four views a work item, each item
 		// computing the tile's leaves again (12 trees, 74 tiles, 1-16 views: 40.8
 		// -> 32.2 us; 171 tiles 39.8 -> 41.9, so not there)
@@ -2259,15 +2268,15 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	// every item of a tile cut by views reads the tile's local matrices, so one
 	// whose world matrices take their place is left whole
 	if (leaves && std::any_of(hostLeaves, hostLeaves + numJobs, inPlace)) splitTiles = 0;
-	uint64_t totalWork = 0, statusNeed = 0, bytes = 0;
+	const uint64_t totalWork = workItems(splitTiles, groupShift);
+	uint64_t statusNeed = 0, bytes = 0;
 	for (uint32_t j = 0; j < numJobs; j++) {
 		const int rc = checkJob(hostJobs[j]);
 		if (rc != CADR_SUCCESS) return rc;
-		totalWork += jobWorkItems(hostJobs[j].numTiles, hostJobs[j].numViews, splitTiles, groupShift, leaves != nullptr);
 		statusNeed += uint64_t(hostJobs[j].numViews) * hostJobs[j].numTiles;
 		bytes += jobBytes(hostJobs[j], leaves != nullptr);
 	}
-	CADR_REQUIRE(totalWork < 0xffffffffull, name + ": too many tiles in one launch");
+	CADR_REQUIRE(totalWork < kMaxWork, name + ": too many tiles in one launch");
 	CADR_REQUIRE(statusNeed <= ws->statusWords, name + ": workspace has too few status words");
 	int dev = 0;
 	CADR_CHECK_HIP(hipGetDevice(&dev), "hipGetDevice");

@@ -293,3 +293,18 @@ def test_fused_batch_in_place(gpu, block, items, fanouts, views):
     batch.close()
     for ds, *_ in jobs:
         ds.close()
+
+
+@pytest.mark.parametrize("tiles,views,error", [(0x40000000, 16, "too few status words"), (0xfffffff0, 8, "too few status words"),
+                                               (0xffffffff, 1, "too many tiles")])
+def test_work_item_limit_is_that_of_whole_tiles(gpu, tiles, views, error):
+    """Tickets are 32 bits.  Jobs whose tiles only have too many items when cut by four views are not refused for it: the
+    call goes on to the next check, the workspace's status words, which ends it here (nothing is launched)."""
+    import ctypes
+    jobs = np.zeros(1, N.JOB_DTYPE)
+    jobs[0] = (16, 16, 16, 16, 16, 16, 16, 100, tiles, 1, views, 100, 1)
+    ws = cull.Workspace(16, 1)
+    config = cull.make_config(256, 4)
+    with pytest.raises(N.CadrError, match=error):
+        N.check(N.load().cadrCullBatch(ctypes.byref(config), 16, N.ptr(jobs), 1, ws.handle, None))
+    ws.close()
