@@ -95,6 +95,7 @@ struct CullParams {
 	uint32_t groupShift;  // batched: log2 of the views of such a group
 	uint32_t flags;
 	uint64_t waitLimit;                 // steady-counter ticks a look-back may wait
+	uint64_t stuckAfter;                // and after which it leaves its item to the end of the launch (kStuck)
 	LeafParams leaf;                    // one-view fused kernel
 	const cadrTransformLevel* leaves;   // fused batched kernel: leaf level of each job
 };
@@ -399,7 +400,8 @@ __device__ __forceinline__ bool statusReady(uint64_t s, uint32_t epoch)
 
 // Look-back waits are bounded.  In a well-formed tile list every
 // predecessor holds an earlier ticket and is running or done, so a wait ends
-// within one tile's run time.  A caller-built list that names a predecessor
+// within one tile's run time, or is left to the end of the launch (kStuck
+// below).  A caller-built list that names a predecessor
 // no tile publishes (a non-FIRST tile whose chainIndex - 1 is missing) would
 // wait forever; instead, a wait that lasts waitLimit ticks of the steady
 // counter records the launch's epoch in the error word and gives up, and
@@ -411,6 +413,7 @@ struct WaitBound {
 	uint32_t* ctl;
 	uint64_t limit;
 	uint32_t epoch;
+	uint64_t stuck;  // ticks after which a wait returns kStuck
 };
 
 // Work tickets.  An atomic add on one address takes 11-12 ns on this GPU
@@ -427,8 +430,22 @@ struct WaitBound {
 // is always held by a running workgroup, whose predecessors are done, or is
 // the next ticket of its shard.  Workgroups are dispatched round-robin over
 // the XCDs, and (b / 8) spreads a shard over all of them, so each shard has
-// running workgroups as soon as 8 S of the launch's workgroups run; the
-// bounded waits below turn anything else into an error.
+// running workgroups as soon as 8 S of the launch's workgroups run.
+//
+// Where fewer do (a stream held to some compute units, other streams' kernels
+// on the rest), the ones that run would wait for tiles of shards that none of
+// them serves.  A wait that lasts kStuckUs therefore leaves its item: the
+// item's total is published, so no other item waits for it, the workgroup
+// ends and makes room or, a persistent one, goes on with tickets of whichever
+// shard is furthest behind, and the last workgroup of the launch finishes what
+// was left (finishLeft), when every total is published.  So a launch
+// progresses with any number of workgroups running.
+constexpr uint32_t kStuck = ~0u;         // for an exclusive prefix (30 bits)
+constexpr uint64_t kStuckUs = 1000;      // some hundred times the usual wait, and as long as most other launches
+constexpr uint64_t kStuckShare = 4;      // at most this part of the wait limit
+constexpr uint32_t kAgainShare = 16;     // the part of that which a workgroup waits once it was stuck
+constexpr uint32_t kLeftFlag = 1u << 31; // in a count of workgroups that left: one of them left an item
+
 struct Shard {
 	uint32_t shift;  // log2 of the launch's shards
 	uint32_t g;      // this workgroup's shard
@@ -462,20 +479,12 @@ __device__ __forceinline__ uint32_t askTicket(const CullParams& P, Shard s)
 	return __hip_atomic_fetch_add(globalMut<uint32_t>(a), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Called by one thread of each workgroup when it leaves: the last one of the
-// launch resets the tickets and retires the launch's epoch, so the next
-// launch on the workspace never sees this launch's status words as its own.
-// The workgroups of a shard count among themselves, then the shards.
-__device__ __forceinline__ void leaveLaunch(const CullParams& P, Shard s, uint32_t epoch)
+// Resets the tickets and retires the launch's epoch, so the next launch on the
+// workspace never sees this launch's status words as its own.
+__device__ __forceinline__ void endLaunch(const CullParams& P, Shard s, uint32_t epoch)
 {
-	const uint32_t S = 1u << s.shift, runs = gridDim.x >> (s.shift + 3u), rest = gridDim.x & (8u * S - 1u);
-	const uint32_t mine = 8u * runs + (rest > s.g * 8u ? min(rest - s.g * 8u, 8u) : 0u);
-	if (atomicAdd(&P.ctl[kCtlShard + 64u * s.g + 32u], 1u) != mine - 1u) return;
-	if (S > 1u) {
-		const uint32_t shards = min(S, (gridDim.x + 7u) / 8u);
-		if (atomicAdd(&P.ctl[kCtlDone], 1u) != shards - 1u) return;
-		atomicExch(&P.ctl[kCtlDone], 0u);
-	}
+	const uint32_t S = 1u << s.shift;
+	if (S > 1u) atomicExch(&P.ctl[kCtlDone], 0u);
 	for (uint32_t g = 0; g < S; g++) {
 		atomicExch(&P.ctl[kCtlShard + 64u * g], 0u);
 		atomicExch(&P.ctl[kCtlShard + 64u * g + 32u], 0u);
@@ -484,23 +493,92 @@ __device__ __forceinline__ void leaveLaunch(const CullParams& P, Shard s, uint32
 	atomicExch(&P.ctl[kCtlEpoch], e == 0u ? 1u : e);
 }
 
-// Called after an unready poll; start is 0 until the first such poll.
-__device__ __forceinline__ bool waitGiveUp(const WaitBound& B, uint64_t& start)
+// Called by one wave of each workgroup when it has taken its last ticket and
+// published its last status word.  The workgroups of a shard count among
+// themselves, then the shards.  The launch's last workgroup ends it; if items
+// were left on the way, it returns true instead, and the wave goes on to
+// finishLaunch when its own commands are stored.
+__device__ __forceinline__ bool signOff(const CullParams& P, Shard s, uint32_t epoch, uint32_t lane)
 {
-	if (__hip_atomic_load(&B.ctl[kCtlError], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == B.epoch) return true;
+	bool left = false;
+	if (lane == 0) {
+		const uint32_t S = 1u << s.shift, runs = gridDim.x >> (s.shift + 3u), rest = gridDim.x & (8u * S - 1u);
+		const uint32_t mine = 8u * runs + (rest > s.g * 8u ? min(rest - s.g * 8u, 8u) : 0u);
+		uint32_t d = atomicAdd(&P.ctl[kCtlShard + 64u * s.g + 32u], 1u);
+		bool last = (d & ~kLeftFlag) == mine - 1u;
+		if (last && S > 1u) {
+			const uint32_t shards = min(S, (gridDim.x + 7u) / 8u);
+			if ((d & kLeftFlag) != 0u) (void)atomicOr(&P.ctl[kCtlDone], kLeftFlag);
+			d = atomicAdd(&P.ctl[kCtlDone], 1u);
+			last = (d & ~kLeftFlag) == shards - 1u;
+		}
+		left = last && (d & kLeftFlag) != 0u;
+		if (last && !left) endLaunch(P, s, epoch);
+	}
+	return __ballot(left) != 0ull;
+}
+
+// Where a workgroup's tickets come from (kept by its wave 0).
+struct Tickets {
+	Shard s;
+	bool roam;  // it was stuck: from the shard furthest behind
+
+	__device__ __forceinline__ explicit Tickets(Shard home) : s(home), roam(false) {}
+
+	// Before a ticket is asked for: the shard whose next ticket is the smallest item.
+	__device__ __forceinline__ void choose(const CullParams& P, uint32_t lane)
+	{
+		if (!roam) return;
+		uint64_t next = ~0ull;  // (item, shard)
+		if (lane < (1u << s.shift)) {
+			const uint32_t r = __hip_atomic_load(&P.ctl[kCtlShard + 64u * lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			next = (uint64_t(itemOfTicket(Shard{s.shift, lane}, r)) << 32) | lane;
+		}
+#pragma unroll
+		for (int off = 8; off >= 1; off >>= 1) {
+			const uint64_t o = __shfl_xor(next, off);
+			next = o < next ? o : next;
+		}
+		s.g = uniform(uint32_t(next));
+	}
+};
+
+// Called by a wave whose item is left (its total is published): marks the
+// launch before the workgroup can sign off.
+__device__ __forceinline__ void leaveItem(const CullParams& P, Shard home, uint32_t lane)
+{
+	if (lane == 0) (void)atomicOr(&P.ctl[kCtlShard + 64u * home.g + 32u], kLeftFlag);
+	__threadfence();
+}
+
+// ANY_STUCK: whether the kernel leaves items; again: the workgroup was stuck before.
+template <bool ANY_STUCK>
+__device__ __forceinline__ WaitBound waitBound(const CullParams& P, uint32_t epoch, bool again = false)
+{
+	return WaitBound{P.ctl, P.waitLimit, epoch, !ANY_STUCK ? ~0ull : again ? P.stuckAfter / kAgainShare : P.stuckAfter};
+}
+
+constexpr uint32_t kPollAgain = 0, kGiveUp = 1, kWaitLater = 2;
+
+// Called after an unready poll; start is 0 until the first such poll.
+__device__ __forceinline__ uint32_t waitStep(const WaitBound& B, uint64_t& start)
+{
+	if (__hip_atomic_load(&B.ctl[kCtlError], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == B.epoch) return kGiveUp;
 	const uint64_t now = uint64_t(wall_clock64());
 	if (start == 0) {
 		start = now == 0 ? 1 : now;
-		return false;
+		return kPollAgain;
 	}
-	if (now - start <= B.limit) return false;
+	if (now - start > B.stuck) return kWaitLater;
+	if (now - start <= B.limit) return kPollAgain;
 	__hip_atomic_store(&B.ctl[kCtlError], B.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-	return true;
+	return kGiveUp;
 }
 
 // Exclusive prefix of chain position c, one chain per lane: walk back over the
 // predecessors adding aggregates until an inclusive prefix is found; position
-// 0 ends the walk in any case, and a wait bounded as above ends it early.
+// 0 ends the walk in any case, and a wait bounded as above ends it early
+// (kStuck if it is left for later).
 __device__ uint32_t lookBackSerial(const uint64_t* chain, uint32_t c, const WaitBound& B)
 {
 	uint32_t excl = 0;
@@ -512,7 +590,7 @@ __device__ uint32_t lookBackSerial(const uint64_t* chain, uint32_t c, const Wait
 		for (;;) {
 			s = readStatus(chain + p);
 			if (statusReady(s, B.epoch)) break;
-			if (waitGiveUp(B, start)) return excl;
+			if (const uint32_t step = waitStep(B, start)) return step == kWaitLater ? kStuck : excl;
 			__builtin_amdgcn_s_sleep(1);
 		}
 		excl += uint32_t(s) & kValueMask;
@@ -539,7 +617,7 @@ __device__ uint32_t lookBackWave(const uint64_t* chain, uint32_t c, const WaitBo
 		const uint32_t f = pmask ? uint32_t(__builtin_ctzll(pmask)) : 64u;
 		const uint64_t need = f >= 63u ? ~0ull : ((2ull << f) - 1ull);
 		if (nmask & need) {
-			if (uniform(uint32_t(waitGiveUp(B, start)))) return excl;
+			if (const uint32_t step = uniform(waitStep(B, start))) return step == kWaitLater ? kStuck : excl;
 			__builtin_amdgcn_s_sleep(1);
 			continue;
 		}
@@ -582,7 +660,12 @@ __device__ uint32_t lookBackGroups(const uint64_t* chain, uint32_t c, const Wait
 			p = f < W ? 0 : p - int64_t(W);
 		}
 		if (__ballot(wait) != 0ull) {
-			if (uniform(uint32_t(waitGiveUp(B, start)))) return excl;
+			const uint32_t step = uniform(waitStep(B, start));
+			if (step == kGiveUp) return excl;
+			if (step == kWaitLater && wait) {  // the other chains go on
+				excl = kStuck;
+				p = 0;
+			}
 			__builtin_amdgcn_s_sleep(1);
 		}
 	}
@@ -801,6 +884,161 @@ __device__ __forceinline__ void propagateTileItems(const LeafParams& Lf, const c
 	}
 }
 
+// ------------------------------------------------------- the end of a launch
+
+// Makes an address one that the compiler takes for a lane's own, not known
+// before `after` is.
+__device__ __forceinline__ uint64_t perLane(uint64_t address, float after = 0.f)
+{
+	asm volatile("" : "+v"(address) : "v"(after));
+	return address;
+}
+
+// One tile in one view from its status word on, by one wave and without the
+// mesh table's LDS copy: what a workgroup left because its look-back was stuck.
+// job, tile, view, leaf: addresses.  This code almost never runs, and scalar
+// registers for its descriptors would cost the kernels a wave per SIMD: it
+// reads them through perLane, the view row by row.
+template <int TILE, bool FUSED>
+__device__ __forceinline__ void finishTile(const CullParams& P, uint64_t job, uint64_t tile, uint64_t view, uint32_t v,
+                                           const LeafParams& Lf, uint64_t* chain, uint32_t pos, uint32_t epoch,
+                                           uint32_t lane)
+{
+	const uint32_t excl = lookBackWave(chain, pos, waitBound<false>(P, epoch), lane);
+	tile = perLane(tile);
+	// loadTile's clamps
+	const uint32_t start = globalPtr<uint32_t>(tile)[0], drawables = globalPtr<uint32_t>(perLane(job))[14];
+	const uint32_t count =
+	    uniform(start >= drawables ? 0u : min(min(globalPtr<uint32_t>(tile)[1], drawables - start), uint32_t(TILE)));
+	uint32_t at = globalPtr<uint32_t>(tile)[2] + excl, total = 0;
+#pragma unroll 1
+	for (uint32_t e = 0; e < count; e += 64u) {
+		uint64_t J = perLane(job);
+		const uint32_t i = start + min(e + lane, count - 1u);
+		const uint32_t m = globalPtr<uint32_t>(globalPtr<uint64_t>(J)[1])[i];
+		const bool live = e + lane < count && m < globalPtr<uint32_t>(J)[19];
+		float4 s = make_float4(0.f, 0.f, 0.f, -__builtin_inff());
+		if constexpr (FUSED) {
+			float4 L[4], W[4];
+#pragma unroll
+			for (int c = 0; c < 4; c++) W[c] = L[c] = loadF4(globalPtr<float4>(Lf.local) + (4 * uint64_t(i) + c));
+			const uint32_t p = Lf.parentCount > 0 ? globalPtr<uint32_t>(Lf.parentIndex)[i] : ~0u;
+			if (p < Lf.parentCount) {
+				float4 A[4];
+#pragma unroll
+				for (int c = 0; c < 4; c++) A[c] = loadF4(globalPtr<float4>(Lf.parentWorld) + (4 * uint64_t(p) + c));
+				mat4Mul(A, L, W);
+			}
+			if (live) s = sphereTransform(W, loadF4(globalPtr<float4>(globalPtr<uint64_t>(J)[2]) + 4 * uint64_t(m)));
+		} else {
+			s = loadF4(globalPtr<float4>(globalPtr<uint64_t>(J)[0]) + i);
+		}
+		// the test of sphereVisible
+		const gptr<float> r2 = globalPtr<float>(perLane(view, s.w));
+		const float vz = viewCoord(make_float4(r2[8], r2[9], r2[10], r2[11]), s);
+		bool vis = live & (vz + s.w >= r2[12]) & (vz - s.w <= r2[13]);
+		const gptr<float> r0 = globalPtr<float>(perLane(view, vz));
+		const float vx = viewCoord(make_float4(r0[0], r0[1], r0[2], r0[3]), s);
+		vis &= fabsf(vx) * r0[14] - vz * r0[15] <= s.w;
+		const gptr<float> r1 = globalPtr<float>(perLane(view, vx));
+		const float vy = viewCoord(make_float4(r1[4], r1[5], r1[6], r1[7]), s);
+		vis &= fabsf(vy) * r1[16] - vz * r1[17] <= s.w;
+		const uint64_t mask = __ballot(vis);
+		const uint32_t slot = at + maskRank(mask);
+		J = perLane(job, vy);
+		if (vis && slot < globalPtr<uint32_t>(J)[18]) {
+			ViewC V{};
+			const gptr<float> lod = globalPtr<float>(perLane(view, vy)) + 18;
+			V.lodScale = lod[0];
+			V.th0 = lod[1];
+			V.th1 = lod[2];
+			V.th2 = lod[3];
+			uint32_t n, first, vofs;
+			meshCommand<false>(MeshTable{nullptr, globalPtr<cadrMesh>(globalPtr<uint64_t>(J)[2]), false}, m, s.w, vz, V, n,
+			                   first, vofs);
+			const gmut<uint32_t> o = globalMut<uint32_t>(globalPtr<uint64_t>(J)[5]) +
+			                         (uint64_t(v) * globalPtr<uint32_t>(J)[18] + slot) * 5ull;
+			o[0] = n;
+			o[1] = 1u;
+			o[2] = first;
+			o[3] = vofs;
+			o[4] = i;
+		}
+		at += uint32_t(__builtin_popcountll(mask));
+		total += uint32_t(__builtin_popcountll(mask));
+	}
+	if (lane == 0) {
+		publish(chain + pos, packStatus(epoch, kStatePrefix, excl + total));
+		const uint64_t J = perLane(job);
+		const uint32_t flags = globalPtr<uint32_t>(tile)[3], k = flags & CADR_TILE_STATESET_MASK, K = globalPtr<uint32_t>(J)[16];
+		if ((flags & CADR_TILE_LAST) != 0u && k < K)
+			globalMut<uint32_t>(globalPtr<uint64_t>(J)[6])[uint64_t(v) * K + k] = excl + total;
+	}
+}
+
+// The items that the launch's workgroups left: every tile and view whose
+// status word holds a total and no inclusive prefix.  Called by one wave of
+// the last workgroup.  (A word whose prefix is still on its way here is
+// finished again, with the same outputs.)
+template <int TILE, bool FUSED>
+__device__ __forceinline__ void finishLeft(const CullParams& P, uint32_t epoch, uint32_t lane)
+{
+	uint64_t* chain = P.status;
+#pragma unroll 1
+	for (uint32_t j = 0; j < P.numJobs; j++) {
+		const uint64_t job = addr(P.jobs) + uint64_t(j) * sizeof(cadrCullJob);
+		const uint32_t numTiles = uniform(globalPtr<uint32_t>(perLane(job))[15]);
+		const uint32_t numViews = uniform(globalPtr<uint32_t>(perLane(job))[17]);
+		LeafParams Lf{};
+		if constexpr (FUSED) Lf = P.leaves ? loadLeaf(P.leaves, j) : P.leaf;
+#pragma unroll 1
+		for (uint32_t v = 0; v < numViews; v++, chain += numTiles) {
+#pragma unroll 1
+			for (uint32_t e = 0; e < numTiles; e += 64u) {
+				const uint64_t tiles = globalPtr<uint64_t>(perLane(job))[3];
+				uint64_t s = 0;
+				uint32_t c = 0;
+				if (e + lane < numTiles) {
+					c = globalPtr<uint32_t>(tiles)[8 * uint64_t(e + lane) + 4];
+					if (c >= numTiles) c = e + lane;  // as loadTile
+					s = readStatus(chain + c);
+				}
+				uint64_t left = __ballot(uint32_t(s >> 32) == epoch && (uint32_t(s) >> 30) == kStateAggregate);
+#pragma unroll 1
+				for (; left != 0ull; left &= left - 1ull) {
+					const uint32_t l = uniform(uint32_t(__builtin_ctzll(left)));
+					finishTile<TILE, FUSED>(P, job, tiles + sizeof(cadrCullTile) * uint64_t(e + l),
+					                        globalPtr<uint64_t>(perLane(job))[4] + uint64_t(v) * sizeof(cadrView), v, Lf, chain,
+					                        uint32_t(__builtin_amdgcn_readlane(c, l)), epoch, lane);
+				}
+			}
+		}
+	}
+}
+
+// After signOff, by the wave for which it returned true.  The kernel's
+// arguments (one CullParams) are loaded anew, so that none is held for this.
+template <int TILE, bool FUSED>
+__device__ __forceinline__ void finishLaunch(Shard s, uint32_t epoch, uint32_t lane)
+{
+	uint64_t a = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
+	asm volatile("" : "+s"(a));
+	const cptr<CullParams> K = constPtr<CullParams>(a);
+	CullParams P{};
+	P.jobs = K->jobs;
+	P.status = K->status;
+	P.ctl = K->ctl;
+	P.numJobs = K->numJobs;
+	P.waitLimit = K->waitLimit;
+	if constexpr (FUSED) {
+		P.leaves = K->leaves;
+		P.leaf = LeafParams{K->leaf.local, K->leaf.parentIndex, K->leaf.parentWorld, K->leaf.world, K->leaf.spheres,
+		                    K->leaf.parentCount};
+	}
+	finishLeft<TILE, FUSED>(P, epoch, lane);
+	if (lane == 0) endLaunch(P, s, epoch);
+}
+
 // ---------------------------------------------------------------- one view
 
 // A wave's visible items as a compact list in its own LDS, in drawable order:
@@ -889,9 +1127,10 @@ __device__ __forceinline__ void storeListed(const uint32_t* run, uint32_t n, uin
 
 // Look-back of a tile by wave 0, from the waves' counts; the exclusive prefix
 // goes to *sExclP and a StateSet's last tile writes its count.
-template <int WAVES>
+template <int WAVES, int TILE>
 __device__ __forceinline__ void tileOffset(const CullParams& P, const cadrCullJob& J, const TileDesc& T, uint32_t epoch,
-                                           const uint32_t* sCnt, uint32_t* sExclP, uint32_t lane)
+                                           Shard home, Tickets& tickets, const uint32_t* sCnt, uint32_t* sExclP,
+                                           uint32_t lane)
 {
 	uint32_t total = 0;
 #pragma unroll
@@ -902,7 +1141,13 @@ __device__ __forceinline__ void tileOffset(const CullParams& P, const cadrCullJo
 		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
 	} else {
 		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
-		excl = lookBackWave(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch}, lane);
+		excl = lookBackWave(chain, T.chain, waitBound<!oneShard(TILE)>(P, epoch, tickets.roam), lane);
+		if (excl == kStuck) {
+			leaveItem(P, home, lane);
+			tickets.roam = true;
+			*sExclP = kStuck;
+			return;
+		}
 		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
 	}
 	if (lane == 0) {
@@ -911,8 +1156,9 @@ __device__ __forceinline__ void tileOffset(const CullParams& P, const cadrCullJo
 	}
 }
 
+// Returns signOff's result in the wave that called it, else false.
 template <int BLOCK, int ITEMS, bool LDS, bool FUSED>
-__device__ __forceinline__ void cullViewTile(const CullParams& P, const cadrCullJob& J, uint32_t t, uint32_t epoch,
+__device__ __forceinline__ bool cullViewTile(const CullParams& P, const cadrCullJob& J, uint32_t t, uint32_t epoch,
                                              Shard shard, const MeshTable& meshes, uint32_t* sCnt, uint32_t* sExclP,
                                              float4* sMat, uint32_t* run, uint32_t lane, uint32_t wave)
 {
@@ -935,17 +1181,20 @@ __device__ __forceinline__ void cullViewTile(const CullParams& P, const cadrCull
 	const uint32_t n = listVisible<ITEMS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
 	if (lane == 0) sCnt[wave] = n;
 	__syncthreads();
-	if (wave == 0) tileOffset<WAVES>(P, J, T, epoch, sCnt, sExclP, lane);
+	Tickets tickets(shard);
+	if (wave == 0) tileOffset<WAVES, BLOCK * ITEMS>(P, J, T, epoch, shard, tickets, sCnt, sExclP, lane);
 	__syncthreads();
 	// the workgroup is done with the launch's tickets and status words: the
 	// last wave signs off while the others store, so that no wave waits for
 	// its stores behind the atomics
-	if (wave == WAVES - 1 && lane == 0) leaveLaunch(P, shard, epoch);
+	bool left = false;
+	if (wave == WAVES - 1) left = signOff(P, shard, epoch, lane);
 
 	uint32_t pos = T.segBase + *sExclP;
 	for (uint32_t q = 0; q < wave; q++) pos += sCnt[q];
-	storeListed<LDS>(run, n, uniform(pos), T.start + wave * WAVE_ITEMS, meshes, J.numMeshes, meshIndex,
-	                 globalMut<uint32_t>(J.commands), J.commandStride, lane);
+	storeListed<LDS>(run, *sExclP == kStuck ? 0u : n, uniform(pos), T.start + wave * WAVE_ITEMS, meshes, J.numMeshes,
+	                 meshIndex, globalMut<uint32_t>(J.commands), J.commandStride, lane);
+	return left;
 }
 
 template <int BLOCK, int ITEMS, bool FUSED>
@@ -973,16 +1222,19 @@ __device__ __forceinline__ void cullViewBody(const CullParams& P)
 	__syncthreads();
 	const uint32_t t = uniform(sTicket);
 	const MeshTable meshes{sMeshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
+	bool left = false;
 	if (t >= P.totalWork) {
-		if (tid == 0) leaveLaunch(P, shard, epoch);
-		return;
+		if (wave == 0) left = signOff(P, shard, epoch, lane);
+	} else {
+		float4* mat = sMat[wave];
+		uint32_t* run = reinterpret_cast<uint32_t*>(mat);
+		if (ldsMeshes)
+			left = cullViewTile<BLOCK, ITEMS, true, FUSED>(P, J, t, epoch, shard, meshes, sCnt, &sExcl, mat, run, lane, wave);
+		else
+			left = cullViewTile<BLOCK, ITEMS, false, FUSED>(P, J, t, epoch, shard, meshes, sCnt, &sExcl, mat, run, lane, wave);
 	}
-	float4* mat = sMat[wave];
-	uint32_t* run = reinterpret_cast<uint32_t*>(mat);
-	if (ldsMeshes)
-		cullViewTile<BLOCK, ITEMS, true, FUSED>(P, J, t, epoch, shard, meshes, sCnt, &sExcl, mat, run, lane, wave);
-	else
-		cullViewTile<BLOCK, ITEMS, false, FUSED>(P, J, t, epoch, shard, meshes, sCnt, &sExcl, mat, run, lane, wave);
+	if constexpr (!oneShard(BLOCK * ITEMS))
+		if (left) finishLaunch<BLOCK * ITEMS, FUSED>(shard, epoch, lane);
 }
 
 template <int BLOCK, int ITEMS>
@@ -1002,7 +1254,7 @@ __global__ __launch_bounds__(BLOCK) void cullViewKernel(CullParams P)
 // tiles than that; a view of fewer tiles takes one tile per workgroup
 // (cullViewKernel), which saves the loop's extra ticket and barrier.
 template <int BLOCK, int ITEMS, bool LDS>
-__device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCullJob& J, uint32_t t, uint32_t epoch,
+__device__ __forceinline__ bool cullViewTiles(const CullParams& P, const cadrCullJob& J, uint32_t t, uint32_t epoch,
                                               Shard shard, const MeshTable& meshes, uint32_t* sTicket,
                                               uint32_t (*sCnt)[BLOCK / 64], uint32_t* sExcl, uint32_t* run,
                                               uint32_t tid, uint32_t lane, uint32_t wave)
@@ -1016,10 +1268,13 @@ __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCul
 	float4 sp[ITEMS];
 	uint32_t mi[ITEMS];
 	loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
+	Tickets tickets(shard);
 	for (uint32_t b = 0;; b ^= 1u) {
 		const uint32_t n = listVisible<ITEMS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
 		if (lane == 0) sCnt[b][wave] = n;
-		if (tid == 0) *sTicket = itemOfTicket(shard, askTicket(P, shard));
+		if constexpr (!oneShard(BLOCK * ITEMS))
+			if (wave == 0) tickets.choose(P, lane);
+		if (tid == 0) *sTicket = itemOfTicket(tickets.s, askTicket(P, tickets.s));
 		__syncthreads();
 
 		// the next tile's loads, in flight through this tile's look-back and stores
@@ -1030,16 +1285,17 @@ __device__ __forceinline__ void cullViewTiles(const CullParams& P, const cadrCul
 			T = loadTile(J, tn, BLOCK * ITEMS);
 			loadTileItems<ITEMS>(spheres, meshIndex, T, wave * WAVE_ITEMS + lane, sp, mi);
 		}
-		if (wave == 0) tileOffset<WAVES>(P, J, Tc, epoch, sCnt[b], &sExcl[b], lane);
+		if (wave == 0) tileOffset<WAVES, BLOCK * ITEMS>(P, J, Tc, epoch, shard, tickets, sCnt[b], &sExcl[b], lane);
 		__syncthreads();
 
-		if (!more && wave == WAVES - 1 && lane == 0) leaveLaunch(P, shard, epoch);  // as in cullViewTile
+		bool left = false;
+		if (!more && wave == WAVES - 1) left = signOff(P, shard, epoch, lane);  // as in cullViewTile
 
 		uint32_t pos = Tc.segBase + sExcl[b];
 		for (uint32_t q = 0; q < wave; q++) pos += sCnt[b][q];
-		storeListed<LDS>(run, n, uniform(pos), Tc.start + wave * WAVE_ITEMS, meshes, J.numMeshes, meshIndex, out,
-		                 J.commandStride, lane);
-		if (!more) break;
+		storeListed<LDS>(run, sExcl[b] == kStuck ? 0u : n, uniform(pos), Tc.start + wave * WAVE_ITEMS, meshes, J.numMeshes,
+		                 meshIndex, out, J.commandStride, lane);
+		if (!more) return left;
 	}
 }
 
@@ -1068,16 +1324,18 @@ __global__ __launch_bounds__(BLOCK) void cullViewLoopKernel(CullParams P)
 	const uint32_t t = uniform(sTicket);
 	__syncthreads();  // every wave has read the first ticket before the loop rewrites it
 	const MeshTable meshes{sMeshes, globalPtr<cadrMesh>(J.meshes), ldsMeshes};
+	bool left = false;
 	if (t >= P.totalWork) {
-		if (tid == 0) leaveLaunch(P, shard, epoch);
-		return;
+		if (wave == 0) left = signOff(P, shard, epoch, lane);
+	} else if (ldsMeshes) {
+		left = cullViewTiles<BLOCK, ITEMS, true>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, sRun[wave], tid, lane,
+		                                        wave);
+	} else {
+		left = cullViewTiles<BLOCK, ITEMS, false>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, sRun[wave], tid, lane,
+		                                         wave);
 	}
-	if (ldsMeshes)
-		cullViewTiles<BLOCK, ITEMS, true>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, sRun[wave], tid, lane,
-		                                  wave);
-	else
-		cullViewTiles<BLOCK, ITEMS, false>(P, J, t, epoch, shard, meshes, &sTicket, sCnt, sExcl, sRun[wave], tid, lane,
-		                                   wave);
+	if constexpr (!oneShard(BLOCK * ITEMS))
+		if (left) finishLaunch<BLOCK * ITEMS, false>(shard, epoch, lane);
 }
 
 // The fused kernel is latency-bound (a chain of dependent loads per item), so
@@ -1304,21 +1562,25 @@ __device__ __forceinline__ void fewPublish(const FewItem& f, uint32_t total, uin
 // Wave 0: an item's exclusive prefixes, published as inclusive ones, to excl[].
 template <int CH>
 __device__ __forceinline__ void fewLookBack(const CullParams& P, const FewItem& f, uint32_t total, uint32_t epoch,
-                                            uint32_t* excl, uint32_t lane)
+                                            Shard home, Tickets& tickets, uint32_t* excl, uint32_t lane)
 {
 	const FewChain<CH> c(f, lane);
 	uint32_t e = 0;
 	if (!f.T.first) {
-		const WaitBound B{P.ctl, P.waitLimit, epoch};
+		const WaitBound B = waitBound<true>(P, epoch, tickets.roam);
 		if constexpr (CH == 1)
 			e = lookBackWave(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane);
 		else
 			e = lookBackGroups<64 / CH>(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane);
-		if (c.lead) publish(c.chain, packStatus(epoch, kStatePrefix, e + total));
+		if (__ballot(c.on && e == kStuck) != 0ull) {
+			leaveItem(P, home, lane);
+			tickets.roam = true;
+		}
+		if (c.lead && e != kStuck) publish(c.chain, packStatus(epoch, kStatePrefix, e + total));
 	}
 	if (c.lead) {
 		excl[lane / (64 / CH)] = e;
-		if (f.T.last && f.T.k < f.J.numStateSets)
+		if (e != kStuck && f.T.last && f.T.k < f.J.numStateSets)
 			globalMut<uint32_t>(f.J.counts)[uint64_t(c.view) * f.J.numStateSets + f.T.k] = e + total;
 	}
 }
@@ -1333,7 +1595,7 @@ __device__ __forceinline__ void fewStore(const FewItem& f, const MeshTable& stag
 	const MeshTable meshes{staged.lds, globalPtr<cadrMesh>(f.J.meshes), LDS};
 #pragma unroll
 	for (int c = 0; c < CH; c++) {
-		if (n[c] == 0) continue;
+		if (n[c] == 0 || excl[c] == kStuck) continue;
 		const uint32_t pos = uniform(f.T.segBase + excl[c] + off[c]);
 		storeListed<LDS>(run[c], n[c], pos, f.T.start + wave * N, meshes, f.J.numMeshes, globalPtr<uint32_t>(f.J.meshIndex),
 		                 globalMut<uint32_t>(f.J.commands) + uint64_t(f.viewBegin + c) * f.J.commandStride * 5ull,
@@ -1341,8 +1603,9 @@ __device__ __forceinline__ void fewStore(const FewItem& f, const MeshTable& stag
 	}
 }
 
+// Returns signOff's result in the wave that called it, else false.
 template <int BLOCK, int ITEMS, int CH, bool DEFER, bool JOBS, bool LDS>
-__device__ __forceinline__ void cullFewItems(const CullParams& P, FewShared<BLOCK, ITEMS, CH, DEFER>& sh,
+__device__ __forceinline__ bool cullFewItems(const CullParams& P, FewShared<BLOCK, ITEMS, CH, DEFER>& sh,
                                              const cadrCullJob& only, uint32_t t, Shard shard, uint32_t epoch, uint32_t tid,
                                              uint32_t lane, uint32_t wave)
 {
@@ -1355,6 +1618,7 @@ __device__ __forceinline__ void cullFewItems(const CullParams& P, FewShared<BLOC
 	loadTileItems<ITEMS>(globalPtr<float4>(cur.J.spheres), globalPtr<uint32_t>(cur.J.meshIndex), cur.T,
 	                     wave * WAVE_ITEMS + lane, sp, mi);
 	bool pending = false;
+	Tickets tickets(shard);
 	for (uint32_t b = 0;; b ^= 1u) {
 		asm volatile("" : "+v"(lane));  // nothing derived from it stays in registers across tiles
 		uint32_t n[CH], off[CH];
@@ -1366,7 +1630,8 @@ __device__ __forceinline__ void cullFewItems(const CullParams& P, FewShared<BLOC
 				                          wave * WAVE_ITEMS, lane, sh.run[DEFER ? b : 0][wave][c]);
 			if (lane == 0) sh.cnt[b][c][wave] = n[c];
 		}
-		if (DEFER && tid == 0) sh.ticket[b] = itemOfTicket(shard, askTicket(P, shard));
+		if (DEFER && wave == 0) tickets.choose(P, lane);
+		if (DEFER && tid == 0) sh.ticket[b] = itemOfTicket(tickets.s, askTicket(P, tickets.s));
 		__syncthreads();
 		FewItem next;
 		bool more = false;
@@ -1392,20 +1657,21 @@ __device__ __forceinline__ void cullFewItems(const CullParams& P, FewShared<BLOC
 			for (int q = 0; q < WAVES; q++) total += sh.cnt[b][lane / (64 / CH)][q];
 			fewPublish<CH>(cur, total, epoch, lane);
 			if constexpr (DEFER) {
-				if (pending) fewLookBack<CH>(P, prev, totalPrev, epoch, sh.excl[b], lane);
+				if (pending) fewLookBack<CH>(P, prev, totalPrev, epoch, shard, tickets, sh.excl[b], lane);
 			} else {
-				fewLookBack<CH>(P, cur, total, epoch, sh.excl[b], lane);
+				fewLookBack<CH>(P, cur, total, epoch, shard, tickets, sh.excl[b], lane);
 			}
 		}
 		__syncthreads();
 		if constexpr (DEFER) {
 			if (pending) fewStore<CH, LDS, WAVE_ITEMS>(prev, staged, sh.run[b ^ 1u][wave], nPrev, offPrev, sh.excl[b], wave, lane);
 			if (!more) {
-				if (wave == 0) fewLookBack<CH>(P, cur, total, epoch, sh.excl[b ^ 1u], lane);
+				if (wave == 0) fewLookBack<CH>(P, cur, total, epoch, shard, tickets, sh.excl[b ^ 1u], lane);
 				__syncthreads();
-				if (wave == WAVES - 1 && lane == 0) leaveLaunch(P, shard, epoch);
+				bool left = false;
+				if (wave == WAVES - 1) left = signOff(P, shard, epoch, lane);
 				fewStore<CH, LDS, WAVE_ITEMS>(cur, staged, sh.run[b][wave], n, off, sh.excl[b ^ 1u], wave, lane);
-				return;
+				return left;
 			}
 			prev = cur;
 			totalPrev = total;
@@ -1418,13 +1684,14 @@ __device__ __forceinline__ void cullFewItems(const CullParams& P, FewShared<BLOC
 			cur = next;
 		} else {
 			fewStore<CH, LDS, WAVE_ITEMS>(cur, staged, sh.run[0][wave], n, off, sh.excl[b], wave, lane);
-			if (tid == 0) sh.ticket[b] = itemOfTicket(shard, askTicket(P, shard));
+			if (wave == 0) tickets.choose(P, lane);
+			if (tid == 0) sh.ticket[b] = itemOfTicket(tickets.s, askTicket(P, tickets.s));
 			__syncthreads();
 			takeNext(cur);
 			if (!more) break;
 		}
 	}
-	if (tid == 0) leaveLaunch(P, shard, epoch);
+	return wave == 0 && signOff(P, shard, epoch, lane);
 }
 
 template <int BLOCK, int ITEMS, int CH, bool DEFER, bool JOBS>
@@ -1449,14 +1716,15 @@ __global__ __launch_bounds__(BLOCK) void cullFewKernel(CullParams P)
 	if (tid == 0) sh.ticket[1] = itemOfTicket(shard, ticket);
 	__syncthreads();
 	const uint32_t t = uniform(sh.ticket[1]);
+	bool left = false;
 	if (t >= P.totalWork) {
-		if (tid == 0) leaveLaunch(P, shard, epoch);
-		return;
+		if (wave == 0) left = signOff(P, shard, epoch, lane);
+	} else if (!JOBS && ldsMeshes) {
+		left = cullFewItems<BLOCK, ITEMS, CH, DEFER, JOBS, true>(P, sh, only, t, shard, epoch, tid, lane, wave);
+	} else {
+		left = cullFewItems<BLOCK, ITEMS, CH, DEFER, JOBS, false>(P, sh, only, t, shard, epoch, tid, lane, wave);
 	}
-	if (!JOBS && ldsMeshes)
-		cullFewItems<BLOCK, ITEMS, CH, DEFER, JOBS, true>(P, sh, only, t, shard, epoch, tid, lane, wave);
-	else
-		cullFewItems<BLOCK, ITEMS, CH, DEFER, JOBS, false>(P, sh, only, t, shard, epoch, tid, lane, wave);
+	if (left) finishLaunch<BLOCK * ITEMS, false>(shard, epoch, lane);
 }
 
 template <int BLOCK, int ITEMS>
@@ -1475,8 +1743,10 @@ struct CullShared {
 // COOP (fused form only): parent matrices read whole, 16 per instruction
 // (issueParentLoads), for leaves whose parents are scattered; it holds more
 // registers, so it is chosen per shape, like WPE, the waves per SIMD asked of
-// the register allocator (see the kernel table).
-template <int BLOCK, int ITEMS, bool FUSED, bool COOP = false, int WPE = 1>
+// the register allocator (see the kernel table; 256 x 8 takes one register
+// more than 3 waves leave it: 2.5M drawables x 256 views 488 us with 2, 407
+// with 3).
+template <int BLOCK, int ITEMS, bool FUSED, bool COOP = false, int WPE = BLOCK == 256 && ITEMS == 8 ? 3 : 1>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void cullKernel(CullParams P)
 {
 	using S = CullShared<BLOCK, ITEMS>;
@@ -1501,8 +1771,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 	// Two tickets in turn: the barriers of an item's body are inside its view
 	// groups, so without them a wave could still have to read one ticket when
 	// thread 0 writes the next; it has read it by that one's barrier.
+	Tickets tickets(shard);
 	for (uint32_t b = 0;; b ^= 1u) {
-		if (tid == 0) sh.ticket[b] = itemOfTicket(shard, askTicket(P, shard));
+		if (wave == 0) tickets.choose(P, lane);
+		if (tid == 0) sh.ticket[b] = itemOfTicket(tickets.s, askTicket(P, tickets.s));
 		__syncthreads();
 		const uint32_t w = uniform(sh.ticket[b]);
 		if (w >= P.totalWork) break;
@@ -1709,6 +1981,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 			__syncthreads();
 
 			// 2. look-back, one view per lane of wave 0
+			bool stuck = false;
 			if (wave == 0 && lane < vg) {
 				uint32_t total = 0;
 #pragma unroll
@@ -1719,8 +1992,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 					publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
 				} else {
 					publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
-					excl = lookBackSerial(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch});
-					publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
+					excl = lookBackSerial(chain, T.chain, waitBound<true>(P, epoch, tickets.roam));
+					if (excl != kStuck) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
 				}
 				uint32_t b = T.segBase + excl;
 #pragma unroll
@@ -1728,8 +2001,17 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 					sh.base[lane][q] = b;
 					b += sh.cnt[lane][q];
 				}
-				if (T.last && T.k < J.numStateSets)
+				if (excl == kStuck) {
+					stuck = true;
+#pragma unroll
+					for (int q = 0; q < WAVES; q++) sh.cnt[lane][q] = 0;
+				} else if (T.last && T.k < J.numStateSets) {
 					globalMut<uint32_t>(J.counts)[uint64_t(g0 + lane) * J.numStateSets + T.k] = excl + total;
+				}
+			}
+			if (__ballot(stuck) != 0ull) {
+				leaveItem(P, shard, lane);
+				tickets.roam = true;
 			}
 			__syncthreads();
 
@@ -1794,7 +2076,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 		}
 	}
 
-	if (tid == 0) leaveLaunch(P, shard, epoch);
+	if (wave == 0 && signOff(P, shard, epoch, lane)) finishLaunch<S::TILE, FUSED>(shard, epoch, lane);
 }
 
 // Job offsets of a batched launch of more than kInlineJobs jobs (prefix sums
@@ -1847,7 +2129,7 @@ __global__ __launch_bounds__(256) void cullSetupKernel(const cadrCullJob* __rest
 // loses: the look-back waits a little longer where a chain's neighbours come
 // from different counters (10M drawables in 1024 x 8 tiles, 8 shards: 64.4
 // against 60.4 us with one).  Below 256 workgroups one counter costs less
-// than the second level of leaveLaunch.
+// than the second level of signOff.
 inline uint32_t shardShiftFor(uint32_t tile, uint64_t workgroups, uint64_t work, uint64_t bytes)
 {
 	if (oneShard(tile) || workgroups < 256 || work >= (1ull << 31)) return 0;
@@ -1882,6 +2164,8 @@ struct cadrCullWorkspace {
 using namespace cadr;
 
 namespace {
+
+uint64_t stuckAfter(const cadrCullWorkspace& ws) { return std::min(ws.waitLimit / kStuckShare, kStuckUs * ws.ticksPerUs); }
 
 using KernelFn = void (*)(CullParams);
 
@@ -2266,8 +2550,10 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	}
 	if (config->flags & CADR_CULL_WHOLE_TILES) splitTiles = 0;
 	// every item of a tile cut by views reads the tile's local matrices, so one
-	// whose world matrices take their place is left whole
-	if (leaves && std::any_of(hostLeaves, hostLeaves + numJobs, inPlace)) splitTiles = 0;
+	// whose world matrices take their place is left whole; nor can its items be
+	// left to the end of the launch, which one ticket counter never needs
+	const bool inPlaceLeaves = leaves && std::any_of(hostLeaves, hostLeaves + numJobs, inPlace);
+	if (inPlaceLeaves) splitTiles = 0;
 	const uint64_t totalWork = workItems(splitTiles, groupShift);
 	uint64_t statusNeed = 0, bytes = 0;
 	for (uint32_t j = 0; j < numJobs; j++) {
@@ -2301,9 +2587,10 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	p.totalWork = uint32_t(totalWork);
 	p.splitTiles = splitTiles;
 	p.groupShift = groupShift;
-	p.shardShift = shardShiftFor(ke.block * ke.items, grid, totalWork, bytes);
+	p.shardShift = inPlaceLeaves ? 0u : shardShiftFor(ke.block * ke.items, grid, totalWork, bytes);
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
+	p.stuckAfter = inPlaceLeaves ? ~0ull : stuckAfter(*ws);
 	p.leaves = leaves;
 	launchKernel(fn, dim3(uint32_t(grid)), dim3(ke.block), s, p);
 	CADR_CHECK_HIP(hipGetLastError(), "cullKernel launch");
@@ -2363,6 +2650,7 @@ CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, cons
 	p.totalWork = hostJob->numTiles;
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
+	p.stuckAfter = stuckAfter(*ws);
 	// a persistent kernel fills the GPU once; the other takes one tile per workgroup
 	// more tiles than workgroups fit on the GPU at once: the persistent kernel
 	// (grid = resident workgroups); else one tile per workgroup, which saves
@@ -2407,10 +2695,13 @@ CADR_API int cadrPropagateCullView(const cadrTransformLevel* leaf, const cadrCul
 	p.totalWork = hostJob->numTiles;
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
+	p.stuckAfter = stuckAfter(*ws);
 	p.leaf = LeafParams{leaf->localMatrices, leaf->parentIndex, leaf->parentWorld, leaf->worldMatrices, leaf->spheres,
 	                    leaf->parentWorld ? leaf->parentCount : 0u};
-	p.shardShift = shardShiftFor(ke->block * ke->items, hostJob->numTiles, hostJob->numTiles,
-	                             jobBytes(*hostJob, true));
+	if (inPlace(*leaf))  // as in launchBatch
+		p.stuckAfter = ~0ull;
+	else
+		p.shardShift = shardShiftFor(ke->block * ke->items, hostJob->numTiles, hostJob->numTiles, jobBytes(*hostJob, true));
 	if (ke->block < 512) ke = shapeFor(ke, hostJob->numTiles, computeUnits(), &KernelEntry::fused);
 	launchKernel(ke->fused, dim3(hostJob->numTiles), dim3(ke->block), hipStream_t(stream), p);
 	CADR_CHECK_HIP(hipGetLastError(), "fused cullViewKernel launch");

@@ -448,8 +448,10 @@ typedef struct cadrCullWorkspace cadrCullWorkspace;
 int cadrCullWorkspaceCreate(uint64_t statusWords, uint32_t maxJobs, cadrCullWorkspace** workspace);
 int cadrCullWorkspaceDestroy(cadrCullWorkspace* workspace);
 /* Look-back waits are bounded, so a launch ends whatever tile list it is
- * given.  A well-formed list (cadrBuildCullTiles) only waits on tiles with
- * earlier tickets, which are running or done; a caller-built list that names
+ * given.  A launch of a well-formed list (cadrBuildCullTiles) completes with
+ * any number of its workgroups running at once: a work item that has waited a
+ * millisecond (or a quarter of the limit) for tiles of workgroups that do not
+ * run is left to the end of the launch.  A caller-built list that names
  * a predecessor no tile publishes would otherwise wait forever.  A wait that
  * lasts longer than the limit (default 1 s, at least 1 us) gives up, every
  * other wait of the same launch gives up at its next unready poll, and the
