@@ -2476,11 +2476,19 @@ KernelFn viewLoopOf(const KernelEntry& ke)
 // 105 / 86; 128 views 100k 33 / 64, 333k 75 / 75; 512 x 4: 16 views 865k 33 /
 // 36, 27 views 1.2M 70 / 62.  So few wins up to about 16 views a drawable, and
 // for more views where the tiles do not fill the chip twice and the launch has
-// no more than about 2^25 tests.
-KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t numJobs, uint32_t flags)
+// no more than about 2^25 tests.  A launch whose jobs differ goes by its average,
+// unless jobs that are the many-view kernel's by themselves have more than 6
+// tests per drawable of the others, which that kernel is slower on: 10M
+// drawables x 1 view + 1M x 128 (a tree's) 332 / 187 us, 4M x 1 + 2M x 32 121 /
+// 93, 8M x 1 + 1M x 64 157 / 129, but 16M x 1 in 8 scenes + 1M x 64 223 / 237,
+// 10M x 1 + 100k x 256 111 / 117.  (Scattered drawables, which no bounding
+// sphere helps: 310 / 377, 224 / 304 and 107 / 231 in the first and the last two.)
+KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t numJobs, uint32_t flags, uint32_t cu)
 {
+	constexpr uint64_t kFewViews = 16, kFewTests = 1ull << 25;
 	uint64_t drawables = 0, tests = 0, tiles = 0;
 	uint32_t mostViews = 0;
+	uint64_t manyTests = 0, others = 0;  // tests of jobs of many views and tests, drawables of the other jobs
 	for (uint32_t j = 0; j < numJobs; j++) {
 		if (jobs[j].numViews == 0) continue;  // no work items
 		// (a tile of few or no drawables costs what some 256 tests do)
@@ -2489,10 +2497,14 @@ KernelFn fewKernelFor(const KernelEntry& ke, const cadrCullJob* jobs, uint32_t n
 		tests += n * jobs[j].numViews;
 		tiles += jobs[j].numTiles;
 		mostViews = std::max(mostViews, jobs[j].numViews);
+		if (jobs[j].numViews > kFewViews && n * jobs[j].numViews > kFewTests)
+			manyTests += n * jobs[j].numViews;
+		else
+			others += n;
 	}
 	const bool split = (flags & CADR_CULL_WHOLE_TILES) == 0;
-	const bool small = tiles <= 512 && tests <= (1ull << 25);
-	if (split ? tests > 16 * drawables && !small : mostViews > 4) return nullptr;
+	const bool small = tiles <= 2 * cu && tests <= kFewTests;
+	if (split ? manyTests > 6 * others || (tests > kFewViews * drawables && !small) : mostViews > 4) return nullptr;
 	return ke.few[numJobs > 1][mostViews <= 1 ? 0 : mostViews == 2 ? 1 : 2];
 }
 
@@ -2532,7 +2544,7 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	constexpr uint64_t kMaxWork = 0xffffffffull;  // tickets are 32 bits
 	// every tile cut by four views: only what still has its tickets
 	const bool cut = workItems(0xffffffffu, 2) < kMaxWork;
-	const KernelFn few = leaves || !cut ? nullptr : fewKernelFor(ke, hostJobs, numJobs, config->flags);
+	const KernelFn few = leaves || !cut ? nullptr : fewKernelFor(ke, hostJobs, numJobs, config->flags, cu);
 	uint32_t splitTiles = uint32_t(std::min<uint64_t>(grid, 1u << 20)), groupShift = 6;
 	if (few) {
 		fn = few;
