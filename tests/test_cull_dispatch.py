@@ -308,3 +308,13 @@ def test_work_item_limit_is_that_of_whole_tiles(gpu, tiles, views, error):
     with pytest.raises(N.CadrError, match=error):
         N.check(N.load().cadrCullBatch(ctypes.byref(config), 16, N.ptr(jobs), 1, ws.handle, None))
     ws.close()
+
+
+@pytest.mark.parametrize("meshes", [1 << 19, (1 << 19) + 77])
+def test_mesh_tables_past_the_list_entries(gpu, meshes):
+    """A list entry holds 19 bits of mesh index; the meshes of a larger table are read again when commands are stored."""
+    print(f"{meshes} meshes", flush=True)
+    _run([(30_001, 3, meshes, 1)], 256, 4, lambda b: b.run_view())
+    _run([(30_001, 3, meshes, 1)], 1024, 1, lambda b: b.run_view())
+    _run([(9000, 2, meshes, 3), (700, 1, 9, 1)], 256, 2, lambda b: b.run())
+    _run([(9000, 2, meshes, 70)], 256, 8, lambda b: b.run(), N.CULL_WHOLE_TILES)
