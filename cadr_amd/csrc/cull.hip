@@ -2268,11 +2268,16 @@ const KernelEntry* shapeFor(const KernelEntry* ke, uint32_t numTiles, uint32_t c
 // The same for a batched launch: 512 x 4 for 256 x 8, the one pair of shapes
 // that has every batched kernel (150k drawables, 4 / 20 views: 14.4 / 21.0 us at
 // 256 x 8, 11.4 / 18.4 at 512 x 4; 400k, 196 tiles, 16.1 / 29.4 and 13.1 / 28.4;
-// 12 small trees, leaves fused, 49.5 and 39.8).
+// 12 small trees, leaves fused, 49.5 and 39.8).  With fused leaves up to 8 tiles
+// a compute unit, where 256 x 8's longer chain per wave is not yet covered by
+// other workgroups: 640 tiles, 1-10 views, 73.9 and 61.9 us (256 x 8 with its
+// spheres in registers 64.8), 1,408 tiles, 1-32 views, 129.4 and 117.7, 1,930,
+// 1-10 views, 141.7 and 131.2, but at 2,048, one view, 106.6 and 108.1, 9,920, 1-2
+// views, 462.7 and 475.5.
 const KernelEntry* batchShapeFor(const KernelEntry* ke, uint64_t tiles, uint32_t cu, KernelFn KernelEntry::*path)
 {
-	if (tiles > cu) return ke;
-	const KernelEntry* wide = shapeFor(ke, uint32_t(tiles), cu, path);
+	if (path == &KernelEntry::fusedBatch ? tiles >= 8ull * cu : tiles > cu) return ke;
+	const KernelEntry* wide = shapeFor(ke, uint32_t(std::min<uint64_t>(tiles, cu)), cu, path);
 	return ke->few[0][0] && wide->few[0][0] ? wide : ke;
 }
 
