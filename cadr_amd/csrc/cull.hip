@@ -10,7 +10,8 @@
 // Work is split into tiles of at most blockSize*itemsPerThread drawables that
 // never cross a StateSet boundary; tiles are taken by atomic tickets in array
 // order (dealt over several counters where small tiles need it, askTicket),
-// so a tile only ever waits on tiles that already run or come next.  Within a
+// so a tile waits on tiles that already run or come next, and what waits too
+// long is finished at the end of the launch (finishLeft).  Within a
 // tile, wave w owns a contiguous run of 64*itemsPerThread drawables (item j of
 // lane l is drawable w*64*itemsPerThread + j*64 + l): loads are coalesced and
 // the visibility of 64 drawables is one wave64 ballot.  Offsets come from a
@@ -2668,7 +2669,6 @@ CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, cons
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
 	p.stuckAfter = stuckAfter(*ws);
-	// a persistent kernel fills the GPU once; the other takes one tile per workgroup
 	// more tiles than workgroups fit on the GPU at once: the persistent kernel
 	// (grid = resident workgroups); else one tile per workgroup, which saves
 	// the loop's extra ticket and barrier on a launch-bound view

@@ -422,8 +422,8 @@ typedef struct cadrCullJob {
 } cadrCullJob;                  /* 80 B */
 
 /* Kernel shape.  tileSize = blockSize * itemsPerThread.  A launch whose tiles
- * do not fill the compute units once may run another shape of the same tile
- * size; results do not depend on it. */
+ * do not fill the compute units (once, or 8 times with fused leaf levels) may
+ * run another shape of the same tile size; results do not depend on it. */
 typedef struct cadrCullConfig {
 	uint32_t blockSize;         /* 256 or 512 threads                          */
 	uint32_t itemsPerThread;    /* 2, 4, 8 or 16                               */
