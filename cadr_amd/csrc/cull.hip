@@ -54,6 +54,7 @@
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <type_traits>
 #include <vector>
 
 namespace cadr {
@@ -96,7 +97,6 @@ struct CullParams {
 	uint32_t groupShift;  // batched: log2 of the views of such a group
 	uint32_t flags;
 	uint64_t waitLimit;                 // steady-counter ticks a look-back may wait
-	uint64_t stuckAfter;                // and after which it leaves its item to the end of the launch (kStuck)
 	LeafParams leaf;                    // one-view fused kernel
 	const cadrTransformLevel* leaves;   // fused batched kernel: leaf level of each job
 };
@@ -414,7 +414,6 @@ struct WaitBound {
 	uint32_t* ctl;
 	uint64_t limit;
 	uint32_t epoch;
-	uint64_t stuck;  // ticks after which a wait returns kStuck
 };
 
 // Work tickets.  An atomic add on one address takes 11-12 ns on this GPU
@@ -435,14 +434,14 @@ struct WaitBound {
 //
 // Where fewer do (a stream held to some compute units, other streams' kernels
 // on the rest), the ones that run would wait for tiles of shards that none of
-// them serves.  A wait that lasts kStuckUs therefore leaves its item: the
+// them serves.  A wait that lasts kStuckTicks therefore leaves its item: the
 // item's total is published, so no other item waits for it, the workgroup
 // ends and makes room or, a persistent one, goes on with tickets of whichever
 // shard is furthest behind, and the last workgroup of the launch finishes what
 // was left (finishLeft), when every total is published.  So a launch
 // progresses with any number of workgroups running.
 constexpr uint32_t kStuck = ~0u;         // for an exclusive prefix (30 bits)
-constexpr uint64_t kStuckUs = 1000;      // some hundred times the usual wait, and as long as most other launches
+constexpr uint64_t kStuckTicks = 100000; // 1 ms: some hundred times the usual wait, and as long as most other launches
 constexpr uint64_t kStuckShare = 4;      // at most this part of the wait limit
 constexpr uint32_t kAgainShare = 16;     // the part of that which a workgroup waits once it was stuck
 constexpr uint32_t kLeftFlag = 1u << 31; // in a count of workgroups that left: one of them left an item
@@ -526,21 +525,39 @@ struct Tickets {
 
 	__device__ __forceinline__ explicit Tickets(Shard home) : s(home), roam(false) {}
 
-	// Before a ticket is asked for: the shard whose next ticket is the smallest item.
-	__device__ __forceinline__ void choose(const CullParams& P, uint32_t lane)
+	// The next work item, at or past P.totalWork if there is none, to *item
+	// (called by wave 0).  A roaming workgroup may be the last one that serves
+	// its own shard, or any other, so it ends only when every shard is empty: a
+	// shard whose last ticket another took between its look and its own ticket
+	// is one less to look at.
+	__device__ __forceinline__ void next(const CullParams& P, uint32_t lane, uint32_t* item)
 	{
-		if (!roam) return;
-		uint64_t next = ~0ull;  // (item, shard)
-		if (lane < (1u << s.shift)) {
-			const uint32_t r = __hip_atomic_load(&P.ctl[kCtlShard + 64u * lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			next = (uint64_t(itemOfTicket(Shard{s.shift, lane}, r)) << 32) | lane;
+		if (!roam) {
+			if (lane == 0) *item = itemOfTicket(s, askTicket(P, s));
+			return;
 		}
+		for (;;) {
+			uint64_t first = ~0ull;  // the smallest (item of a shard's next ticket, shard)
+			if (lane < (1u << s.shift)) {
+				const uint32_t r = __hip_atomic_load(&P.ctl[kCtlShard + 64u * lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+				first = (uint64_t(itemOfTicket(Shard{s.shift, lane}, r)) << 32) | lane;
+			}
 #pragma unroll
-		for (int off = 8; off >= 1; off >>= 1) {
-			const uint64_t o = __shfl_xor(next, off);
-			next = o < next ? o : next;
+			for (int off = 8; off >= 1; off >>= 1) {
+				const uint64_t o = __shfl_xor(first, off);
+				first = o < first ? o : first;
+			}
+			s.g = uniform(uint32_t(first));
+			uint32_t t = uniform(uint32_t(first >> 32));
+			if (t < P.totalWork) {
+				t = 0;
+				if (lane == 0) t = itemOfTicket(s, askTicket(P, s));
+				t = uniform(t);
+				if (t >= P.totalWork) continue;
+			}
+			if (lane == 0) *item = t;
+			return;
 		}
-		s.g = uniform(uint32_t(next));
 	}
 };
 
@@ -552,17 +569,29 @@ __device__ __forceinline__ void leaveItem(const CullParams& P, Shard home, uint3
 	__threadfence();
 }
 
-// ANY_STUCK: whether the kernel leaves items; again: the workgroup was stuck before.
-template <bool ANY_STUCK>
-__device__ __forceinline__ WaitBound waitBound(const CullParams& P, uint32_t epoch, bool again = false)
-{
-	return WaitBound{P.ctl, P.waitLimit, epoch, !ANY_STUCK ? ~0ull : again ? P.stuckAfter / kAgainShare : P.stuckAfter};
-}
+// Whether and when a wait leaves its item.  Only launches of several shards
+// need it, and only they may: an in-place fused launch, whose items cannot be
+// computed again, takes one.  The time comes from the wait limit at hand:
+// another kernel argument, loaded where a look-back begins, cost fused batches
+// up to 1% (and loaded at the poll, from outside the caches, several us a poll).
+struct NeverStuck {
+	static constexpr bool kCan = false;
+	bool again = false;
+	uint32_t shift = 0;
+};
+struct MayBeStuck {
+	static constexpr bool kCan = true;
+	bool again;      // the workgroup was stuck before
+	uint32_t shift;  // Shard::shift
+};
+template <int TILE>
+using StuckFor = std::conditional_t<oneShard(TILE), NeverStuck, MayBeStuck>;
 
 constexpr uint32_t kPollAgain = 0, kGiveUp = 1, kWaitLater = 2;
 
 // Called after an unready poll; start is 0 until the first such poll.
-__device__ __forceinline__ uint32_t waitStep(const WaitBound& B, uint64_t& start)
+template <class Stuck>
+__device__ __forceinline__ uint32_t waitStep(const WaitBound& B, uint64_t& start, Stuck stuck)
 {
 	if (__hip_atomic_load(&B.ctl[kCtlError], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == B.epoch) return kGiveUp;
 	const uint64_t now = uint64_t(wall_clock64());
@@ -570,7 +599,10 @@ __device__ __forceinline__ uint32_t waitStep(const WaitBound& B, uint64_t& start
 		start = now == 0 ? 1 : now;
 		return kPollAgain;
 	}
-	if (now - start > B.stuck) return kWaitLater;
+	if constexpr (Stuck::kCan) {
+		const uint64_t most = min(B.limit / kStuckShare, kStuckTicks);
+		if (stuck.shift != 0u && now - start > (stuck.again ? most / kAgainShare : most)) return kWaitLater;
+	}
 	if (now - start <= B.limit) return kPollAgain;
 	__hip_atomic_store(&B.ctl[kCtlError], B.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	return kGiveUp;
@@ -580,7 +612,8 @@ __device__ __forceinline__ uint32_t waitStep(const WaitBound& B, uint64_t& start
 // predecessors adding aggregates until an inclusive prefix is found; position
 // 0 ends the walk in any case, and a wait bounded as above ends it early
 // (kStuck if it is left for later).
-__device__ uint32_t lookBackSerial(const uint64_t* chain, uint32_t c, const WaitBound& B)
+template <class Stuck>
+__device__ __forceinline__ uint32_t lookBackSerial(const uint64_t* chain, uint32_t c, const WaitBound& B, Stuck stuck)
 {
 	uint32_t excl = 0;
 	uint32_t p = c;
@@ -591,7 +624,7 @@ __device__ uint32_t lookBackSerial(const uint64_t* chain, uint32_t c, const Wait
 		for (;;) {
 			s = readStatus(chain + p);
 			if (statusReady(s, B.epoch)) break;
-			if (const uint32_t step = waitStep(B, start)) return step == kWaitLater ? kStuck : excl;
+			if (const uint32_t step = waitStep(B, start, stuck)) return step == kWaitLater ? kStuck : excl;
 			__builtin_amdgcn_s_sleep(1);
 		}
 		excl += uint32_t(s) & kValueMask;
@@ -604,7 +637,9 @@ __device__ uint32_t lookBackSerial(const uint64_t* chain, uint32_t c, const Wait
 // position p-1-l, the walk stops at the nearest inclusive prefix, and 64
 // predecessors cost one round trip.  Returns the same value in every lane
 // (the give-up decision is made from wave-uniform values).
-__device__ uint32_t lookBackWave(const uint64_t* chain, uint32_t c, const WaitBound& B, uint32_t lane)
+template <class Stuck>
+__device__ __forceinline__ uint32_t lookBackWave(const uint64_t* chain, uint32_t c, const WaitBound& B, uint32_t lane,
+                                                 Stuck stuck)
 {
 	uint32_t excl = 0;
 	int64_t p = c;
@@ -618,7 +653,7 @@ __device__ uint32_t lookBackWave(const uint64_t* chain, uint32_t c, const WaitBo
 		const uint32_t f = pmask ? uint32_t(__builtin_ctzll(pmask)) : 64u;
 		const uint64_t need = f >= 63u ? ~0ull : ((2ull << f) - 1ull);
 		if (nmask & need) {
-			if (const uint32_t step = uniform(waitStep(B, start))) return step == kWaitLater ? kStuck : excl;
+			if (const uint32_t step = uniform(waitStep(B, start, stuck))) return step == kWaitLater ? kStuck : excl;
 			__builtin_amdgcn_s_sleep(1);
 			continue;
 		}
@@ -635,8 +670,9 @@ __device__ uint32_t lookBackWave(const uint64_t* chain, uint32_t c, const WaitBo
 // lookBackWave for 64 / W chains at once: each run of W lanes walks its own
 // chain with a window of W predecessors.  c is the lane's chain's position
 // (0: nothing before it); returns the lane's chain's prefix.
-template <uint32_t W>
-__device__ uint32_t lookBackGroups(const uint64_t* chain, uint32_t c, const WaitBound& B, uint32_t lane)
+template <uint32_t W, class Stuck>
+__device__ __forceinline__ uint32_t lookBackGroups(const uint64_t* chain, uint32_t c, const WaitBound& B, uint32_t lane,
+                                                   Stuck stuck)
 {
 	static_assert(W >= 2 && W <= 32 && (W & (W - 1)) == 0, "lanes a chain");
 	constexpr uint32_t kAll = W == 32 ? ~0u : (1u << (W & 31u)) - 1u;
@@ -661,7 +697,7 @@ __device__ uint32_t lookBackGroups(const uint64_t* chain, uint32_t c, const Wait
 			p = f < W ? 0 : p - int64_t(W);
 		}
 		if (__ballot(wait) != 0ull) {
-			const uint32_t step = uniform(waitStep(B, start));
+			const uint32_t step = uniform(waitStep(B, start, stuck));
 			if (step == kGiveUp) return excl;
 			if (step == kWaitLater && wait) {  // the other chains go on
 				excl = kStuck;
@@ -905,7 +941,7 @@ __device__ __forceinline__ void finishTile(const CullParams& P, uint64_t job, ui
                                            const LeafParams& Lf, uint64_t* chain, uint32_t pos, uint32_t epoch,
                                            uint32_t lane)
 {
-	const uint32_t excl = lookBackWave(chain, pos, waitBound<false>(P, epoch), lane);
+	const uint32_t excl = lookBackWave(chain, pos, WaitBound{P.ctl, P.waitLimit, epoch}, lane, NeverStuck{});
 	tile = perLane(tile);
 	// loadTile's clamps
 	const uint32_t start = globalPtr<uint32_t>(tile)[0], drawables = globalPtr<uint32_t>(perLane(job))[14];
@@ -1142,7 +1178,7 @@ __device__ __forceinline__ void tileOffset(const CullParams& P, const cadrCullJo
 		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
 	} else {
 		if (lane == 0) publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
-		excl = lookBackWave(chain, T.chain, waitBound<!oneShard(TILE)>(P, epoch, tickets.roam), lane);
+		excl = lookBackWave(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch}, lane, StuckFor<TILE>{tickets.roam, home.shift});
 		if (excl == kStuck) {
 			leaveItem(P, home, lane);
 			tickets.roam = true;
@@ -1273,9 +1309,7 @@ __device__ __forceinline__ bool cullViewTiles(const CullParams& P, const cadrCul
 	for (uint32_t b = 0;; b ^= 1u) {
 		const uint32_t n = listVisible<ITEMS>(sp, mi, T, J.numMeshes, V, wave * WAVE_ITEMS, lane, run);
 		if (lane == 0) sCnt[b][wave] = n;
-		if constexpr (!oneShard(BLOCK * ITEMS))
-			if (wave == 0) tickets.choose(P, lane);
-		if (tid == 0) *sTicket = itemOfTicket(tickets.s, askTicket(P, tickets.s));
+		if (wave == 0) tickets.next(P, lane, sTicket);
 		__syncthreads();
 
 		// the next tile's loads, in flight through this tile's look-back and stores
@@ -1568,11 +1602,12 @@ __device__ __forceinline__ void fewLookBack(const CullParams& P, const FewItem& 
 	const FewChain<CH> c(f, lane);
 	uint32_t e = 0;
 	if (!f.T.first) {
-		const WaitBound B = waitBound<true>(P, epoch, tickets.roam);
+		const WaitBound B{P.ctl, P.waitLimit, epoch};
+		const MayBeStuck stuck{tickets.roam, home.shift};
 		if constexpr (CH == 1)
-			e = lookBackWave(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane);
+			e = lookBackWave(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane, stuck);
 		else
-			e = lookBackGroups<64 / CH>(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane);
+			e = lookBackGroups<64 / CH>(c.chain - f.T.chain, c.on ? f.T.chain : 0u, B, lane, stuck);
 		if (__ballot(c.on && e == kStuck) != 0ull) {
 			leaveItem(P, home, lane);
 			tickets.roam = true;
@@ -1631,8 +1666,7 @@ __device__ __forceinline__ bool cullFewItems(const CullParams& P, FewShared<BLOC
 				                          wave * WAVE_ITEMS, lane, sh.run[DEFER ? b : 0][wave][c]);
 			if (lane == 0) sh.cnt[b][c][wave] = n[c];
 		}
-		if (DEFER && wave == 0) tickets.choose(P, lane);
-		if (DEFER && tid == 0) sh.ticket[b] = itemOfTicket(tickets.s, askTicket(P, tickets.s));
+		if (DEFER && wave == 0) tickets.next(P, lane, &sh.ticket[b]);
 		__syncthreads();
 		FewItem next;
 		bool more = false;
@@ -1685,8 +1719,7 @@ __device__ __forceinline__ bool cullFewItems(const CullParams& P, FewShared<BLOC
 			cur = next;
 		} else {
 			fewStore<CH, LDS, WAVE_ITEMS>(cur, staged, sh.run[0][wave], n, off, sh.excl[b], wave, lane);
-			if (wave == 0) tickets.choose(P, lane);
-			if (tid == 0) sh.ticket[b] = itemOfTicket(tickets.s, askTicket(P, tickets.s));
+			if (wave == 0) tickets.next(P, lane, &sh.ticket[b]);
 			__syncthreads();
 			takeNext(cur);
 			if (!more) break;
@@ -1695,8 +1728,9 @@ __device__ __forceinline__ bool cullFewItems(const CullParams& P, FewShared<BLOC
 	return wave == 0 && signOff(P, shard, epoch, lane);
 }
 
+// (256 x 8 with one view takes one register more than the 6 waves its LDS allows)
 template <int BLOCK, int ITEMS, int CH, bool DEFER, bool JOBS>
-__global__ __launch_bounds__(BLOCK) void cullFewKernel(CullParams P)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(ITEMS == 8 && CH == 1 ? 6 : 1))) void cullFewKernel(CullParams P)
 {
 	__shared__ FewShared<BLOCK, ITEMS, CH, DEFER> sh;
 	const uint32_t tid = threadIdx.x, lane = laneId(), wave = uniform(tid / 64);
@@ -1744,10 +1778,11 @@ struct CullShared {
 // COOP (fused form only): parent matrices read whole, 16 per instruction
 // (issueParentLoads), for leaves whose parents are scattered; it holds more
 // registers, so it is chosen per shape, like WPE, the waves per SIMD asked of
-// the register allocator (see the kernel table; 256 x 8 takes one register
-// more than 3 waves leave it: 2.5M drawables x 256 views 488 us with 2, 407
-// with 3).
-template <int BLOCK, int ITEMS, bool FUSED, bool COOP = false, int WPE = BLOCK == 256 && ITEMS == 8 ? 3 : 1>
+// the register allocator (see the kernel table; unfused, 256 x 8 and 256 x 4
+// take a register or two more than 3 and 4 waves leave them: 2.5M drawables x
+// 256 views 488 us with 2 waves at 256 x 8, 407 with 3).
+template <int BLOCK, int ITEMS, bool FUSED, bool COOP = false,
+          int WPE = BLOCK != 256 ? 1 : ITEMS == 8 ? 3 : ITEMS == 4 ? 4 : 1>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) void cullKernel(CullParams P)
 {
 	using S = CullShared<BLOCK, ITEMS>;
@@ -1772,12 +1807,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 	// Two tickets in turn: the barriers of an item's body are inside its view
 	// groups, so without them a wave could still have to read one ticket when
 	// thread 0 writes the next; it has read it by that one's barrier.
-	Tickets tickets(shard);
+	// (Wave 0's b also holds Tickets::roam.)
+	constexpr uint32_t kRoam = 2;
 	for (uint32_t b = 0;; b ^= 1u) {
-		if (wave == 0) tickets.choose(P, lane);
-		if (tid == 0) sh.ticket[b] = itemOfTicket(tickets.s, askTicket(P, tickets.s));
+		if (wave == 0) {
+			Tickets tickets(shard);
+			tickets.roam = (b & kRoam) != 0u;
+			tickets.next(P, lane, &sh.ticket[b & 1u]);
+		}
 		__syncthreads();
-		const uint32_t w = uniform(sh.ticket[b]);
+		const uint32_t w = uniform(sh.ticket[b & 1u]);
 		if (w >= P.totalWork) break;
 		// a lane index of its own for each tile: the compiler otherwise keeps
 		// dozens of addresses derived from it in registers across tiles
@@ -1993,14 +2032,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 					publish(chain + T.chain, packStatus(epoch, kStatePrefix, total));
 				} else {
 					publish(chain + T.chain, packStatus(epoch, kStateAggregate, total));
-					excl = lookBackSerial(chain, T.chain, waitBound<true>(P, epoch, tickets.roam));
+					excl = lookBackSerial(chain, T.chain, WaitBound{P.ctl, P.waitLimit, epoch}, MayBeStuck{(b & kRoam) != 0u, shard.shift});
 					if (excl != kStuck) publish(chain + T.chain, packStatus(epoch, kStatePrefix, excl + total));
 				}
-				uint32_t b = T.segBase + excl;
+				uint32_t slot = T.segBase + excl;
 #pragma unroll
 				for (int q = 0; q < WAVES; q++) {
-					sh.base[lane][q] = b;
-					b += sh.cnt[lane][q];
+					sh.base[lane][q] = slot;
+					slot += sh.cnt[lane][q];
 				}
 				if (excl == kStuck) {
 					stuck = true;
@@ -2012,7 +2051,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 			}
 			if (__ballot(stuck) != 0ull) {
 				leaveItem(P, shard, lane);
-				tickets.roam = true;
+				b |= kRoam;
 			}
 			__syncthreads();
 
@@ -2165,8 +2204,6 @@ struct cadrCullWorkspace {
 using namespace cadr;
 
 namespace {
-
-uint64_t stuckAfter(const cadrCullWorkspace& ws) { return std::min(ws.waitLimit / kStuckShare, kStuckUs * ws.ticksPerUs); }
 
 using KernelFn = void (*)(CullParams);
 
@@ -2608,7 +2645,6 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	p.shardShift = inPlaceLeaves ? 0u : shardShiftFor(ke.block * ke.items, grid, totalWork, bytes);
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
-	p.stuckAfter = inPlaceLeaves ? ~0ull : stuckAfter(*ws);
 	p.leaves = leaves;
 	launchKernel(fn, dim3(uint32_t(grid)), dim3(ke.block), s, p);
 	CADR_CHECK_HIP(hipGetLastError(), "cullKernel launch");
@@ -2668,7 +2704,6 @@ CADR_API int cadrCullView(const cadrCullConfig* config, uint64_t deviceJob, cons
 	p.totalWork = hostJob->numTiles;
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
-	p.stuckAfter = stuckAfter(*ws);
 	// more tiles than workgroups fit on the GPU at once: the persistent kernel
 	// (grid = resident workgroups); else one tile per workgroup, which saves
 	// the loop's extra ticket and barrier on a launch-bound view
@@ -2712,12 +2747,9 @@ CADR_API int cadrPropagateCullView(const cadrTransformLevel* leaf, const cadrCul
 	p.totalWork = hostJob->numTiles;
 	p.flags = config->flags;
 	p.waitLimit = ws->waitLimit;
-	p.stuckAfter = stuckAfter(*ws);
 	p.leaf = LeafParams{leaf->localMatrices, leaf->parentIndex, leaf->parentWorld, leaf->worldMatrices, leaf->spheres,
 	                    leaf->parentWorld ? leaf->parentCount : 0u};
-	if (inPlace(*leaf))  // as in launchBatch
-		p.stuckAfter = ~0ull;
-	else
+	if (!inPlace(*leaf))  // as in launchBatch
 		p.shardShift = shardShiftFor(ke->block * ke->items, hostJob->numTiles, hostJob->numTiles, jobBytes(*hostJob, true));
 	if (ke->block < 512) ke = shapeFor(ke, hostJob->numTiles, computeUnits(), &KernelEntry::fused);
 	launchKernel(ke->fused, dim3(hostJob->numTiles), dim3(ke->block), hipStream_t(stream), p);
