@@ -2311,10 +2311,16 @@ const KernelEntry* shapeFor(const KernelEntry* ke, uint32_t numTiles, uint32_t c
 // other workgroups: 640 tiles, 1-10 views, 73.9 and 61.9 us (256 x 8 with its
 // spheres in registers 64.8), 1,408 tiles, 1-32 views, 129.4 and 117.7, 1,930,
 // 1-10 views, 141.7 and 131.2, but at 2,048, one view, 106.6 and 108.1, 9,920, 1-2
-// views, 462.7 and 475.5.
-const KernelEntry* batchShapeFor(const KernelEntry* ke, uint64_t tiles, uint32_t cu, KernelFn KernelEntry::*path)
+// views, 462.7 and 475.5.  Past 4 tiles a compute unit only if they are a quarter
+// full, or the rounds of its fewer workgroups count for more: 512 tiles of 352
+// drawables, 1-3 views, 33.4 and 27.4, but 1,280 of 274, one view, 46.9 and 49.6.
+const KernelEntry* batchShapeFor(const KernelEntry* ke, uint64_t tiles, uint64_t drawables, uint32_t cu,
+                                 KernelFn KernelEntry::*path)
 {
-	if (path == &KernelEntry::fusedBatch ? tiles >= 8ull * cu : tiles > cu) return ke;
+	const uint64_t full = uint64_t(ke->block) * ke->items;
+	if (path == &KernelEntry::fusedBatch ? tiles >= 8ull * cu || (tiles > 4ull * cu && 4 * drawables < full * tiles)
+	                                     : tiles > cu)
+		return ke;
 	const KernelEntry* wide = shapeFor(ke, uint32_t(std::min<uint64_t>(tiles, cu)), cu, path);
 	return ke->few[0][0] && wide->few[0][0] ? wide : ke;
 }
@@ -2571,9 +2577,12 @@ int launchBatch(KernelFn KernelEntry::*path, const KernelEntry& asked, const cad
 	// the persistent grid; unless CADR_CULL_WHOLE_TILES, a job's last grid
 	// tiles are handed out per view group
 	const uint32_t cu = computeUnits();
-	uint64_t tiles = 0;
-	for (uint32_t j = 0; j < numJobs; j++) tiles += hostJobs[j].numTiles;
-	const KernelEntry& ke = *batchShapeFor(&asked, tiles, cu, path);
+	uint64_t tiles = 0, drawables = 0;
+	for (uint32_t j = 0; j < numJobs; j++) {
+		tiles += hostJobs[j].numTiles;
+		drawables += hostJobs[j].numDrawables;
+	}
+	const KernelEntry& ke = *batchShapeFor(&asked, tiles, drawables, cu, path);
 	KernelFn fn = ke.*path;
 	uint32_t perCU = config->workgroupsPerCU;
 	if (perCU == 0) perCU = ke.block >= 512 ? 2 : 4;
